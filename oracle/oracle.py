@@ -27,7 +27,8 @@ def build(ref=False):
     """Compile the oracle (and, when the Nek5000 sources are present, the
     reference speclib.f) with oracle/Makefile."""
     subprocess.run(["make", "-s", "-C", HERE, "libnekoracle.so"], check=True)
-    if ref and os.path.isdir(os.environ.get("NEKREF", "/root/reference")):
+    src = os.path.join(os.environ.get("NEKREF", "/root/reference"), "core", "speclib.f")
+    if ref and os.path.isfile(src):
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
 
