@@ -12,7 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libnekamd.so")
 OBJ = os.path.join(HERE, "_objs")
 SOURCES = ["capi.cpp", "kernels.hip", "axhelm.hip", "axhelm_cg.hip", "axhelm_gated.hip", "gs.hip", "cg.hip", "hsmg.hip",
-           "hsmg_setup.hip", "coarse.hip",
+           "hsmg_setup.hip", "coarse.hip", "coarse_direct.hip",
            "gmres.hip", "proj.hip", "adjoint.hip", "mesh_io.cpp", "mixed.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -1,12 +1,13 @@
-// Coarse-space solver of the H1 multigrid: the assembled trilinear Galerkin
-// problem (navier8.f:83-233 set_up_h1_crs) solved to a tight relative
-// residual by conjugate gradients preconditioned with a smoothed-aggregation
-// algebraic multigrid V-cycle (damped-Jacobi smoothing, dense inverse on the
-// last level).  Stands in for the reference's exact XXT factor
-// (crs_xxt.c:922-960): same solution to the CG tolerance.
+// Coarse-space solver of the H1 multigrid, in place of the reference's exact
+// XXT factor (crs_xxt.c:922-960): the assembled trilinear Galerkin problem
+// (navier8.f:83-233 set_up_h1_crs) solved directly (coarse_direct.h) up to the
+// size that allows, beyond it to a tight relative residual by conjugate
+// gradients preconditioned with a smoothed-aggregation algebraic multigrid
+// V-cycle (damped-Jacobi smoothing, dense inverse on the last level).
 #pragma once
 #include <vector>
 
+#include "coarse_direct.h"
 #include "nekamd_internal.h"
 
 namespace nekamd {
@@ -55,6 +56,12 @@ struct CrsPcg {
 
 struct CoarseSolver {
   int n = 0;                 // unknowns
+  DirectCoarse direct;       // the solve, where it is set up
+  // the assembled problem, kept while direct holds the solve: its AMG
+  // hierarchy is built when vcycle_only first asks for it
+  std::vector<int32_t> h_rp, h_ci;
+  std::vector<double> h_v;
+  bool has_amg = false;
   std::vector<AmgLevel> lev; // lev[0] is the coarse problem itself
   int ndense = 0;            // size of the last level, solved by a dense inverse
   double *dinv_dense = nullptr;
@@ -71,16 +78,20 @@ struct CoarseSolver {
   int64_t iters_total = 0, solves = 0;
   int nlevels_amg = 0;
 
-  // A: CSR of the assembled problem (rows sorted, diagonal present).
+  // A: CSR of the assembled problem (rows sorted, diagonal present); xyz:
+  // three coordinates per unknown.
   int setup(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
-            const std::vector<double> &val, hipStream_t s);
-  // x = A^-1 b to the relative residual rtol (or rtol_use when > 0); host
-  // waits on stream s.
+            const std::vector<double> &val, const std::vector<double> &xyz, hipStream_t s);
+  int setup_amg(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
+                const std::vector<double> &val);
+  // x = A^-1 b, directly, or to the relative residual rtol (or rtol_use when
+  // > 0) by PCG, where the host waits on stream s.
   int solve(double *xout, const double *b, hipStream_t s, double rtol_use = 0.0);
   // x = M b, one AMG V-cycle (no host wait)
   int vcycle_only(double *xout, const double *b, hipStream_t s);
   void vcycle(const double *rhs, double *out, double *part_out, hipStream_t s,
               const PcgUpdate *up = nullptr);
+  void release_amg();
   void release();
 };
 

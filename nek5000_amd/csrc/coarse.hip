@@ -1,4 +1,5 @@
-// Coarse-space solver: PCG with a smoothed-aggregation AMG V-cycle.
+// Coarse-space solver beyond the size of the direct one (coarse_direct.hip):
+// PCG with a smoothed-aggregation AMG V-cycle.
 //
 // Set-up (host): strength-of-connection graph, greedy aggregation (seed
 // aggregates of a node and its free strong neighbours, leftovers joined to a
@@ -598,10 +599,23 @@ inline int wblocks(int n) { return std::max(1, std::min((n + 3) / 4, 8192)); }
 }  // namespace
 
 int CoarseSolver::setup(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
-                        const std::vector<double> &val, hipStream_t s) {
+                        const std::vector<double> &val, const std::vector<double> &xyz,
+                        hipStream_t s) {
   release();
   n = (int)rowptr.size() - 1;
   if (n <= 0) return NKH_OK;
+  bool ok = false;
+  NK_TRY(direct.setup(rowptr, col, val, xyz, s, &ok));
+  if (!ok) return setup_amg(rowptr, col, val);
+  h_rp = rowptr;
+  h_ci = col;
+  h_v = val;
+  return NKH_OK;
+}
+
+int CoarseSolver::setup_amg(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
+                            const std::vector<double> &val) {
+  release_amg();
   Csr A;
   A.n = A.m = n;
   A.rp = rowptr;
@@ -664,17 +678,27 @@ int CoarseSolver::setup(const std::vector<int32_t> &rowptr, const std::vector<in
     NK_TRY(dalloc(&L.r, L.n));
     NK_TRY(dalloc(&L.b, L.n));
   }
+  has_amg = true;
   if (nlevels_amg == 0) return NKH_OK;  // dense solve of the whole problem
   for (double **q : {&x, &rb[0], &rb[1], &z, &w, &p[0], &p[1]}) NK_TRY(dalloc(q, n));
   NK_TRY(dalloc(&part, 4 * kCrsBlocks));
   NK_HIP(hipMalloc(&st, sizeof(CrsPcg)));
   CrsPcg init{};
   NK_HIP(hipMemcpy(st, &init, sizeof(CrsPcg), hipMemcpyHostToDevice));
-  (void)s;
   return NKH_OK;
 }
 
 void CoarseSolver::release() {
+  direct.release();
+  h_rp.clear();
+  h_ci.clear();
+  h_v.clear();
+  release_amg();
+  n = 0;
+}
+
+void CoarseSolver::release_amg() {
+  has_amg = false;
   for (AmgLevel &L : lev) {
     free_ell(L.A);
     free_csr(L.Aw);
@@ -689,7 +713,7 @@ void CoarseSolver::release() {
   if (st) (void)hipFree(st);
   dinv_dense = xd = bd = x = rb[0] = rb[1] = z = w = p[0] = p[1] = part = nullptr;
   st = nullptr;
-  n = ndense = nlevels_amg = 0;
+  ndense = nlevels_amg = 0;
 }
 
 // z = M rhs: one V(1,1)-cycle; the partial sums of rhs.z land in part_out.
@@ -741,6 +765,7 @@ void CoarseSolver::vcycle(const double *rhs, double *out, double *part_out, hipS
 // param(40) = 1, applies its hierarchy once: crs_amg.c:129-).
 int CoarseSolver::vcycle_only(double *xout, const double *b, hipStream_t s) {
   if (n == 0) return NKH_OK;
+  if (n > kDenseMax && !has_amg) NK_TRY(setup_amg(h_rp, h_ci, h_v));
   if (nlevels_amg == 0) return solve(xout, b, s);
   hipLaunchKernelGGL(k_pcg_reset, dim3(1), dim3(1), 0, s, st);
   vcycle(b, xout, nullptr, s);
@@ -752,6 +777,10 @@ int CoarseSolver::vcycle_only(double *xout, const double *b, hipStream_t s) {
 int CoarseSolver::solve(double *xout, const double *b, hipStream_t s, double rtol_use) {
   if (n == 0) return NKH_OK;
   const dim3 B(256);
+  if (direct.ready()) {
+    solves += 1;
+    return direct.solve(xout, b, s);
+  }
   if (nlevels_amg == 0) {  // small problem: the dense inverse is the solve
     hipLaunchKernelGGL(k_dense_apply, dim3(wblocks(n)), B, 0, s, dinv_dense, n, b, xout,
                        (const CrsPcg *)nullptr);

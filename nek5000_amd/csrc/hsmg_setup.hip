@@ -955,7 +955,19 @@ int mg_setup(Mesh &mesh, const int *fbc_h, const int64_t *vertex, const double *
       rp[i + 1] = (int32_t)ci.size();
       std::vector<std::pair<int32_t, double>>().swap(rw);
     }
-    NK_TRY(mg.crs.setup(rp, ci, va, s));
+    // where the unknowns lie: any element's corner will do (level-1 node q of
+    // an element is its corner with bits r, s, t of q)
+    std::vector<double> at((size_t)(3 * ncrs));
+    for (int64_t q = 0; q < 8 * nel; ++q)
+      if (slot[(size_t)q] >= 0) {
+        const int64_t c = (q & 1 ? n - 1 : 0) + n * (q & 2 ? n - 1 : 0) +
+                          (int64_t)n * n * (q & 4 ? n - 1 : 0) + q / 8 * nxyz;
+        double *p = at.data() + 3 * (size_t)slot[(size_t)q];
+        p[0] = x[c];
+        p[1] = y[c];
+        p[2] = z[c];
+      }
+    NK_TRY(mg.crs.setup(rp, ci, va, at, s));
     NK_TRY(mg_dalloc(&mg.cb, ncrs));
     NK_TRY(mg_dalloc(&mg.cx, ncrs));
   }

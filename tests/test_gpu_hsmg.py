@@ -227,6 +227,55 @@ def test_flex_cg_amg_coarse_vcycle(gpu):
     F.destroy()
 
 
+@pytest.mark.parametrize("case", [
+    dict(nel=(15, 14, 15), lx1=4, deform=0.05),  # 2548 unknowns
+    dict(nel=(13, 15, 14), lx1=4, periodic_x=True),  # cuts across the period
+    dict(nel=(12, 14, 13), lx1=4, neumann_all=True),  # one unknown held
+])
+def test_h1mg_solve_dissected_coarse(gpu, case):
+    """Coarse problems large enough to be solved in parts with a separator
+    (smaller ones are one plain inverse): one V-cycle against the oracle's
+    exact factor."""
+    P, mg, F = build(gpu, case)
+    assert F.h1mg_info()["ncrs"] > 2300
+    rng = np.random.default_rng(12)
+    r = P.field.dssum(P.bm1 * rng.standard_normal(P.shape))
+    zo = mg.solve(r)
+    zd = F.zeros()
+    F.h1mg_solve(zd, F.to_dev(r))
+    e = l2rel(host(zd), zo)
+    say(f"[dissected coarse] {case} rel L2 = {e:.3e}")
+    assert e < 1e-10
+    F.destroy()
+
+
+def test_flex_cg_coarse_beyond_direct(gpu):
+    """A coarse problem too large for the direct solver goes through the
+    AMG-preconditioned CG: same iteration count as a smaller mesh whose
+    coarse problem is solved directly (multigrid, elements of one size)."""
+    its = []
+    for m in (20, 44):
+        b = box(m, 4, deform=0.05, lengths=(m / 20.0,) * 3)
+        F = gpu.box_field(b, multigrid=True)
+        one = F.zeros() + 1.0
+        rhs = F.mass()[0] * F.to_dev(np.random.default_rng(3).standard_normal(F.shape))
+        u = F.zeros()
+        out = F.hmholtz("PRES", u, rhs, one, F.zeros(), F.mask, F.mult, -1e-8, 100,
+                        params=gpu.default_params(param42=2, param21=-1e-8))
+        its.append((out["niter"], F.h1mg_info()["crs_avg_iters"]))
+        say(f"[coarse beyond direct] m={m} iterations, coarse iterations {its[-1]}")
+        assert out["converged"]
+        # the residual of the solution through the plain operator calls
+        w = F.zeros()
+        F.axhelm(w, u, one, F.zeros())
+        F.dssum(w)
+        res = host((rhs - w) * F.mask)
+        assert np.linalg.norm(res) < 1e-6 * np.linalg.norm(host(rhs))
+        F.destroy()
+    assert its[0][1] == 0.0 and its[1][1] > 2.0
+    assert abs(its[0][0] - its[1][0]) <= 3
+
+
 @pytest.mark.parametrize("case", [MG_CASES[0], MG_CASES[3], MG_CASES[6]])
 def test_gmres(gpu, case):
     """hmholtz('PRES') with param(42) = 0 -> hmh_gmres (gmres.f:304-545)."""
