@@ -17,8 +17,9 @@ static int wide_mask(int np) {
 #undef CALL
 }
 
-// Autotuner: on the first apply of an order on a mesh of at least 2^20
-// local nodes (and not inside a graph capture), time every kernel variant
+// Autotuner: on the first apply of an order and kind of coefficients
+// (constants or fields) on a mesh of at least 2^20 local nodes (and not
+// inside a graph capture), time every kernel variant
 // the order has (element- or plane-staged slabs; the orders whose NP x NP
 // slabs leave lanes idle also pack epb_wide slabs per block; NP = 8..16 also
 // the matrix-core contractions, element- or plane-group-staged) with two
@@ -30,7 +31,7 @@ static int wide_mask(int np) {
 // each.
 static int tune_axhelm(const Mesh &m, double *au, const double *u, Coef h1, Coef h2,
                        hipStream_t s) {
-  AxhelmChoice &ch = g_axhelm_choice[m.np];
+  AxhelmChoice &ch = g_axhelm_choice[axhelm_kind(h1, h2)][m.np];
   hipEvent_t e0, e1;
   NK_HIP(hipEventCreate(&e0));
   NK_HIP(hipEventCreate(&e1));
@@ -76,6 +77,7 @@ static int tune_axhelm(const Mesh &m, double *au, const double *u, Coef h1, Coef
     double *p = buf, *r = buf + n, *d = buf + 2 * n, *w = buf + 3 * n, *rho = buf + 4 * n;
     CgState *st = reinterpret_cast<CgState *>(buf + 4 * n + part);
     NK_HIP(hipMemsetAsync(buf, 0, bytes, s));
+    NK_HIP(hipMemsetAsync(&st->iter, 1, sizeof(int), s));  // past iteration 1: p is read
     float ms[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int c = 0; c < nv; ++c) {
       ch.variant_cg = vars[c];
@@ -114,8 +116,8 @@ static int tune_axhelm(const Mesh &m, double *au, const double *u, Coef h1, Coef
 
 int axhelm_autotune(const Mesh &m, double *au, const double *u, Coef h1, Coef h2,
                     hipStream_t s) {
-  if (m.np >= 2 && m.np <= kMaxNP && !g_axhelm_choice[m.np].tuned && m.n >= ((int64_t)1 << 20) &&
-      au != u) {
+  if (m.np >= 2 && m.np <= kMaxNP && !g_axhelm_choice[axhelm_kind(h1, h2)][m.np].tuned &&
+      m.n >= ((int64_t)1 << 20) && au != u) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     NK_HIP(hipStreamIsCapturing(s, &cs));
     if (cs == hipStreamCaptureStatusNone) NK_TRY(tune_axhelm(m, au, u, h1, h2, s));
@@ -129,9 +131,15 @@ int launch_axhelm(const Mesh &m, double *au, const double *u, Coef h1, Coef h2,
   return axhelm_apply(m, au, u, h1, h2, s);
 }
 
+// the choice reported for an order: that of constant coefficients, or of
+// fields where only those were tuned
+static const AxhelmChoice &reported(int np) {
+  return g_axhelm_choice[!g_axhelm_choice[0][np].tuned && g_axhelm_choice[1][np].tuned ? 1 : 0][np];
+}
+
 int axhelm_tuning(int np, int *variant, int *grid, int *tuned) {
   NK_CHECK(np >= 2 && np <= kMaxNP, NKH_ERR_ARG, "axhelm tuning: lx1=%d", np);
-  const AxhelmChoice &c = g_axhelm_choice[np];
+  const AxhelmChoice &c = reported(np);
   if (variant) *variant = c.variant;
   if (grid) *grid = c.grid;
   if (tuned) *tuned = c.tuned ? 1 : 0;
@@ -141,13 +149,14 @@ int axhelm_tuning(int np, int *variant, int *grid, int *tuned) {
 int axhelm_set_tuning(int np, int variant, int grid) {
   NK_CHECK(np >= 2 && np <= kMaxNP && variant >= 0 && variant <= 5 && grid >= 0,
            NKH_ERR_ARG, "axhelm tuning: lx1=%d variant=%d grid=%d", np, variant, grid);
-  g_axhelm_choice[np] = AxhelmChoice{variant, grid, variant, variant, true};
+  for (auto &kind : g_axhelm_choice)
+    kind[np] = AxhelmChoice{variant, grid, variant, variant, true};
   return NKH_OK;
 }
 
 int axhelm_tuning_fused(int np, int *variant_cg, int *variant_flex) {
   NK_CHECK(np >= 2 && np <= kMaxNP, NKH_ERR_ARG, "axhelm tuning: lx1=%d", np);
-  const AxhelmChoice &c = g_axhelm_choice[np];
+  const AxhelmChoice &c = reported(np);
   if (variant_cg) *variant_cg = c.variant_cg;
   if (variant_flex) *variant_flex = c.variant_flex;
   return NKH_OK;

@@ -752,10 +752,10 @@ int nkd_axhelm(int id, double *au, const double *u, const double *h1, const doub
   NK_TRY(ready(m, id, false));
   NK_CHECK(au && u && h1 && h2, NKH_ERR_ARG, "nkd_axhelm: null array");
   NK_CHECK(isd == 1 || isd == 2, NKH_ERR_ARG, "nkd_axhelm: isd=%d", isd);
-  Coef c1, c2;
-  NK_TRY(classify_coefs(*m, h1, h2, &c1, &c2, g_stream));
-  NK_TRY(launch_axhelm(*m, au, u, c1, c2, g_stream));
-  return NKH_OK;
+  // the coefficients are read as the fields they come as: telling whether they
+  // are constant takes a pass over them and a host wait, more than the apply
+  // saves (the product by a constant field is the product by the constant)
+  return launch_axhelm(*m, au, u, Coef{h1, 0.0}, Coef{h2, 0.0}, g_stream);
 }
 
 int nkh_axhelm_tuning(int lx1, int *variant, int *grid, int *tuned) {
@@ -818,9 +818,7 @@ int nkd_setprec(int id, double *d, const double *h1, const double *h2) {
   Mesh *m = get_mesh(id);
   NK_TRY(ready(m, id, true));
   NK_CHECK(d && h1 && h2, NKH_ERR_ARG, "nkd_setprec: null array");
-  Coef c1, c2;
-  NK_TRY(classify_coefs(*m, h1, h2, &c1, &c2, g_stream));
-  return run_setprec(*m, d, c1, c2, g_stream);
+  return run_setprec(*m, d, Coef{h1, 0.0}, Coef{h2, 0.0}, g_stream);
 }
 
 // Nek's defaults (reader_par.f:26-27,76-79,86-89,159-162): param(22) =
@@ -832,17 +830,18 @@ static const nkh_params kDefaultParams = {1, 0, 1.0e-7, 1.0e-7, 0, 0, 0.0, 0,
 // cggo from its head (hmholtz.f:611-653): the PRES branches copy f into x and
 // run hmh_gmres (param42 = 0) or hmh_flex_cg (param42 = 2) in place; other
 // fields take the Jacobi PCG.
-static int cggo_branches(Mesh &m, bool pres, double *x, const double *f, Coef c1, Coef c2,
-                         const double *mask, const double *mult, double tin, int maxit,
-                         const nkh_params &p, nkh_result *res, double *history, hipStream_t s) {
+static int cggo_branches(Mesh &m, bool pres, double *x, const double *f,
+                         const SolveFacts &facts, const double *mask, const double *mult,
+                         double tin, int maxit, const nkh_params &p, nkh_result *res,
+                         double *history, hipStream_t s) {
   if (pres) {
     NK_HIP(hipMemcpyAsync(x, f, sizeof(double) * m.n, hipMemcpyDeviceToDevice, s));
-    if (p.param42 == 0) return run_gmres(m, x, c1, c2, mult, mask, maxit, p, res, history);
+    if (p.param42 == 0) return run_gmres(m, x, facts, mult, mask, maxit, p, res, history);
     if (p.precision == 2)
-      return run_flex_cg_mixed(m, x, c1, c2, mult, mask, maxit, p, res, history);
-    return run_flex_cg(m, x, c1, c2, mult, mask, maxit, p, res, history);
+      return run_flex_cg_mixed(m, x, facts, mult, mask, maxit, p, res, history);
+    return run_flex_cg(m, x, facts, mult, mask, maxit, p, res, history);
   }
-  return run_cggo(m, x, f, c1, c2, mask, mult, tin, maxit, p, res, history);
+  return run_cggo(m, x, f, facts, mask, mult, tin, maxit, p, res, history);
 }
 
 static int check_solver_params(const nkh_params &p, bool pres, const char *who) {
@@ -868,9 +867,10 @@ int nkd_cggo(int id, double *x, const double *f, const double *h1, const double 
   const nkh_params &p = prm ? *prm : kDefaultParams;
   NK_CHECK(p.precision == 0 || p.precision == 2, NKH_ERR_UNSUPPORTED,
            "nkd_cggo: precision=%d", p.precision);
-  Coef c1, c2;
-  NK_TRY(classify_coefs(*m, h1, h2, &c1, &c2, g_stream));
-  return run_cggo(*m, x, f, c1, c2, mask, mult, tin, maxit, p, res, history);
+  SolveFacts facts;
+  NK_TRY(gather_facts(*m, h1, h2, mask, mult, const_cast<double *>(f), FactsAsk(), &facts,
+                      g_stream));
+  return run_cggo(*m, x, f, facts, mask, mult, tin, maxit, p, res, history);
 }
 
 int nkd_cggo_noalloc(int id, double *x, const double *f, const double *h1, const double *h2,
@@ -898,18 +898,22 @@ int nkd_hmholtz(int id, const char *name, double *u, double *rhs, const double *
   const bool pres = name && std::strncmp(name, "PRES", 4) == 0;
   NK_TRY(check_solver_params(p, pres, "nkd_hmholtz"));
   hipStream_t s = g_stream;
-  Coef c1, c2;
-  NK_TRY(classify_coefs(*m, h1, h2, &c1, &c2, s));
-  // hmholtz.f:50-51: dssum(rhs); rhs *= mask
+  // hmholtz.f:50-51: dssum(rhs); rhs *= mask (in the pass over the arrays)
   NK_TRY(gs_op(m->gs, rhs, 0, s));
-  NK_TRY(mul_inplace(rhs, mask, m->n, s));
+  const bool chk = !pres && (p.param22 == 0.0 || p.istep <= 10);
+  FactsAsk ask;
+  ask.mask_f = true;
+  ask.chk = chk;
+  if (pres) NK_TRY(mg_facts_ask(*m, &ask));
+  SolveFacts facts;
+  NK_TRY(gather_facts(*m, h1, h2, mask, mult, rhs, ask, &facts, s));
   // hmholtz.f:52-55's chktcg1 only sets cggo's tolerance, which the PRES
   // branches (hmholtz.f:639-653) do not read
-  if (pres) return cggo_branches(*m, true, u, rhs, c1, c2, mask, mult, 0.0, maxit, p, res, history, s);
   double tol = std::fabs(tli);
-  if (p.param22 == 0.0 || p.istep <= 10) NK_TRY(run_chktcg1(*m, &tol, rhs, c1, c2, mask, mult));
+  if (chk) NK_TRY(run_chktcg1(*m, &tol, facts));
   if (tli < 0) tol = tli;
-  return run_cggo(*m, u, rhs, c1, c2, mask, mult, tol, maxit, p, res, history);
+  return cggo_branches(*m, pres, u, rhs, facts, mask, mult, pres ? 0.0 : tol, maxit, p, res,
+                       history, s);
 }
 
 int nkd_hsolve(int id, const char *name, double *u, double *r, const double *h1,
@@ -945,13 +949,16 @@ int nkd_hsolve(int id, const char *name, double *u, double *r, const double *h1,
   NK_TRY(mul_inplace(r, vmk, m->n, s));
   NK_TRY(gs_op(m->gs, r, 0, s));
   NK_TRY(proj_project1(proj, r, h1, h2, vmk, vml, p.ifmvbd, nullptr, nullptr));
-  Coef c1, c2;
-  NK_TRY(classify_coefs(*m, h1, h2, &c1, &c2, s));
+  FactsAsk ask;
+  ask.chk = true;
+  if (pres) NK_TRY(mg_facts_ask(*m, &ask));
+  SolveFacts facts;
+  NK_TRY(gather_facts(*m, h1, h2, vmk, vml, r, ask, &facts, s));
   // hmhzpf (navier4.f:513-560): tol = tli or |param22|, chktcg1, cggo
   double t = tol;
   if (p.param22 != 0.0) t = std::fabs(p.param22);
-  NK_TRY(run_chktcg1(*m, &t, r, c1, c2, vmk, vml));
-  NK_TRY(cggo_branches(*m, pres, u, r, c1, c2, vmk, vml, t, maxit, p, res, history, s));
+  NK_TRY(run_chktcg1(*m, &t, facts));
+  NK_TRY(cggo_branches(*m, pres, u, r, facts, vmk, vml, t, maxit, p, res, history, s));
   return proj_project2(proj, u, h1, h2, vmk, vml);
 }
 
@@ -974,21 +981,23 @@ int nkd_hmholtz_batch(int batch, const nkh_batch_solve *solves, int maxit,
   nb = (int)meshes.size();
   hipStream_t s = g_stream;
   std::vector<const double *> x(nb), f(nb), mk(nb), mu(nb);
-  std::vector<Coef> c1(nb), c2(nb);
+  std::vector<SolveFacts> facts(nb);
   std::vector<double> tin(nb);
+  const bool chk = p.param22 == 0.0 || p.istep <= 10;
   for (int k = 0; k < nb; ++k) {
     Mesh *m = get_mesh(meshes[k]);
     NK_TRY(ready(m, meshes[k], true));
     const nkh_batch_solve &q = solves[k];
     NK_CHECK(q.u && q.rhs && q.h1 && q.h2 && q.mask && q.mult, NKH_ERR_ARG,
              "nkd_hmholtz_batch: null array in solve %d", k);
-    NK_TRY(classify_coefs(*m, q.h1, q.h2, &c1[k], &c2[k], s));
     // hmholtz.f:50-57: dssum(rhs); rhs *= mask; chktcg1; tli < 0 relative
     NK_TRY(gs_op(m->gs, q.rhs, 0, s));
-    NK_TRY(mul_inplace(q.rhs, q.mask, m->n, s));
+  }
+  NK_TRY(batch_facts(batch, solves, chk, facts.data(), s));
+  for (int k = 0; k < nb; ++k) {
+    const nkh_batch_solve &q = solves[k];
     double tol = std::fabs(q.tli);
-    if (p.param22 == 0.0 || p.istep <= 10)
-      NK_TRY(run_chktcg1(*m, &tol, q.rhs, c1[k], c2[k], q.mask, q.mult));
+    if (chk) NK_TRY(run_chktcg1(*get_mesh(meshes[k]), &tol, facts[k]));
     if (q.tli < 0) tol = q.tli;
     x[k] = q.u;
     f[k] = q.rhs;
@@ -996,7 +1005,7 @@ int nkd_hmholtz_batch(int batch, const nkh_batch_solve *solves, int maxit,
     mu[k] = q.mult;
     tin[k] = tol;
   }
-  return run_cggo_batch(batch, x.data(), f.data(), c1.data(), c2.data(), mk.data(), mu.data(),
+  return run_cggo_batch(batch, x.data(), f.data(), facts.data(), mk.data(), mu.data(),
                         tin.data(), maxit, p, res, graph_launches);
 }
 
@@ -1070,11 +1079,13 @@ int nkd_hmh_flex_cg(int id, double *res, const double *h1, const double *h2, con
   const nkh_params &p = prm ? *prm : kDefaultParams;
   NK_CHECK(p.precision >= 0 && p.precision <= 2, NKH_ERR_UNSUPPORTED,
            "nkd_hmh_flex_cg: precision=%d", p.precision);
-  Coef c1, c2;
-  NK_TRY(classify_coefs(*m, h1, h2, &c1, &c2, g_stream));
+  FactsAsk ask;
+  NK_TRY(mg_facts_ask(*m, &ask));
+  SolveFacts facts;
+  NK_TRY(gather_facts(*m, h1, h2, pmask, wt, res, ask, &facts, g_stream));
   if (p.precision == 2)
-    return run_flex_cg_mixed(*m, res, c1, c2, wt, pmask, maxit, p, out, rnorm_history);
-  return run_flex_cg(*m, res, c1, c2, wt, pmask, maxit, p, out, rnorm_history);
+    return run_flex_cg_mixed(*m, res, facts, wt, pmask, maxit, p, out, rnorm_history);
+  return run_flex_cg(*m, res, facts, wt, pmask, maxit, p, out, rnorm_history);
 }
 
 int nkd_hmh_gmres(int id, double *res, const double *h1, const double *h2, const double *wt,
@@ -1087,9 +1098,11 @@ int nkd_hmh_gmres(int id, double *res, const double *h1, const double *h2, const
   const nkh_params &p = prm ? *prm : kDefaultParams;
   NK_CHECK(p.precision == 0 || p.precision == 1, NKH_ERR_UNSUPPORTED,
            "nkd_hmh_gmres: precision=%d", p.precision);
-  Coef c1, c2;
-  NK_TRY(classify_coefs(*m, h1, h2, &c1, &c2, g_stream));
-  return run_gmres(*m, res, c1, c2, wt, pmask, maxit, p, out, rnorm_history);
+  FactsAsk ask;
+  NK_TRY(mg_facts_ask(*m, &ask));
+  SolveFacts facts;
+  NK_TRY(gather_facts(*m, h1, h2, pmask, wt, res, ask, &facts, g_stream));
+  return run_gmres(*m, res, facts, wt, pmask, maxit, p, out, rnorm_history);
 }
 
 int nkh_mg_info(int id, int *lmax, int *nh, int *ncrs, double *crs_avg_iters) {

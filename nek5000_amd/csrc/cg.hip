@@ -66,77 +66,131 @@ inline int upd_blocks(int64_t n) {
   return (int)(b < 64 ? 64 : (b > kUpdBlocks ? kUpdBlocks : b));
 }
 
-// ---- generic reductions (setup) ----------------------------------------
-// kind 0: sum a*b*c (c may be null -> 1, b may be null -> 1)
-// kind 1: max |a|   kind 2: max a   kind 3: min a
-__global__ void __launch_bounds__(256)
-    k_reduce(const double *__restrict__ a, const double *__restrict__ b,
-             const double *__restrict__ c, int64_t n, int kind, double *__restrict__ part) {
-  __shared__ double sb[4];
-  double v = (kind == 0 || kind == 1) ? 0.0 : (kind == 2 ? -INFINITY : INFINITY);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double x = a[i];
-    if (kind == 0) {
-      double t = x;
-      if (b) t = t * b[i];
-      if (c) t = t * c[i];
-      v += t;
-    } else if (kind == 1) {
-      v = fmax(v, fabs(x));
-    } else if (kind == 2) {
-      v = fmax(v, x);
-    } else {
-      v = fmin(v, x);
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    const double t = __shfl_down(v, o, 64);
-    if (kind == 0) v += t;
-    else if (kind == 3) v = fmin(v, t);
-    else v = fmax(v, t);
-  }
-  if ((threadIdx.x & 63) == 0) sb[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = sb[0];
-    for (int q = 1; q < 4; ++q) {
-      if (kind == 0) t += sb[q];
-      else if (kind == 3) t = fmin(t, sb[q]);
-      else t = fmax(t, sb[q]);
-    }
-    part[blockIdx.x] = t;
-  }
+// ---- what a solve has to know of its arrays (SolveFacts) -------------------
+// One pass over h1, h2, mask, mult, f and, where asked, binv (the sums of
+// chktcg1), another mask and the count codes of mult; f masked in place where
+// asked.  Bound by its streams (6 to 9 words per node: 149 us, 5.4 TB/s, on
+// 32,768 elements at lx1 = 8, where one reduction after another, each with
+// its own host wait, took 0.5 ms; on 336 elements 10 us).  kNF results per block, fixed grid; the sums by
+// one block in a fixed order.
+enum { kF_h1min, kF_h1max, kF_h2min, kF_h2max, kF_fmax, kF_fmasked, kF_skmin, kF_inner, kF_mgdiff,
+       kF_nocode, kF_rr, kF_bc1, kF_bc2, kNF };
+__host__ __device__ constexpr int fact_op(int q) {  // 0 sum, 1 min, 2 max
+  return (q == kF_h1min || q == kF_h2min || q == kF_skmin) ? 1 : (q >= kF_rr ? 0 : 2);
+}
+__device__ __forceinline__ double fact_join(int op, double a, double b) {
+  return op == 0 ? a + b : (op == 1 ? fmin(a, b) : fmax(a, b));
+}
+__device__ __forceinline__ double fact_start(int op) {
+  return op == 0 ? 0.0 : (op == 1 ? INFINITY : -INFINITY);
 }
 
 __global__ void __launch_bounds__(256)
-    k_reduce_final(const double *__restrict__ part, int count, int kind,
-                   double *__restrict__ out) {
+    k_facts(const double *__restrict__ h1, const double *__restrict__ h2,
+            const double *__restrict__ mask, const double *__restrict__ mult, double *f,
+            int mask_f, const double *__restrict__ binv, const double *__restrict__ other,
+            uint8_t *__restrict__ code, int64_t n, int np, double *__restrict__ part,
+            double *__restrict__ groups) {
+  __shared__ double sb[4][kNF];
+  __shared__ uint8_t s_in[kMaxNP * kMaxNP * kMaxNP];
+  const int np3 = np * np * np;
+  for (int q = threadIdx.x; q < np3; q += 256) {
+    const int i = q % np, j = (q / np) % np, k = q / (np * np);
+    s_in[q] = i > 0 && i < np - 1 && j > 0 && j < np - 1 && k > 0 && k < np - 1;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *groups = 0.0;  // gs_prepare runs after this
+  __syncthreads();
+  double v[kNF];
+#pragma unroll
+  for (int q = 0; q < kNF; ++q) v[q] = fact_start(fact_op(q));
+  v[kF_fmax] = v[kF_fmasked] = v[kF_inner] = v[kF_mgdiff] = v[kF_nocode] = 0.0;
+  const int64_t i0 = blockIdx.x * (int64_t)256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+  int at = (int)(i0 % np3);
+  const int step = (int)(stride % np3);
+  for (int64_t i = i0; i < n; i += stride) {
+    const double a1 = h1[i], a2 = h2[i], m = mask[i], u = mult[i];
+    v[kF_h1min] = fmin(v[kF_h1min], a1);
+    v[kF_h1max] = fmax(v[kF_h1max], a1);
+    v[kF_h2min] = fmin(v[kF_h2min], a2);
+    v[kF_h2max] = fmax(v[kF_h2max], a2);
+    v[kF_skmin] = fmin(v[kF_skmin], m);
+    if (s_in[at]) v[kF_inner] = fmax(v[kF_inner], fmax(fabs(m - 1.0), fabs(u - 1.0)));
+    at += step;
+    at -= at >= np3 ? np3 : 0;
+    double fi = 0.0;
+    if (f) {
+      fi = f[i];
+      if (mask_f) {
+        fi = fi * m;
+        f[i] = fi;
+      }
+      v[kF_fmax] = fmax(v[kF_fmax], fabs(fi));
+      if (m == 0.0) v[kF_fmasked] = fmax(v[kF_fmasked], fabs(fi));
+    }
+    if (binv) {
+      v[kF_rr] += ((binv[i] * fi) * fi) * u;
+      v[kF_bc1] += m * u;
+      v[kF_bc2] += u;
+    }
+    if (other && other[i] != m) v[kF_mgdiff] = 1.0;
+    if (code) {
+      const double c = u > 0.0 ? rint(1.0 / u) : 0.0;
+      const bool ok = c >= 1.0 && c <= 255.0 && 1.0 / c == u;
+      code[i] = ok ? (uint8_t)c : (uint8_t)0;
+      if (!ok) v[kF_nocode] = 1.0;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kNF; ++q) {
+    for (int o = 32; o > 0; o >>= 1)
+      v[q] = fact_join(fact_op(q), v[q], __shfl_down(v[q], o, 64));
+    if ((threadIdx.x & 63) == 0) sb[threadIdx.x >> 6][q] = v[q];
+  }
+  __syncthreads();
+  if (threadIdx.x < kNF) {
+    const int q = threadIdx.x, op = fact_op(q);
+    double t = sb[0][q];
+    for (int w = 1; w < 4; ++w) t = fact_join(op, t, sb[w][q]);
+    part[(int64_t)q * kRedBlocks + blockIdx.x] = t;
+  }
+}
+
+// block q: result q over the count partials
+__global__ void __launch_bounds__(256)
+    k_facts_final(const double *__restrict__ part, int count, double *__restrict__ out) {
   __shared__ double sb[4];
-  double v = (kind == 0 || kind == 1) ? 0.0 : (kind == 2 ? -INFINITY : INFINITY);
-  for (int q = threadIdx.x; q < count; q += blockDim.x) {
-    const double x = part[q];
-    if (kind == 0) v += x;
-    else if (kind == 3) v = fmin(v, x);
-    else v = fmax(v, x);
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    const double t = __shfl_down(v, o, 64);
-    if (kind == 0) v += t;
-    else if (kind == 3) v = fmin(v, t);
-    else v = fmax(v, t);
-  }
+  const int q = blockIdx.x, op = fact_op(q);
+  double v = fact_start(op);
+  for (int t = threadIdx.x; t < count; t += 256)
+    v = fact_join(op, v, part[(int64_t)q * kRedBlocks + t]);
+  for (int o = 32; o > 0; o >>= 1) v = fact_join(op, v, __shfl_down(v, o, 64));
   if ((threadIdx.x & 63) == 0) sb[threadIdx.x >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
     double t = sb[0];
-    for (int q = 1; q < 4; ++q) {
-      if (kind == 0) t += sb[q];
-      else if (kind == 3) t = fmin(t, sb[q]);
-      else t = fmax(t, sb[q]);
-    }
-    *out = t;
+    for (int w = 1; w < 4; ++w) t = fact_join(op, t, sb[w]);
+    out[q] = t;
   }
+}
+
+// partial sums of a*a*b
+__global__ void __launch_bounds__(256)
+    k_sq_sum(const double *__restrict__ a, const double *__restrict__ b, int64_t n,
+             double *__restrict__ part) {
+  __shared__ double sb[4];
+  double v = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    v += (a[i] * a[i]) * b[i];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) sb[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = ((sb[0] + sb[1]) + sb[2]) + sb[3];
+}
+__global__ void __launch_bounds__(1024)
+    k_sum_final(const double *__restrict__ part, int count, double *__restrict__ out) {
+  const double t = block_sum_array(part, count);
+  if (threadIdx.x == 0) *out = t;
 }
 
 // ---- elementwise ----------------------------------------------------------
@@ -155,26 +209,36 @@ __global__ void k_inv(double *__restrict__ a, int64_t n) {
        i += (int64_t)gridDim.x * blockDim.x)
     a[i] = 1.0 / a[i];
 }
-// r = f, x = 0, p = 0; dm = d*mult; bm = binv*mult (or mult when param18=1)
-__global__ void k_cg_init(double *__restrict__ x, double *__restrict__ r,
-                          double *__restrict__ p, const double *__restrict__ f,
-                          const double *__restrict__ d, const double *__restrict__ mult,
-                          const double *__restrict__ binv, double *__restrict__ dm,
-                          double *__restrict__ bm, int plain_norm, int64_t n) {
+// d = 1/d (the assembled diagonal); r = f, x = 0; dm = d*mult; bm = binv*mult
+// (or mult when param18=1); and the first iteration's partial sums (those of
+// k_cg_update_dots without an update)
+__global__ void __launch_bounds__(256)
+    k_cg_init(double *__restrict__ x, double *__restrict__ r, const double *__restrict__ f,
+              double *__restrict__ d, const double *__restrict__ mult,
+              const double *__restrict__ binv, double *__restrict__ dm,
+              double *__restrict__ bm, int plain_norm, int64_t n, double *__restrict__ part1,
+              double *__restrict__ part2) {
+  double s1 = 0.0, s2 = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    r[i] = f[i];
+    const double di = 1.0 / d[i], mu = mult[i], fi = f[i];
+    const double a = di * mu, b = plain_norm ? mu : binv[i] * mu;
+    d[i] = di;
+    r[i] = fi;
     x[i] = 0.0;
-    p[i] = 0.0;
-    dm[i] = d[i] * mult[i];
-    bm[i] = plain_norm ? mult[i] : binv[i] * mult[i];
+    dm[i] = a;
+    bm[i] = b;
+    const double rr = fi * fi;
+    s1 += a * rr;
+    s2 += b * rr;
   }
+  block_store2(s1, s2, part1, part2);
 }
 
-// x += alpha p ; r -= alpha w (when an update is pending) ; partial sums of
-// (d*r)*r*mult and binv*mult*r*r (vlsc3 / vlsc32, hmholtz.f:754-759).
+// x += alpha p ; r -= alpha w (the update of the previous iteration) ; partial
+// sums of (d*r)*r*mult and binv*mult*r*r (vlsc3 / vlsc32, hmholtz.f:754-759).
 // VEC: 16-byte loads of node pairs (all six arrays 16-byte aligned).
-template <bool VEC, bool UPD>
+template <bool VEC>
 __global__ void __launch_bounds__(256)
     k_cg_update_dots(double *__restrict__ x, double *__restrict__ r,
                      const double *__restrict__ p, const double *__restrict__ w,
@@ -182,9 +246,6 @@ __global__ void __launch_bounds__(256)
                      const CgState *__restrict__ st, double *__restrict__ part1,
                      double *__restrict__ part2) {
   if (st->done) return;
-  // UPD: the host launches the update variant for every iteration after the
-  // first; a pending update exists exactly then (or the solve is done).
-  constexpr bool upd = UPD;
   const double alpha = st->alpha;
   double s1 = 0.0, s2 = 0.0;
   const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -202,16 +263,14 @@ __global__ void __launch_bounds__(256)
     const v2 *bm2 = reinterpret_cast<const v2 *>(bm);
     for (int64_t i = tid; i < n2; i += stride) {
       v2 ri = __builtin_nontemporal_load(r2 + i);
-      if constexpr (upd) {
-        v2 xi = __builtin_nontemporal_load(x2 + i);
-        const v2 pi = __builtin_nontemporal_load(p2 + i), wi = __builtin_nontemporal_load(w2 + i);
-        xi.x = xi.x + alpha * pi.x;
-        xi.y = xi.y + alpha * pi.y;
-        ri.x = ri.x + (-alpha) * wi.x;
-        ri.y = ri.y + (-alpha) * wi.y;
-        __builtin_nontemporal_store(xi, x2 + i);
-        __builtin_nontemporal_store(ri, r2 + i);
-      }
+      v2 xi = __builtin_nontemporal_load(x2 + i);
+      const v2 pi = __builtin_nontemporal_load(p2 + i), wi = __builtin_nontemporal_load(w2 + i);
+      xi.x = xi.x + alpha * pi.x;
+      xi.y = xi.y + alpha * pi.y;
+      ri.x = ri.x + (-alpha) * wi.x;
+      ri.y = ri.y + (-alpha) * wi.y;
+      __builtin_nontemporal_store(xi, x2 + i);
+      __builtin_nontemporal_store(ri, r2 + i);
       const v2 d = __builtin_nontemporal_load(dm2 + i), b = __builtin_nontemporal_load(bm2 + i);
       const double rr0 = ri.x * ri.x, rr1 = ri.y * ri.y;
       s1 += d.x * rr0;
@@ -222,12 +281,9 @@ __global__ void __launch_bounds__(256)
     done_upto = n2 * 2;
   }
   for (int64_t i = done_upto + tid; i < n; i += stride) {
-    double ri = r[i];
-    if constexpr (upd) {
-      x[i] = x[i] + alpha * p[i];
-      ri = ri + (-alpha) * w[i];
-      r[i] = ri;
-    }
+    x[i] = x[i] + alpha * p[i];
+    const double ri = r[i] + (-alpha) * w[i];
+    r[i] = ri;
     const double rr = ri * ri;
     s1 += dm[i] * rr;
     s2 += bm[i] * rr;
@@ -315,29 +371,6 @@ __global__ void k_mask_guarded(double *__restrict__ w, const double *__restrict_
     w[i] = w[i] * mask[i];
 }
 
-// max(|mask-1|, |mult-1|) over element-interior nodes and max |f| over
-// masked nodes, one partial per block
-__global__ void __launch_bounds__(256)
-    k_fused_checks(const double *__restrict__ mask, const double *__restrict__ mult,
-                   const double *__restrict__ f, int64_t n, int np,
-                   double *__restrict__ part) {
-  __shared__ double sb[4];
-  const int64_t np3 = (int64_t)np * np * np;
-  double v = 0.0;
-  for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; l < n;
-       l += (int64_t)gridDim.x * blockDim.x) {
-    const int q = (int)(l % np3);
-    const int i = q % np, j = (q / np) % np, k = q / (np * np);
-    if (i > 0 && i < np - 1 && j > 0 && j < np - 1 && k > 0 && k < np - 1)
-      v = fmax(v, fmax(fabs(mask[l] - 1.0), fabs(mult[l] - 1.0)));
-    if (f && mask[l] == 0.0) v = fmax(v, fabs(f[l]));
-  }
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
-  if ((threadIdx.x & 63) == 0) sb[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = fmax(fmax(sb[0], sb[1]), fmax(sb[2], sb[3]));
-}
-
 // ---- mixed precision: FP32 iteration, FP64 solution and true residual ----
 // The Jacobi PCG iterates in single precision (r, p, w, the correction xs
 // accumulated since the last refresh, the preconditioner; FP32 operator),
@@ -378,7 +411,7 @@ inline int refresh_blocks(int64_t n) {
 }
 
 // xs += alpha p ; r -= alpha w (FP32) ; FP64 partials of dm*r*r and bm*r*r
-template <bool VEC, bool UPD>
+template <bool VEC>
 __global__ void __launch_bounds__(256)
     k_mcg_update_dots(float *__restrict__ xs, float *__restrict__ r,
                       const float *__restrict__ p, const float *__restrict__ w,
@@ -402,20 +435,18 @@ __global__ void __launch_bounds__(256)
     const v4 *b4 = reinterpret_cast<const v4 *>(bm);
     for (int64_t i = tid; i < n4; i += stride) {
       v4 ri = __builtin_nontemporal_load(r4 + i);
-      if constexpr (UPD) {
-        v4 xi = __builtin_nontemporal_load(x4 + i);
-        const v4 pi = __builtin_nontemporal_load(p4 + i), wi = __builtin_nontemporal_load(w4 + i);
-        xi.x += alpha * pi.x;
-        xi.y += alpha * pi.y;
-        xi.z += alpha * pi.z;
-        xi.w += alpha * pi.w;
-        ri.x -= alpha * wi.x;
-        ri.y -= alpha * wi.y;
-        ri.z -= alpha * wi.z;
-        ri.w -= alpha * wi.w;
-        __builtin_nontemporal_store(xi, x4 + i);
-        __builtin_nontemporal_store(ri, r4 + i);
-      }
+      v4 xi = __builtin_nontemporal_load(x4 + i);
+      const v4 pi = __builtin_nontemporal_load(p4 + i), wi = __builtin_nontemporal_load(w4 + i);
+      xi.x += alpha * pi.x;
+      xi.y += alpha * pi.y;
+      xi.z += alpha * pi.z;
+      xi.w += alpha * pi.w;
+      ri.x -= alpha * wi.x;
+      ri.y -= alpha * wi.y;
+      ri.z -= alpha * wi.z;
+      ri.w -= alpha * wi.w;
+      __builtin_nontemporal_store(xi, x4 + i);
+      __builtin_nontemporal_store(ri, r4 + i);
       const v4 d = __builtin_nontemporal_load(d4 + i), b = __builtin_nontemporal_load(b4 + i);
       const double q0 = (double)ri.x * ri.x, q1 = (double)ri.y * ri.y,
                    q2 = (double)ri.z * ri.z, q3 = (double)ri.w * ri.w;
@@ -425,12 +456,9 @@ __global__ void __launch_bounds__(256)
     done_upto = n4 * 4;
   }
   for (int64_t i = done_upto + tid; i < n; i += stride) {
-    float ri = r[i];
-    if constexpr (UPD) {
-      xs[i] = xs[i] + alpha * p[i];
-      ri = ri - alpha * w[i];
-      r[i] = ri;
-    }
+    xs[i] = xs[i] + alpha * p[i];
+    const float ri = r[i] - alpha * w[i];
+    r[i] = ri;
     const double q = (double)ri * ri;
     s1 += dm[i] * q;
     s2 += bm[i] * q;
@@ -550,24 +578,32 @@ __global__ void __launch_bounds__(kScalThreads)
   st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
 }
 
-// x = 0, xs = 0, p = 0, r = f (rounded), d, d*mult and binv*mult (or mult)
-// in FP32
-__global__ void k_mcg_init(double *__restrict__ x, float *__restrict__ xs,
-                           float *__restrict__ p, float *__restrict__ r,
-                           float *__restrict__ d32, float *__restrict__ dm,
-                           float *__restrict__ bm, const double *__restrict__ f,
-                           const double *__restrict__ d, const double *__restrict__ mult,
-                           const double *__restrict__ binv, int plain_norm, int64_t n) {
+// x = 0, xs = 0, r = f (rounded), and 1/d (d the assembled diagonal), its
+// product with mult and binv*mult (or mult) in FP32; the first iteration's
+// partial sums
+__global__ void __launch_bounds__(256)
+    k_mcg_init(double *__restrict__ x, float *__restrict__ xs, float *__restrict__ r,
+               float *__restrict__ d32, float *__restrict__ dm, float *__restrict__ bm,
+               const double *__restrict__ f, const double *__restrict__ d,
+               const double *__restrict__ mult, const double *__restrict__ binv, int plain_norm,
+               int64_t n, double *__restrict__ part1, double *__restrict__ part2) {
+  double s1 = 0.0, s2 = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
+    const double di = 1.0 / d[i], mu = mult[i];
+    const float a = (float)(di * mu), b = (float)(plain_norm ? mu : binv[i] * mu);
+    const float ri = (float)f[i];
     x[i] = 0.0;
     xs[i] = 0.0f;
-    p[i] = 0.0f;
-    r[i] = (float)f[i];
-    d32[i] = (float)d[i];
-    dm[i] = (float)(d[i] * mult[i]);
-    bm[i] = (float)(plain_norm ? mult[i] : binv[i] * mult[i]);
+    r[i] = ri;
+    d32[i] = (float)di;
+    dm[i] = a;
+    bm[i] = b;
+    const double q = (double)ri * ri;
+    s1 += a * q;
+    s2 += b * q;
   }
+  block_store2(s1, s2, part1, part2);
 }
 
 int grid_for(int64_t n) {
@@ -575,20 +611,6 @@ int grid_for(int64_t n) {
   if (g > 8192) g = 8192;
   if (g < 1) g = 1;
   return (int)g;
-}
-
-// Reduce on the device and read the scalar back (synchronous).
-int reduce_host(const Mesh &m, const double *a, const double *b, const double *c, int64_t n,
-                int kind, double *out, hipStream_t s) {
-  NK_CHECK(m.red != nullptr, NKH_ERR_STATE, "reduction buffer not allocated");
-  hipLaunchKernelGGL(k_reduce, dim3(kRedBlocks), dim3(256), 0, s, a, b, c, n, kind,
-                     m.red + kRedScratch);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, s, m.red + kRedScratch, kRedBlocks,
-                     kind, m.red + kRedOut);
-  NK_HIP(hipGetLastError());
-  NK_HIP(hipMemcpyAsync(out, m.red + kRedOut, sizeof(double), hipMemcpyDeviceToHost, s));
-  NK_HIP(hipStreamSynchronize(s));
-  return NKH_OK;
 }
 
 }  // namespace
@@ -614,28 +636,57 @@ int ensure_workspace(Mesh &m) {
   return NKH_OK;
 }
 
-// Reduce a coefficient field to a uniform value when it is constant (the
-// multiply by the scalar is then bit-identical to the multiply by the field).
-static int classify(Mesh &m, const double *f, Coef *c, hipStream_t s) {
-  NK_TRY(ensure_small(m));
-  double mn, mx;
-  NK_TRY(reduce_host(m, f, nullptr, nullptr, m.n, 3, &mn, s));
-  NK_TRY(reduce_host(m, f, nullptr, nullptr, m.n, 2, &mx, s));
-  if (mn == mx) {
-    c->f = nullptr;
-    c->s = mn;
-  } else {
-    c->f = f;
-    c->s = 0.0;
-  }
+// The passes of gather_facts on s: partial sums in red, the kNF + 1 results
+// at red + kRedOut, the group flags of mask in flag.
+static int enqueue_facts(Mesh &m, const double *h1, const double *h2, const double *mask,
+                         const double *mult, double *f, const FactsAsk &ask, double *red,
+                         uint8_t *flag, hipStream_t s) {
+  static_assert(kNF * kRedBlocks <= kRedRho2, "the partial sums take the dots' place");
+  double *part = red + kRedPart1, *res = red + kRedOut;
+  const int64_t per = 1024;  // nodes per block, up to the fixed grid
+  const int nb = (int)std::min<int64_t>(std::max<int64_t>((m.n + per - 1) / per, 1), kRedBlocks);
+  hipLaunchKernelGGL(k_facts, dim3(nb), dim3(256), 0, s, h1, h2, mask, mult, f,
+                     ask.mask_f ? 1 : 0, ask.chk ? m.binv : nullptr, ask.other_mask, ask.code,
+                     m.n, m.np, part, res + kNF);
+  NK_TRY(gs_prepare(m.gs, mask, mult, flag, res + kNF, s));
+  hipLaunchKernelGGL(k_facts_final, dim3(kNF), dim3(256), 0, s, part, nb, res);
+  NK_HIP(hipGetLastError());
   return NKH_OK;
 }
 
-int classify_coefs(Mesh &m, const double *h1, const double *h2, Coef *c1, Coef *c2,
-                   hipStream_t s) {
-  NK_TRY(classify(m, h1, c1, s));
-  // setfast (hmholtz.f:303-305): ifh2 = vlamax(h2) > 0; a uniform 0 drops the term
-  NK_TRY(classify(m, h2, c2, s));
+// the facts from the kNF + 1 results (on the host)
+static SolveFacts read_facts(const Mesh &m, const double *h1, const double *h2, const double *h) {
+  SolveFacts o;
+  o.h1min = h[kF_h1min];
+  o.h1max = h[kF_h1max];
+  o.h2min = h[kF_h2min];
+  o.h2max = h[kF_h2max];
+  o.fmax = h[kF_fmax];
+  o.fmasked = h[kF_fmasked];
+  o.skmin = h[kF_skmin];
+  o.inner = h[kF_inner];
+  o.mgdiff = h[kF_mgdiff];
+  o.nocode = h[kF_nocode];
+  o.rr = h[kF_rr];
+  o.bcneu1 = h[kF_bc1];
+  o.bcneu2 = h[kF_bc2];
+  o.groups = m.gs.ngroups > 0 ? h[kNF] : 1.0;  // no ids at all: never fused
+  o.h1 = h1;
+  o.h2 = h2;
+  o.interior_zero = m.gs.interior_zero;
+  return o;
+}
+
+int gather_facts(Mesh &m, const double *h1, const double *h2, const double *mask,
+                 const double *mult, double *f, const FactsAsk &ask, SolveFacts *out,
+                 hipStream_t s) {
+  NK_TRY(ensure_small(m));
+  if (!m.gs.flag && m.gs.ngroups > 0) NK_HIP(hipMalloc(&m.gs.flag, (size_t)m.gs.ngroups));
+  NK_TRY(enqueue_facts(m, h1, h2, mask, mult, f, ask, m.red, m.gs.flag, s));
+  double h[kNF + 1];
+  NK_HIP(hipMemcpyAsync(h, m.red + kRedOut, sizeof(h), hipMemcpyDeviceToHost, s));
+  NK_HIP(hipStreamSynchronize(s));
+  *out = read_facts(m, h1, h2, h);
   return NKH_OK;
 }
 
@@ -645,61 +696,44 @@ int mul_inplace(double *a, const double *b, int64_t n, hipStream_t s) {
   return NKH_OK;
 }
 
-int run_setprec(Mesh &m, double *d, Coef h1, Coef h2, hipStream_t s) {
+// the assembled Jacobi diagonal, not inverted
+static int setprec_sum(Mesh &m, double *d, Coef h1, Coef h2, hipStream_t s) {
   NK_TRY(launch_setprec(m, d, h1, h2, s));
-  NK_TRY(gs_op(m.gs, d, 0, s));
+  return gs_op(m.gs, d, 0, s);
+}
+
+int run_setprec(Mesh &m, double *d, Coef h1, Coef h2, hipStream_t s) {
+  NK_TRY(setprec_sum(m, d, h1, h2, s));
   hipLaunchKernelGGL(k_inv, dim3(grid_for(m.n)), dim3(256), 0, s, d, m.n);
   NK_HIP(hipGetLastError());
   return NKH_OK;
 }
 
-// The conditions under which a CG denominator (mask * QQ^T w, p)_mult may be
-// taken as sum_l p_l w_l before the assembly: ids zero exactly at element
-// interiors, mask 1 and mult 1 there, f (when given) zero where masked, and
-// per group a 0/1 mask and mult summing to 1.  Leaves the group flags of
-// gs_prepare in m.gs.
-int fused_conditions(Mesh &m, const double *mask, const double *mult, const double *f, bool *ok,
-                     hipStream_t s) {
-  *ok = false;
-  if (!m.gs.interior_zero) return NKH_OK;
-  NK_TRY(ensure_small(m));
-  hipLaunchKernelGGL(k_fused_checks, dim3(kRedBlocks), dim3(256), 0, s, mask, mult, f, m.n, m.np,
-                     m.red + kRedScratch);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, s, m.red + kRedScratch, kRedBlocks,
-                     2, m.red + kRedOut);
-  NK_HIP(hipGetLastError());
-  double dev;
-  NK_HIP(hipMemcpyAsync(&dev, m.red + kRedOut, sizeof(double), hipMemcpyDeviceToHost, s));
-  NK_HIP(hipStreamSynchronize(s));
-  if (dev != 0.0) return NKH_OK;
-  return gs_prepare(m.gs, mask, mult, m.red + kRedScratch, ok, s);
-}
-
-int run_chktcg1(Mesh &m, double *tol, const double *res, Coef h1, Coef h2,
-                const double *mask, const double *mult) {
+int run_chktcg1(Mesh &m, double *tol, const SolveFacts &facts) {
   hipStream_t s = cur_stream();
-  NK_TRY(ensure_workspace(m));
   const int64_t n = m.n;
-  double *w1 = m.ws, *w2 = m.ws + n;
   const double eps = 1.0e-13, acondno = 10.0;
-  double a;
   // rinit = sqrt(glsc3(binv*res, res, mult)/vol)
-  hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(256), 0, s, w1, 1.0, n);
-  NK_HIP(hipMemcpyAsync(w2, m.binv, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-  hipLaunchKernelGGL(k_mul, dim3(grid_for(n)), dim3(256), 0, s, w2, res, n);
-  NK_TRY(reduce_host(m, w2, res, mult, n, 0, &a, s));
-  const double rinit = std::sqrt(a / m.vol);
+  const double rinit = std::sqrt(facts.rr / m.vol);
   const double rmin = eps * rinit;
   if (*tol < rmin) *tol = rmin;
-  double bcneu1, bcneu2;
-  NK_TRY(reduce_host(m, w1, mask, mult, n, 0, &bcneu1, s));
-  NK_TRY(reduce_host(m, w1, w1, mult, n, 0, &bcneu2, s));
-  const double bctest = std::fabs(bcneu1 - bcneu2);
-  NK_TRY(launch_axhelm(m, w2, w1, h1, h2, s));
+  const double bctest = std::fabs(facts.bcneu1 - facts.bcneu2);
+  // the operator's action on constants matters where no node is masked
+  if (!(bctest < 0.1)) return NKH_OK;
+  NK_TRY(ensure_workspace(m));
+  double *w1 = m.ws, *w2 = m.ws + n;
+  hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(256), 0, s, w1, 1.0, n);
+  NK_TRY(launch_axhelm(m, w2, w1, facts.c1(), facts.c2(), s));
+  hipLaunchKernelGGL(k_sq_sum, dim3(kRedBlocks), dim3(256), 0, s, w2, m.bm1, n,
+                     m.red + kRedScratch);
+  hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(1024), 0, s, m.red + kRedScratch, kRedBlocks,
+                     m.red + kRedOut);
+  NK_HIP(hipGetLastError());
   double sq;
-  NK_TRY(reduce_host(m, w2, w2, m.bm1, n, 0, &sq, s));
+  NK_HIP(hipMemcpyAsync(&sq, m.red + kRedOut, sizeof(double), hipMemcpyDeviceToHost, s));
+  NK_HIP(hipStreamSynchronize(s));
   const double bcrob = std::sqrt(sq / m.vol);
-  if (bctest < 0.1 && bcrob < eps * acondno) {
+  if (bcrob < eps * acondno) {
     const double tolmin = rinit * eps * 10.0;
     if (*tol < tolmin) *tol = tolmin;
   }
@@ -725,8 +759,8 @@ struct CgRun {
   // choice of the fused iteration, device state.  ws: 6 n doubles, red:
   // kRedSize doubles, st: the state; all on stream s (host waits).
   int begin(Mesh &mesh, double *ws, double *red_, CgState *st_, double *x_, const double *f,
-            Coef h1_, Coef h2_, const double *mask_, const double *mult_, double tin, int maxit,
-            const nkh_params &prm, bool want_hist, hipStream_t s) {
+            const SolveFacts &facts, const double *mask_, const double *mult_, double tin,
+            int maxit, const nkh_params &prm, bool want_hist, hipStream_t s) {
     m = &mesh;
     const int64_t n = mesh.n;
     x = x_;
@@ -738,34 +772,33 @@ struct CgRun {
     bm = ws + 5 * n;
     red = red_;
     st = st_;
-    h1 = h1_;
-    h2 = h2_;
+    h1 = facts.c1();
+    h2 = facts.c2();
     mask = mask_;
     mult = mult_;
     double tol = std::fabs(tin);
     if (prm.restol != 0.0) tol = prm.restol;
     if (tin < 0) tol = std::fabs(tin);
     niter = maxit < kMaxCg ? maxit : kMaxCg;
-    NK_TRY(run_setprec(mesh, d, h1, h2, s));
-    hipLaunchKernelGGL(k_cg_init, dim3(grid_for(n)), dim3(256), 0, s, x, r, p, f, d, mult,
-                       mesh.binv, dm, bm, prm.param18 == 1 ? 1 : 0, n);
-    NK_HIP(hipGetLastError());
-    double fmax;
-    NK_TRY(reduce_host(mesh, f, nullptr, nullptr, n, 1, &fmax, s));
-    trivial = fmax == 0.0;
-    if (trivial) return NKH_OK;
+    trivial = facts.fmax == 0.0;
+    if (trivial) {
+      hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(256), 0, s, x, 0.0, n);
+      NK_HIP(hipGetLastError());
+      return NKH_OK;
+    }
     // null-space check (hmholtz.f:705-720): pure Neumann with h2 == 0
-    double h2max, skmin;
-    if (h2.uniform()) h2max = h2.s;
-    else NK_TRY(reduce_host(mesh, h2.f, nullptr, nullptr, n, 2, &h2max, s));
-    NK_TRY(reduce_host(mesh, mask, nullptr, nullptr, n, 3, &skmin, s));
-    NK_CHECK(!(skmin > 0 && h2max == 0), NKH_ERR_UNSUPPORTED,
+    NK_CHECK(!(facts.skmin > 0 && facts.h2max == 0), NKH_ERR_UNSUPPORTED,
              "cggo: pure-Neumann mean correction (ifmcor) is not implemented");
+    // the operator's kernel choice for this order (w is scratch until then)
+    NK_TRY(axhelm_autotune(mesh, w, f, h1, h2, s));
+    NK_TRY(setprec_sum(mesh, d, h1, h2, s));
+    hipLaunchKernelGGL(k_cg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, r, f, d, mult,
+                       mesh.binv, dm, bm, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
+                       red + kRedPart2);
+    NK_HIP(hipGetLastError());
     // Fused iteration (rho inside axhelm, mask inside the assembly) when its
-    // conditions hold: ids zero exactly at element interiors, mask 1 and
-    // mult 1 there, f zero where masked, and per group a 0/1 mask and mult
-    // summing to 1.  Checked once per solve.
-    NK_TRY(fused_conditions(mesh, mask, mult, f, &fused, s));
+    // conditions hold and f is zero where masked.
+    fused = facts.fused() && facts.fmasked == 0.0;
     flag = mesh.gs.flag;
     ax_grid_parts = axhelm_cg_grid(mesh);
     auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
@@ -796,12 +829,10 @@ struct CgRun {
     const int64_t n = m->n;
     double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1,
            *rho2 = red + kRedRho2;
-    auto kern = vec_ok ? (launched == 0 ? k_cg_update_dots<true, false>
-                                        : k_cg_update_dots<true, true>)
-                       : (launched == 0 ? k_cg_update_dots<false, false>
-                                        : k_cg_update_dots<false, true>);
     const int ub = upd_blocks(n);
-    hipLaunchKernelGGL(kern, dim3(ub), dim3(256), 0, s, x, r, p, w, dm, bm, n, st, part1, part2);
+    if (launched > 0)  // (the first iteration's sums come from k_cg_init)
+      hipLaunchKernelGGL((vec_ok ? k_cg_update_dots<true> : k_cg_update_dots<false>), dim3(ub),
+                         dim3(256), 0, s, x, r, p, w, dm, bm, n, st, part1, part2);
     hipLaunchKernelGGL(k_cg_scalars1, dim3(1), dim3(kScalThreads), 0, s, st, part1, part2, ub,
                        hist);
     if (fused) {
@@ -859,11 +890,13 @@ struct McgRun {
   double *hist = nullptr;
 
   int begin(Mesh &mesh, double *ws, double *red_, void *st_, double *x_, const double *f_,
-            Coef h1_, Coef h2_, const double *mask, const double *mult, double tin, int maxit,
-            const nkh_params &prm, bool want_hist, hipStream_t s) {
+            const SolveFacts &facts, const double *mask, const double *mult, double tin,
+            int maxit, const nkh_params &prm, bool want_hist, hipStream_t s) {
     m = &mesh;
     const int64_t n = mesh.n;
-    NK_CHECK(h1_.uniform() && h2_.uniform(), NKH_ERR_UNSUPPORTED,
+    h1 = facts.c1();
+    h2 = facts.c2();
+    NK_CHECK(h1.uniform() && h2.uniform(), NKH_ERR_UNSUPPORTED,
              "mixed-precision cggo: h1 and h2 must be uniform");
     x = x_;
     f = f_;
@@ -880,30 +913,28 @@ struct McgRun {
     red = red_;
     ms = static_cast<McgState *>(st_);
     st = &ms->cg;
-    h1 = h1_;
-    h2 = h2_;
     double tol = std::fabs(tin);
     if (prm.restol != 0.0) tol = prm.restol;
     if (tin < 0) tol = std::fabs(tin);
     niter = maxit < kMaxCg ? maxit : kMaxCg;
-    NK_TRY(run_setprec(mesh, ax, h1, h2, s));  // d (FP64) in the ax slot
-    hipLaunchKernelGGL(k_mcg_init, dim3(grid_for(n)), dim3(256), 0, s, x, xs, p, r, d, dm, bm, f,
-                       ax, mult, mesh.binv, prm.param18 == 1 ? 1 : 0, n);
-    NK_HIP(hipGetLastError());
-    double fmax;
-    NK_TRY(reduce_host(mesh, f, nullptr, nullptr, n, 1, &fmax, s));
-    trivial = fmax == 0.0;
-    if (trivial) return NKH_OK;
-    double skmin;
-    NK_TRY(reduce_host(mesh, mask, nullptr, nullptr, n, 3, &skmin, s));
-    NK_CHECK(!(skmin > 0 && h2.s == 0.0), NKH_ERR_UNSUPPORTED,
+    trivial = facts.fmax == 0.0;
+    if (trivial) {
+      hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(256), 0, s, x, 0.0, n);
+      NK_HIP(hipGetLastError());
+      return NKH_OK;
+    }
+    NK_CHECK(!(facts.skmin > 0 && h2.s == 0.0), NKH_ERR_UNSUPPORTED,
              "cggo: pure-Neumann mean correction (ifmcor) is not implemented");
-    bool ok = false;
-    NK_TRY(fused_conditions(mesh, mask, mult, f, &ok, s));
-    NK_CHECK(ok, NKH_ERR_UNSUPPORTED,
+    NK_CHECK(facts.fused() && facts.fmasked == 0.0, NKH_ERR_UNSUPPORTED,
              "mixed-precision cggo: needs ids zero at element interiors, 0/1 masks and "
              "mult summing to 1 per group");
     flag = mesh.gs.flag;
+    NK_TRY(axhelm_autotune(mesh, ax, f, h1, h2, s));  // the refreshes' operator
+    NK_TRY(setprec_sum(mesh, ax, h1, h2, s));  // the diagonal (FP64) in the ax slot
+    hipLaunchKernelGGL(k_mcg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, r, d, dm, bm, f,
+                       ax, mult, mesh.binv, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
+                       red + kRedPart2);
+    NK_HIP(hipGetLastError());
     NK_TRY(ensure_geom32(mesh, s));
     ax_grid_parts = axhelm_cg_grid(mesh);
     auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
@@ -933,12 +964,10 @@ struct McgRun {
     const int64_t n = m->n;
     double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1,
            *rho2 = red + kRedRho2;
-    auto kern = vec_ok ? (launched == 0 ? k_mcg_update_dots<true, false>
-                                        : k_mcg_update_dots<true, true>)
-                       : (launched == 0 ? k_mcg_update_dots<false, false>
-                                        : k_mcg_update_dots<false, true>);
     const int ub = upd_blocks(n);
-    hipLaunchKernelGGL(kern, dim3(ub), dim3(256), 0, s, xs, r, p, w, dm, bm, n, st, part1, part2);
+    if (launched > 0)  // (the first iteration's sums come from k_mcg_init)
+      hipLaunchKernelGGL((vec_ok ? k_mcg_update_dots<true> : k_mcg_update_dots<false>), dim3(ub),
+                         dim3(256), 0, s, xs, r, p, w, dm, bm, n, st, part1, part2);
     hipLaunchKernelGGL(k_mcg_scalars1, dim3(1), dim3(kScalThreads), 0, s, ms, part1, part2, ub,
                        hist);
     // the refresh (its kernels return at once while the gate is closed)
@@ -984,13 +1013,14 @@ size_t cg_ws_doubles(int64_t n) {
 namespace {
 
 template <class Run>
-int drive_cggo(Mesh &m, double *x, const double *f, Coef h1, Coef h2, const double *mask,
-               const double *mult, double tin, int maxit, const nkh_params &prm,
-               nkh_result *res, double *history_host, bool allow_timers = true) {
+int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
+               const double *mask, const double *mult, double tin, int maxit,
+               const nkh_params &prm, nkh_result *res, double *history_host,
+               bool allow_timers = true) {
   hipStream_t s = cur_stream();
   NK_TRY(ensure_workspace(m));
   Run run;
-  NK_TRY(run.begin(m, m.ws, m.red, m.st, x, f, h1, h2, mask, mult, tin, maxit, prm,
+  NK_TRY(run.begin(m, m.ws, m.red, m.st, x, f, facts, mask, mult, tin, maxit, prm,
                    history_host != nullptr, s));
   if (run.trivial) {
     run.result(CgState{}, res);
@@ -1053,12 +1083,12 @@ int drive_cggo(Mesh &m, double *x, const double *f, Coef h1, Coef h2, const doub
 
 }  // namespace
 
-int run_cggo(Mesh &m, double *x, const double *f, Coef h1, Coef h2, const double *mask,
+int run_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts, const double *mask,
              const double *mult, double tin, int maxit, const nkh_params &prm,
              nkh_result *res, double *history_host) {
   if (prm.precision == 2)
-    return drive_cggo<McgRun>(m, x, f, h1, h2, mask, mult, tin, maxit, prm, res, history_host);
-  return drive_cggo<CgRun>(m, x, f, h1, h2, mask, mult, tin, maxit, prm, res, history_host);
+    return drive_cggo<McgRun>(m, x, f, facts, mask, mult, tin, maxit, prm, res, history_host);
+  return drive_cggo<CgRun>(m, x, f, facts, mask, mult, tin, maxit, prm, res, history_host);
 }
 
 // ---------------------------------------------------------------------------
@@ -1120,9 +1150,10 @@ int run_cggo_noalloc(Mesh &m, double *x, const double *f, const double *h1, cons
   v.red = sp + kNoAllocWs;
   v.st = reinterpret_cast<CgState *>(sp + kNoAllocWs + kNoAllocRed);
   v.gs.flag = reinterpret_cast<uint8_t *>(sp + kNoAllocWs + kNoAllocRed + kNoAllocState);
-  Coef c1, c2;
-  NK_TRY(classify_coefs(v, h1, h2, &c1, &c2, cur_stream()));
-  return drive_cggo<CgRun>(v, x, f, c1, c2, mask, mult, tin, maxit, prm, res, history_host,
+  SolveFacts facts;
+  NK_TRY(gather_facts(v, h1, h2, mask, mult, const_cast<double *>(f), FactsAsk(), &facts,
+                      cur_stream()));
+  return drive_cggo<CgRun>(v, x, f, facts, mask, mult, tin, maxit, prm, res, history_host,
                            false);
 }
 
@@ -1252,11 +1283,38 @@ int batch_destroy(int id) {
   return NKH_OK;
 }
 
+int batch_facts(int id, const nkh_batch_solve *solves, bool chk, SolveFacts *out,
+                hipStream_t s) {
+  NK_CHECK(id >= 0 && id < (int)g_batches.size() && g_batches[(size_t)id], NKH_ERR_ARG,
+           "batch: bad handle %d", id);
+  CgBatch &B = *g_batches[(size_t)id];
+  std::vector<double> h((size_t)B.nb * (kNF + 1));
+  FactsAsk ask;
+  ask.mask_f = true;
+  ask.chk = chk;
+  for (int k = 0; k < B.nb; ++k) {
+    Mesh *m = get_mesh(B.mesh[(size_t)k]);
+    NK_CHECK(m && m->n > 0, NKH_ERR_STATE, "batch: mesh of solve %d is gone", k);
+    NK_CHECK(m->gs.ngroups == B.nflag[(size_t)k], NKH_ERR_STATE,
+             "batch: the gather-scatter map of solve %d changed", k);
+    const nkh_batch_solve &q = solves[k];
+    NK_TRY(enqueue_facts(*m, q.h1, q.h2, q.mask, q.mult, q.rhs, ask, B.red[(size_t)k],
+                         B.flag[(size_t)k], s));
+    NK_HIP(hipMemcpyAsync(&h[(size_t)k * (kNF + 1)], B.red[(size_t)k] + kRedOut,
+                          sizeof(double) * (kNF + 1), hipMemcpyDeviceToHost, s));
+  }
+  NK_HIP(hipStreamSynchronize(s));
+  for (int k = 0; k < B.nb; ++k)
+    out[k] = read_facts(*get_mesh(B.mesh[(size_t)k]), solves[k].h1, solves[k].h2,
+                        &h[(size_t)k * (kNF + 1)]);
+  return NKH_OK;
+}
+
 namespace {
 
 template <class Run>
-int batch_drive(CgBatch &B, const double *const *x, const double *const *f, const Coef *h1,
-                const Coef *h2, const double *const *mask, const double *const *mult,
+int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
+                const SolveFacts *facts, const double *const *mask, const double *const *mult,
                 const double *tin, int maxit, const nkh_params &prm, nkh_result *res,
                 int *launches_out) {
   hipStream_t s = cur_stream();
@@ -1265,18 +1323,12 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f, cons
   for (int k = 0; k < B.nb; ++k) {
     Mesh *m = get_mesh(B.mesh[(size_t)k]);
     NK_CHECK(m && m->n > 0, NKH_ERR_STATE, "batch: mesh of solve %d is gone", k);
-    NK_CHECK(m->gs.ngroups == B.nflag[(size_t)k], NKH_ERR_STATE,
-             "batch: the gather-scatter map of solve %d changed", k);
-    // set-up of solve k on s (it uses the mesh's scratch reductions)
+    // set-up of solve k on s
     NK_TRY(runs[(size_t)k].begin(*m, B.ws[(size_t)k], B.red[(size_t)k], B.st[(size_t)k],
-                                 const_cast<double *>(x[k]), f[k], h1[k], h2[k], mask[k],
-                                 mult[k], tin[k], maxit, prm, false, s));
+                                 const_cast<double *>(x[k]), f[k], facts[k], mask[k], mult[k],
+                                 tin[k], maxit, prm, false, s));
     if (runs[(size_t)k].trivial) continue;
-    if (runs[(size_t)k].fused && m->gs.ngroups > 0) {
-      NK_HIP(hipMemcpyAsync(B.flag[(size_t)k], m->gs.flag, (size_t)m->gs.ngroups,
-                            hipMemcpyDeviceToDevice, s));
-      runs[(size_t)k].flag = B.flag[(size_t)k];
-    }
+    if (m->gs.ngroups > 0) runs[(size_t)k].flag = B.flag[(size_t)k];
     active.push_back(k);
   }
   // the first iteration (no pending update) eagerly, then the graph; all of
@@ -1357,16 +1409,16 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f, cons
 
 }  // namespace
 
-int run_cggo_batch(int id, const double *const *x, const double *const *f, const Coef *h1,
-                   const Coef *h2, const double *const *mask, const double *const *mult,
-                   const double *tin, int maxit, const nkh_params &prm, nkh_result *res,
-                   int *launches_out) {
+int run_cggo_batch(int id, const double *const *x, const double *const *f,
+                   const SolveFacts *facts, const double *const *mask,
+                   const double *const *mult, const double *tin, int maxit,
+                   const nkh_params &prm, nkh_result *res, int *launches_out) {
   NK_CHECK(id >= 0 && id < (int)g_batches.size() && g_batches[(size_t)id], NKH_ERR_ARG,
            "batch: bad handle %d", id);
   CgBatch &B = *g_batches[(size_t)id];
   if (prm.precision == 2)
-    return batch_drive<McgRun>(B, x, f, h1, h2, mask, mult, tin, maxit, prm, res, launches_out);
-  return batch_drive<CgRun>(B, x, f, h1, h2, mask, mult, tin, maxit, prm, res, launches_out);
+    return batch_drive<McgRun>(B, x, f, facts, mask, mult, tin, maxit, prm, res, launches_out);
+  return batch_drive<CgRun>(B, x, f, facts, mask, mult, tin, maxit, prm, res, launches_out);
 }
 
 }  // namespace nekamd

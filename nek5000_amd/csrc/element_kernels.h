@@ -111,9 +111,11 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
   __shared__ double s_red[NP2 * EPB];
 
   double beta = 0.0;
+  bool first = false;  // MODE 1, iteration 1: p has no value yet and is not read
   if constexpr (MODE == 1) {
     if (st->done) return;
     beta = st->beta;
+    first = st->iter <= 1;
   }
   double alpha = 0.0;  // MODE 2 with xacc: x += alpha p (the previous p)
   if constexpr (MODE == 2) {
@@ -143,7 +145,7 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
         const int64_t l = base + k * NP2;
         if constexpr (MODE == 1) {
           // add2s1: p = beta*p + z, z = r*d
-          v = beta * ldnt(uin + l) + ldnt(dinv + l) * ldnt(r + l);
+          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
           stnt(v, pout + l);
         } else if constexpr (MODE == 2) {
           const double po = ldnt(uin + l);
@@ -244,9 +246,11 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
   __shared__ double s_ws[EPB][NP2];
   __shared__ double s_red[NP2 * EPB];
   double beta = 0.0;
+  bool first = false;  // MODE 1, iteration 1: p has no value yet and is not read
   if constexpr (MODE == 1) {
     if (st->done) return;
     beta = st->beta;
+    first = st->iter <= 1;
   }
   double alpha = 0.0;  // MODE 2 with xacc: x += alpha p (the previous p)
   if constexpr (MODE == 2) {
@@ -273,7 +277,7 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
       if (valid) {
         const int64_t l = base + k * NP2;
         if constexpr (MODE == 1) {
-          v = beta * ldnt(uin + l) + ldnt(dinv + l) * ldnt(r + l);
+          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
           stnt(v, pout + l);
         } else if constexpr (MODE == 2) {
           const double po = ldnt(uin + l);
@@ -408,9 +412,11 @@ __global__ void __launch_bounds__(mx_threads<NP>())
   __shared__ double s_wr[PK * NP];  // ur, then wr
   __shared__ double s_ws[PK * NP];  // us, then ws
   double beta = 0.0;
+  bool first = false;  // MODE 1, iteration 1: p has no value yet and is not read
   if constexpr (MODE == 1) {
     if (st->done) return;
     beta = st->beta;
+    first = st->iter <= 1;
   }
   double alpha = 0.0;  // MODE 2 with xacc: x += alpha p (the previous p)
   if constexpr (MODE == 2) {
@@ -446,7 +452,7 @@ __global__ void __launch_bounds__(mx_threads<NP>())
       if (own) {
         const int64_t l = base + k * NP2;
         if constexpr (MODE == 1) {
-          v = beta * ldnt(uin + l) + ldnt(dinv + l) * ldnt(r + l);
+          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
           stnt(v, pout + l);
         } else if constexpr (MODE == 2) {
           const double po = ldnt(uin + l);
@@ -593,9 +599,11 @@ __global__ void __launch_bounds__(mx_threads<NP>())
   __shared__ double s_wr[G * PP];  // ur, then wr
   __shared__ double s_ws[G * PP];  // us, then ws
   double beta = 0.0;
+  bool first = false;  // MODE 1, iteration 1: p has no value yet and is not read
   if constexpr (MODE == 1) {
     if (st->done) return;
     beta = st->beta;
+    first = st->iter <= 1;
   }
   double alpha = 0.0;  // MODE 2 with xacc: x += alpha p (the previous p)
   if constexpr (MODE == 2) {
@@ -630,7 +638,7 @@ __global__ void __launch_bounds__(mx_threads<NP>())
       if (own) {
         const int64_t l = base + k * NP2;
         if constexpr (MODE == 1) {
-          v = beta * ldnt(uin + l) + ldnt(dinv + l) * ldnt(r + l);
+          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
           stnt(v, pout + l);
         } else if constexpr (MODE == 2) {
           const double po = ldnt(uin + l);
@@ -775,7 +783,10 @@ struct AxhelmChoice {
   int variant_flex = 0;  // MODE 2
   bool tuned = false;
 };
-inline AxhelmChoice g_axhelm_choice[kMaxNP + 1];
+// by kind of coefficients (0: h1 and h2 both constant, 1: a field among them,
+// which adds one or two streams) and order
+inline AxhelmChoice g_axhelm_choice[2][kMaxNP + 1];
+inline int axhelm_kind(Coef h1, Coef h2) { return h1.uniform() && h2.uniform() ? 0 : 1; }
 
 // One launch of the axhelm kernel (element- or plane-staged, EPB slabs per
 // block; MX 1 or 2: the matrix-core kernel staging the element or groups of
@@ -855,7 +866,7 @@ static int axhelm_dispatch(const Mesh &m, double *au, const double *u, Coef h1, 
                            double *xacc = nullptr, const double *alphap = nullptr) {
   DMat<NP> Dm;
   for (int t = 0; t < NP * NP; ++t) Dm.d[t] = m.D[t];
-  const AxhelmChoice ch = g_axhelm_choice[NP];
+  const AxhelmChoice ch = g_axhelm_choice[axhelm_kind(h1, h2)][NP];
   const int var = MODE == 1 ? ch.variant_cg : (MODE == 2 ? ch.variant_flex : ch.variant);
   const int gc = ch.grid;
 #define NK_GO(PLANE_, EPB_)                                                                  \

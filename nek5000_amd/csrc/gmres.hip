@@ -126,13 +126,15 @@ __global__ void k_gm_zero(double *__restrict__ x, int64_t n) {
 
 }  // namespace
 
-int run_gmres(Mesh &m, double *res, Coef h1, Coef h2, const double *wt, const double *mask,
-              int maxit, const nkh_params &prm, nkh_result *out, double *rnorm_history) {
+int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
+              const double *mask, int maxit, const nkh_params &prm, nkh_result *out,
+              double *rnorm_history) {
   NK_CHECK(m.mg, NKH_ERR_STATE, "hmh_gmres needs the multigrid hierarchy (nkh_mg_setup)");
   NK_CHECK(prm.param40 == 0 || prm.param40 == 1, NKH_ERR_UNSUPPORTED,
            "hmh_gmres: coarse solver param40=%d (0 exact, 1 one AMG V-cycle)", prm.param40);
   Mg &mg = *m.mg;
   hipStream_t s = cur_stream();
+  const Coef h1 = facts.c1(), h2 = facts.c2();
   const int64_t n = m.n;
   const int M = kGmresM;
   if (!mg.gV) {
@@ -150,7 +152,7 @@ int run_gmres(Mesh &m, double *res, Coef h1, Coef h2, const double *wt, const do
   const bool nullsp = mg_null_space_on(mg, h2);
   // hmholtz.f-style tolerance (gmres.f:352-356)
   double tolps = 0.0;
-  NK_TRY(run_chktcg1(m, &tolps, res, h1, h2, mask, wt));
+  NK_TRY(run_chktcg1(m, &tolps, facts));
   if (prm.param21 > 0 && tolps > std::fabs(prm.param21)) tolps = std::fabs(prm.param21);
   if (prm.istep == 0) tolps = 1.e-4;
   double tolpss = tolps;

@@ -402,48 +402,59 @@ __global__ void __launch_bounds__(256)
 // Group flags from mask and mult, plus the check that makes the fused CG
 // exact: in every group mask is 0 or 1 and equal at all members, and the
 // members' mult sum to 1 (then sum_l mult*w*p over the assembled, masked w
-// equals sum_l w_local*p for a masked, continuous p).  part[b] = 0 when the
-// block's groups pass.
+// equals sum_l w_local*p for a masked, continuous p).  One wavefront per
+// packet like the assembly (97 -> 79 us on 32,768 elements at lx1 =
+// 8 against one thread per group).
+__global__ void __launch_bounds__(256)
+    k_gs_prepare_pk(const double *__restrict__ mask, const double *__restrict__ mult,
+                    const int32_t *__restrict__ pk_m, const int32_t *__restrict__ pk_g,
+                    const uint64_t *__restrict__ pk_head, const int32_t *__restrict__ idx,
+                    int64_t npk, uint8_t *__restrict__ flag, double *__restrict__ bad) {
+  const int p = pk_index();
+  if (p >= npk) return;
+  const PkLane L = pk_lane(pk_m, pk_head, idx, p);
+  const double m = L.act ? mask[L.node] : 0.0;
+  const double sm = pk_reduce(L.act ? mult[L.node] : 0.0, L, AddComb());
+  const double m0 = __shfl(m, L.head, 64);
+  const bool off = L.act && (m != m0 || !(m0 == 0.0 || m0 == 1.0) || sm != 1.0);
+  if (L.act && L.head == (int)(threadIdx.x & 63))
+    flag[pk_g[p] + L.local] = (m0 == 0.0) ? 1 : (L.len >= 2 ? 0 : 2);
+  if (__ballot(off) != 0 && (threadIdx.x & 63) == 0) *bad = 1.0;
+}
+
+// one thread per group, groups [g0, ngroups) (those of more than 64 members)
 __global__ void __launch_bounds__(256)
     k_gs_prepare(const double *__restrict__ mask, const double *__restrict__ mult,
-                 const int32_t *__restrict__ off, const int32_t *__restrict__ idx,
-                 int64_t ngroups, uint8_t *__restrict__ flag, double *__restrict__ part) {
-  __shared__ double sbuf[4];
-  double bad = 0.0;
-  for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < ngroups;
+                 const int32_t *__restrict__ off, const int32_t *__restrict__ idx, int64_t g0,
+                 int64_t ngroups, uint8_t *__restrict__ flag, double *__restrict__ bad) {
+  for (int64_t s = g0 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < ngroups;
        s += (int64_t)gridDim.x * blockDim.x) {
     const int32_t a = off[s], e = off[s + 1];
     const double m0 = mask[idx[a]];
     double sm = 0.0;
+    bool o = false;
     for (int32_t q = a; q < e; ++q) {
       const int32_t l = idx[q];
-      if (mask[l] != m0) bad = 1.0;
+      o = o || mask[l] != m0;
       sm += mult[l];
     }
-    if (!(m0 == 0.0 || m0 == 1.0) || sm != 1.0) bad = 1.0;
+    if (o || !(m0 == 0.0 || m0 == 1.0) || sm != 1.0) *bad = 1.0;
     flag[s] = (m0 == 0.0) ? 1 : ((e - a >= 2) ? 0 : 2);
   }
-  for (int o = 32; o > 0; o >>= 1) bad = fmax(bad, __shfl_down(bad, o, 64));
-  if ((threadIdx.x & 63) == 0) sbuf[threadIdx.x >> 6] = bad;
-  __syncthreads();
-  if (threadIdx.x == 0)
-    part[blockIdx.x] = fmax(fmax(sbuf[0], sbuf[1]), fmax(sbuf[2], sbuf[3]));
 }
 
-int gs_prepare(GsMap &gs, const double *mask, const double *mult, double *red, bool *ok,
-               hipStream_t s) {
-  *ok = false;
+int gs_prepare(const GsMap &gs, const double *mask, const double *mult, uint8_t *flag,
+               double *bad, hipStream_t s) {
   if (gs.ngroups == 0) return NKH_OK;
-  if (!gs.flag) NK_HIP(hipMalloc(&gs.flag, (size_t)gs.ngroups));
-  hipLaunchKernelGGL(k_gs_prepare, dim3(kRedBlocks), dim3(256), 0, s, mask, mult, gs.off,
-                     gs.idx, gs.ngroups, gs.flag, red);
+  if (gs.npk > 0)
+    hipLaunchKernelGGL(k_gs_prepare_pk, dim3(pk_blocks(gs.npk)), dim3(256), 0, s, mask, mult,
+                       gs.pk_m, gs.pk_g, gs.pk_head, gs.idx, gs.npk, flag, bad);
+  const int64_t nbig = gs.ngroups - gs.gpk;
+  if (nbig > 0)
+    hipLaunchKernelGGL(k_gs_prepare, dim3((int)std::min<int64_t>((nbig + 255) / 256, 65536)),
+                       dim3(256), 0, s, mask, mult, gs.off, gs.idx, gs.gpk, gs.ngroups, flag,
+                       bad);
   NK_HIP(hipGetLastError());
-  std::vector<double> h(kRedBlocks);
-  NK_HIP(hipMemcpyAsync(h.data(), red, sizeof(double) * kRedBlocks, hipMemcpyDeviceToHost, s));
-  NK_HIP(hipStreamSynchronize(s));
-  double bad = 0.0;
-  for (double v : h) bad = std::max(bad, v);
-  *ok = (bad == 0.0);
   return NKH_OK;
 }
 

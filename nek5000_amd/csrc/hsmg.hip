@@ -673,8 +673,6 @@ __global__ void k_crs_scatter(double *__restrict__ e, const double *__restrict__
   }
 }
 
-__global__ void k_zero_int(int *flag) { *flag = 0; }
-
 // the held coarse unknown's right-hand side: 0
 __global__ void k_crs_pin(double *b, int pin) { b[pin] = 0.0; }
 
@@ -720,13 +718,6 @@ __global__ void __launch_bounds__(256) k_ortho_sub(double *__restrict__ v, int64
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
     v[i] -= m;
-}
-
-// 1 where a != b (flag set, never cleared here)
-__global__ void k_neq(const double *a, const double *b, int64_t n, int *flag) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    if (a[i] != b[i]) atomicOr(flag, 1);
 }
 
 // The local solves with the six contractions on the matrix cores: one wave
@@ -1403,20 +1394,9 @@ __global__ void __launch_bounds__(256)
 // The multiplicity weights wt (Nek's vmult = 1/dssum(1)) read from a byte
 // per node: code c holds wt = 1/c exactly (1/c in FP64 is the value Nek
 // computes), 1/8 of the weight array's traffic in the two streaming kernels
-// of every iteration.  k_wt_code builds the codes and flags any weight that
-// is not 1/c for a count c in 1..255 (then the FP64 weights are read).
-__global__ void k_wt_code(const double *__restrict__ wt, uint8_t *__restrict__ code, int64_t n,
-                          int *bad) {
-  int b = 0;
-  NK_GRID_LOOP(i, n) {
-    const double w = wt[i];
-    const double c = w > 0.0 ? rint(1.0 / w) : 0.0;
-    const bool ok = c >= 1.0 && c <= 255.0 && 1.0 / c == w;
-    code[i] = ok ? (uint8_t)c : (uint8_t)0;
-    b |= ok ? 0 : 1;
-  }
-  if (b) atomicOr(bad, 1);
-}
+// of every iteration.  The pass over the solve's arrays (gather_facts) makes
+// the codes and tells of any weight that is not 1/c for a count c in 1..255
+// (then the FP64 weights are read).
 __device__ __forceinline__ double wt_at(const double *__restrict__ w, int64_t i) {
   return __builtin_nontemporal_load(w + i);
 }
@@ -1555,35 +1535,31 @@ __global__ void __launch_bounds__(256) k_fcg_rnorm(FcgState *st, const double *p
 
 }  // namespace
 
-int mg_wt_codes(Mg &mg, const double *wt, int64_t n, hipStream_t s, const uint8_t **codes) {
-  // the flag after the n code bytes
-  const int64_t wt8_flag = (n + 7) / 8 * 8;
-  if (!mg.wt8) NK_HIP(hipMalloc(&mg.wt8, (size_t)wt8_flag + sizeof(int)));
-  int *wt8_bad = reinterpret_cast<int *>(mg.wt8 + wt8_flag);
-  hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, s, wt8_bad);
-  hipLaunchKernelGGL(k_wt_code, dim3(mg_grid(n)), dim3(256), 0, s, wt, mg.wt8, n, wt8_bad);
-  NK_HIP(hipGetLastError());
-  int wbad = 1;
-  NK_HIP(hipMemcpyAsync(&wbad, wt8_bad, sizeof(int), hipMemcpyDeviceToHost, s));
-  NK_HIP(hipStreamSynchronize(s));
-  *codes = wbad ? nullptr : mg.wt8;
+int mg_facts_ask(Mesh &m, FactsAsk *ask) {
+  NK_CHECK(m.mg, NKH_ERR_STATE, "the pressure solvers need the multigrid hierarchy (nkh_mg_setup)");
+  Mg &mg = *m.mg;
+  if (!mg.wt8) NK_HIP(hipMalloc(&mg.wt8, (size_t)std::max<int64_t>(m.n, 1)));
+  ask->chk = true;
+  ask->other_mask = mg.lev[mg.lmax].mask;
+  ask->code = mg.wt8;
   return NKH_OK;
 }
 
-int run_flex_cg(Mesh &m, double *res, Coef h1, Coef h2, const double *wt, const double *mask,
-                int maxit, const nkh_params &prm, nkh_result *out, double *rnorm_history) {
+int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
+                const double *mask, int maxit, const nkh_params &prm, nkh_result *out,
+                double *rnorm_history) {
   NK_CHECK(m.mg, NKH_ERR_STATE, "hmh_flex_cg needs the multigrid hierarchy (nkh_mg_setup)");
   NK_CHECK(prm.param40 == 0 || prm.param40 == 1, NKH_ERR_UNSUPPORTED,
            "hmh_flex_cg: coarse solver param40=%d (0 exact, 1 one AMG V-cycle)", prm.param40);
   Mg &mg = *m.mg;
   hipStream_t s = cur_stream();
+  const Coef h1 = facts.c1(), h2 = facts.c2();
   const int64_t n = m.n;
   // (the mixed solver allocates fr..fw on its own, so each piece is checked)
   if (!mg.fr)
     for (double **p : {&mg.fr, &mg.fp, &mg.fz, &mg.fw}) NK_TRY(mg_dalloc(p, n));
   if (!mg.fpart) NK_TRY(mg_dalloc(&mg.fpart, 3 * kFcgBlocks));
   if (!mg.fst) NK_HIP(hipMalloc(&mg.fst, sizeof(FcgState)));
-  if (!mg.fflag) NK_HIP(hipMalloc(&mg.fflag, sizeof(int)));
   const double *mgmask = mg.lev[mg.lmax].mask;
   double *r = mg.fr, *p = mg.fp, *z = mg.fz, *w = mg.fw;
   double *pa = mg.fpart, *pb = mg.fpart + kFcgBlocks;
@@ -1592,25 +1568,20 @@ int run_flex_cg(Mesh &m, double *res, Coef h1, Coef h2, const double *wt, const 
   NK_TRY(axhelm_autotune(m, w, res, h1, h2, s));
   // hmholtz.f:2205-2208: tolps from chktcg1 (pmask, vmult), capped by param(21)
   double tolps = 0.0;
-  NK_TRY(run_chktcg1(m, &tolps, res, h1, h2, mask, wt));
+  NK_TRY(run_chktcg1(m, &tolps, facts));
   if (prm.param21 > 0 && tolps > std::fabs(prm.param21)) tolps = std::fabs(prm.param21);
   if (prm.istep == 0) tolps = 1.e-4;
   const dim3 g(kFcgBlocks), b(256);
   // r stays masked by the update (w carries pmask) when pmask is the
   // multigrid's fine mask; otherwise it is masked again before every V-cycle
   // as h1mg_solve does
-  int differ = 0;
-  hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, s, mg.fflag);
-  hipLaunchKernelGGL(k_neq, dim3(mg_grid(n)), b, 0, s, mask, mgmask, n, mg.fflag);
-  NK_HIP(hipMemcpyAsync(&differ, mg.fflag, sizeof(int), hipMemcpyDeviceToHost, s));
+  const bool differ = facts.mgdiff != 0.0;
   // the weights as counts, when every one is 1/count
-  const uint8_t *wtc = nullptr;
-  NK_TRY(mg_wt_codes(mg, wt, n, s, &wtc));
+  const uint8_t *wtc = facts.nocode == 0.0 ? mg.wt8 : nullptr;
   // den inside the fused axhelm (p . A_L p) and the mask inside the
   // assembly, when the conditions for that identity hold (p = beta p + z
   // is continuous and zero where pmask is when pmask is the fine mask)
-  bool fused = false;
-  if (!differ) NK_TRY(fused_conditions(m, mask, wt, nullptr, &fused, s));
+  const bool fused = !differ && facts.fused();
   double *rho_part = m.red + kRedRho1;
   const int nrho = axhelm_cg_grid(m);
   hipLaunchKernelGGL(k_fcg_init, g, b, 0, s, r, res, p, wt, mgmask, n, pa);

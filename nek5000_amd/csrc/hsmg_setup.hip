@@ -574,7 +574,7 @@ void mg_free(Mesh &mesh) {
   for (void *p : {(void *)mg->fbc, (void *)mg->slot, (void *)mg->goff, (void *)mg->gidx,
                   (void *)mg->cb, (void *)mg->cx, (void *)mg->fr, (void *)mg->fp,
                   (void *)mg->fz, (void *)mg->fw, (void *)mg->fpart, (void *)mg->fst,
-                  (void *)mg->fflag, (void *)mg->gV, (void *)mg->gZ, (void *)mg->gx,
+                  (void *)mg->gV, (void *)mg->gZ, (void *)mg->gx,
                   (void *)mg->gr, (void *)mg->gw, (void *)mg->gpart, (void *)mg->gsm,
                   (void *)mg->xr, (void *)mg->xp, (void *)mg->xz, (void *)mg->xw,
                   (void *)mg->xx, (void *)mg->xwt, (void *)mg->xpart, mg->xst,

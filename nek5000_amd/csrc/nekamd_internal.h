@@ -218,6 +218,38 @@ struct Coef {
   bool uniform() const { return f == nullptr; }
 };
 
+// What a solve has to know of its arrays before it starts, from one pass over
+// them and one host wait (gather_facts).
+struct SolveFacts {
+  double h1min, h1max, h2min, h2max;  // NaNs ignored
+  double fmax;     // max |f|
+  double fmasked;  // max |f| where the mask is 0
+  double skmin;    // min mask
+  double inner;    // max |mask - 1|, |mult - 1| over element-interior nodes
+  double groups;   // 0: every id group has one 0/1 mask value and mult summing to 1
+  double mgdiff;   // nonzero: mask and the other mask differ somewhere
+  double nocode;   // nonzero: some mult is not 1/count for a count in 1..255
+  double rr, bcneu1, bcneu2;  // chktcg1: sum binv f f mult, mask mult, mult
+  const double *h1 = nullptr, *h2 = nullptr;
+  bool interior_zero = false;
+  // a coefficient that is constant enters as that value (the multiply by it
+  // is bit-identical to the multiply by the field)
+  Coef c1() const { return h1min == h1max ? Coef{nullptr, h1min} : Coef{h1, 0.0}; }
+  Coef c2() const { return h2min == h2max ? Coef{nullptr, h2min} : Coef{h2, 0.0}; }
+  // The conditions under which a CG denominator (mask * QQ^T w, p)_mult may
+  // be taken as sum_l p_l w_l before the assembly: ids zero exactly at
+  // element interiors, mask 1 and mult 1 there, and per group a 0/1 mask and
+  // mult summing to 1 (for f itself: zero where masked).
+  bool fused() const { return interior_zero && inner == 0.0 && groups == 0.0; }
+};
+// What gather_facts is asked for besides: mask f in place, the sums of
+// chktcg1, compare the mask with another, code mult as count bytes.
+struct FactsAsk {
+  bool mask_f = false, chk = false;
+  const double *other_mask = nullptr;
+  uint8_t *code = nullptr;
+};
+
 int launch_axhelm(const Mesh &m, double *au, const double *u, Coef h1, Coef h2,
                   hipStream_t s);
 // Kernel choice per order (0: element staged in LDS, 1: t-planes staged) and
@@ -284,30 +316,36 @@ int gs_fin(const GsMap &gs, double *z, const double *e, const uint8_t *w, const 
            hipStream_t s);
 int gs_fin(const GsMap &gs, float *z, const float *e, const uint8_t *w, const double *lut,
            hipStream_t s);
-// Flags per group from mask/mult; *ok when every group has a 0/1 mask equal
-// at all members and mult summing to 1 (red: kRedBlocks scratch).
-int gs_prepare(GsMap &gs, const double *mask, const double *mult, double *red, bool *ok,
-               hipStream_t s);
+// Flags per group from mask/mult (0 sum, 1 masked, 2 single); *bad is set to
+// nonzero unless every group has a 0/1 mask equal at all members and mult
+// summing to 1 (never cleared here).
+int gs_prepare(const GsMap &gs, const double *mask, const double *mult, uint8_t *flag,
+               double *bad, hipStream_t s);
 
 // ---- cg.hip ----
-int run_cggo(Mesh &m, double *x, const double *f, Coef h1, Coef h2, const double *mask,
+int run_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts, const double *mask,
              const double *mult, double tin, int maxit, const nkh_params &prm,
              nkh_result *res, double *history_host);
 // batched Jacobi-PCG solves (graph-captured iteration), see nkd_hmholtz_batch
 int batch_create(int nb, const int *meshes, int *id);
 int batch_destroy(int id);
 int batch_meshes(int id, std::vector<int> *meshes);
-int run_cggo_batch(int id, const double *const *x, const double *const *f, const Coef *h1,
-                   const Coef *h2, const double *const *mask, const double *const *mult,
-                   const double *tin, int maxit, const nkh_params &prm, nkh_result *res,
-                   int *launches_out);
-int run_chktcg1(Mesh &m, double *tol, const double *res, Coef h1, Coef h2,
-                const double *mask, const double *mult);
-int classify_coefs(Mesh &m, const double *h1, const double *h2, Coef *c1, Coef *c2,
-                   hipStream_t s);
+// gather_facts for every solve of a batch (right-hand sides masked in place),
+// one host wait; the group flags of solve k stay in the batch
+int batch_facts(int id, const nkh_batch_solve *solves, bool chk, SolveFacts *out,
+                hipStream_t s);
+int run_cggo_batch(int id, const double *const *x, const double *const *f,
+                   const SolveFacts *facts, const double *const *mask,
+                   const double *const *mult, const double *tin, int maxit,
+                   const nkh_params &prm, nkh_result *res, int *launches_out);
+// One pass over the arrays of a solve (f and other_mask may be null) and one
+// host wait; leaves the group flags of the mask in m.gs.flag.
+int gather_facts(Mesh &m, const double *h1, const double *h2, const double *mask,
+                 const double *mult, double *f, const FactsAsk &ask, SolveFacts *out,
+                 hipStream_t s);
+// hmholtz.f:527-609 CHKTCG1 from the sums in facts (asked for with chk)
+int run_chktcg1(Mesh &m, double *tol, const SolveFacts &facts);
 int run_setprec(Mesh &m, double *d, Coef h1, Coef h2, hipStream_t s);
-int fused_conditions(Mesh &m, const double *mask, const double *mult, const double *f, bool *ok,
-                     hipStream_t s);
 int mul_inplace(double *a, const double *b, int64_t n, hipStream_t s);
 
 // ---- hsmg.hip ----
@@ -336,8 +374,12 @@ int axhelm32_set_variant(int np, int v);
 int axhelm32_variant(int np, int *v);
 int mg_mask_fine(Mesh &m, double *r, hipStream_t s);
 int mg_info(const Mesh &m, int *lmax, int *nh, int *ncrs, double *crs_avg_iters);
-int run_flex_cg(Mesh &m, double *res, Coef h1, Coef h2, const double *wt, const double *mask,
-                int maxit, const nkh_params &prm, nkh_result *out, double *rnorm_history);
+// what the pressure solvers ask of their arrays: the mask against the
+// hierarchy's fine mask, the multiplicity weights as count bytes, chktcg1
+int mg_facts_ask(Mesh &m, FactsAsk *ask);
+int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
+                const double *mask, int maxit, const nkh_params &prm, nkh_result *out,
+                double *rnorm_history);
 // ---- mesh_io.cpp ----
 int re2_header(const char *path, int *nelgt, int *ndim, int *nelgv, int *nfields);
 int re2_read(const char *path, int nelgt, int ndim, int nfields, int *group, double *xc,
@@ -363,11 +405,11 @@ int proj_project2(int id, double *x, const double *h1, const double *h2, const d
 // ---- mixed.hip ----
 // hmh_flex_cg to the same FP64 tolerance by defect correction: FP64 true
 // residuals around inner flexible-CG solves in single precision.
-int run_flex_cg_mixed(Mesh &m, double *res, Coef h1, Coef h2, const double *wt,
+int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
                       const double *mask, int maxit, const nkh_params &prm, nkh_result *out,
                       double *rnorm_history);
 // ---- gmres.hip ----
-int run_gmres(Mesh &m, double *res, Coef h1, Coef h2, const double *wt, const double *mask,
+int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt, const double *mask,
               int maxit, const nkh_params &prm, nkh_result *out, double *rnorm_history);
 
 }  // namespace nekamd

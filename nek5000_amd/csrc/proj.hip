@@ -414,9 +414,8 @@ int proj_project1(int id, double *b, const double *h1, const double *h2, const d
     }
   }
   if (ireset_out) *ireset_out = ireset;
-  Coef c1, c2;
   if (ireset) {
-    NK_TRY(classify_coefs(m, h1, h2, &c1, &c2, s));
+    const Coef c1{h1, 0.0}, c2{h2, 0.0};
     for (int j = 0; j < P->m; ++j) NK_TRY(proj_matvec(m, P->B(j), P->X(j), c1, c2, msk, s));
     NK_TRY(ortho_full_cgs2(*P, w, s));
   }
@@ -461,9 +460,7 @@ int proj_project2(int id, double *x, const double *h1, const double *h2, const d
   hipLaunchKernelGGL(k_pj_addcopy, dim3(pj_grid(P->n)), dim3(256), 0, s, x, P->xbar, add,
                      P->X(P->m - 1), P->n);
   NK_HIP(hipGetLastError());
-  Coef c1, c2;
-  NK_TRY(classify_coefs(m, h1, h2, &c1, &c2, s));
-  NK_TRY(proj_matvec(m, P->B(P->m - 1), P->X(P->m - 1), c1, c2, msk, s));
+  NK_TRY(proj_matvec(m, P->B(P->m - 1), P->X(P->m - 1), Coef{h1, 0.0}, Coef{h2, 0.0}, msk, s));
   return ortho_new(*P, w, s);
 }
 
