@@ -11,7 +11,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libnekamd.so")
 OBJ = os.path.join(HERE, "_objs")
-SOURCES = ["capi.cpp", "kernels.hip", "axhelm.hip", "axhelm_cg.hip", "axhelm_gated.hip", "gs.hip", "cg.hip", "hsmg.hip",
+# (the axhelm instantiations take longest and are compiled first)
+SOURCES = ["axhelm_cg.hip", "axhelm_flex.hip", "axhelm.hip", "axhelm_gated.hip", "hsmg.hip",
+           "capi.cpp", "kernels.hip", "gs.hip", "cg.hip",
            "hsmg_setup.hip", "coarse.hip", "coarse_direct.hip",
            "gmres.hip", "proj.hip", "adjoint.hip", "mesh_io.cpp", "mixed.hip"]
 

@@ -134,7 +134,8 @@ int launch_axhelm(const Mesh &m, double *au, const double *u, Coef h1, Coef h2,
 // the choice reported for an order: that of constant coefficients, or of
 // fields where only those were tuned
 static const AxhelmChoice &reported(int np) {
-  return g_axhelm_choice[!g_axhelm_choice[0][np].tuned && g_axhelm_choice[1][np].tuned ? 1 : 0][np];
+  const bool fields = !g_axhelm_choice[0][np].tuned && g_axhelm_choice[1][np].tuned;
+  return g_axhelm_choice[fields ? 1 : 0][np];
 }
 
 int axhelm_tuning(int np, int *variant, int *grid, int *tuned) {
@@ -149,7 +150,7 @@ int axhelm_tuning(int np, int *variant, int *grid, int *tuned) {
 int axhelm_set_tuning(int np, int variant, int grid) {
   NK_CHECK(np >= 2 && np <= kMaxNP && variant >= 0 && variant <= 5 && grid >= 0,
            NKH_ERR_ARG, "axhelm tuning: lx1=%d variant=%d grid=%d", np, variant, grid);
-  for (auto &kind : g_axhelm_choice)
+  for (AxhelmChoices &kind : g_axhelm_choice)
     kind[np] = AxhelmChoice{variant, grid, variant, variant, true};
   return NKH_OK;
 }

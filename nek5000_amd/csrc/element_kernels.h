@@ -54,19 +54,30 @@ constexpr bool has_wide_elem() {
   return has_wide<NP>() && 3 * NP * NP * NP * 8 * epb_wide<NP>() <= 96 * 1024;
 }
 
-// Sum over the block's threads through LDS (blockDim need not fill whole
-// wavefronts), in a fixed tree order -> deterministic.  sbuf holds blockDim
-// doubles.  Result valid on thread 0.
+// Sum over the block's threads (blockDim need not fill whole wavefronts), in
+// a fixed tree order (neighbours first) -> deterministic: in registers within
+// a wavefront, then over the wavefronts' sums.  sbuf holds at least one
+// double per wavefront.  Result valid on thread 0.
 __device__ __forceinline__ double block_sum(double v, double *sbuf) {
-  const int t = threadIdx.x, nt = blockDim.x;
-  __syncthreads();
-  sbuf[t] = v;
-  __syncthreads();
-  for (int h = 1; h < nt; h <<= 1) {
-    if ((t % (2 * h)) == 0 && t + h < nt) sbuf[t] += sbuf[t + h];
-    __syncthreads();
+  const int t = threadIdx.x, lane = t & 63, nt = blockDim.x, nw = (nt + 63) / 64;
+  const int lanes = nt - (t - lane) < 64 ? nt - (t - lane) : 64;  // of this wavefront
+  for (int o = 1; o < 64; o <<= 1) {
+    const double u = __shfl_down(v, o, 64);
+    if ((lane & (2 * o - 1)) == 0 && lane + o < lanes) v += u;
   }
+  __syncthreads();  // sbuf may hold what other threads still read
+  if (lane == 0) sbuf[t >> 6] = v;
+  __syncthreads();
+  if (t == 0)
+    for (int h = 1; h < nw; h <<= 1)
+      for (int w = 0; w + h < nw; w += 2 * h) sbuf[w] += sbuf[w + h];
   return sbuf[0];
+}
+
+// Wavefronts per SIMD to hold a kernel's registers down to: two, where its
+// LDS lets that many be resident.
+constexpr int min_waves(int lds, int threads) {
+  return 160 * 1024 / lds * ((threads + 63) / 64) / 4 >= 2 ? 2 : 1;
 }
 
 // Streaming accesses of the element kernels: every field word is read or
@@ -92,8 +103,90 @@ __device__ __forceinline__ void stnt(double v, double *p) { __builtin_nontempora
 // kernel need not read p and x again.  MODE 3: MODE 0 gated by a state (returns while st->done),
 // for applies that a captured iteration runs only on some passes.
 // ---------------------------------------------------------------------------
+
+// One thread's t-column of the operand (node base + k NP^2, k = 0..NP-1):
+// u itself (MODE 0, 3), p = beta p + d r (MODE 1; without p in iteration 1) or
+// p = beta p + z with x += alpha p (MODE 2), stored where `store`.  Every load
+// is issued, unconditionally, before the first value is used: with each
+// load in a branch of its own the compiler waited for it there (NP = 8, MODE
+// 1, with the other loads of the kernels likewise: 327 -> 270 us on 32,768
+// elements, 49 -> 39 us on 3,360).
+template <int NP, int MODE>
+__device__ __forceinline__ void column_in(double (&v)[NP], int64_t base, bool store,
+                                          const double *__restrict__ uin,
+                                          const double *__restrict__ r,
+                                          const double *__restrict__ dinv, double *pout,
+                                          double *xacc, double beta, double alpha, bool first) {
+  constexpr int NP2 = NP * NP;
+  double a[NP], b[NP], c[NP];
+  if constexpr (MODE == 1) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) a[k] = 0.0;
+    if (!first) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) a[k] = ldnt(uin + base + k * NP2);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) a[k] = ldnt(uin + base + k * NP2);
+  }
+  if constexpr (MODE == 1 || MODE == 2) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) b[k] = ldnt(r + base + k * NP2);
+  }
+  if constexpr (MODE == 1) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) c[k] = ldnt(dinv + base + k * NP2);
+  }
+  if constexpr (MODE == 2) {
+    if (xacc) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) c[k] = ldnt(xacc + base + k * NP2);
+      if (store) {
+#pragma unroll
+        for (int k = 0; k < NP; ++k) stnt(c[k] + alpha * a[k], xacc + base + k * NP2);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    if constexpr (MODE == 1) v[k] = beta * a[k] + c[k] * b[k];  // add2s1, z = r*d
+    else if constexpr (MODE == 2) v[k] = beta * a[k] + b[k];
+    else v[k] = a[k];
+  }
+  if constexpr (MODE == 1 || MODE == 2) {
+    if (store) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) stnt(v[k], pout + base + k * NP2);
+    }
+  }
+}
+
+// the mass term's factor h2*bm1 of a column's nodes (loaded ahead of its use)
+template <int NP, int H2M>
+__device__ __forceinline__ void column_mass(double (&m)[NP], int64_t base,
+                                            const double *__restrict__ h2f, double h2s,
+                                            const double *__restrict__ bm1) {
+  constexpr int NP2 = NP * NP;
+  if constexpr (H2M == 1) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) m[k] = h2s * ldnt(bm1 + base + k * NP2);
+  }
+  if constexpr (H2M == 2) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k)
+      m[k] = ldnt(h2f + base + k * NP2) * ldnt(bm1 + base + k * NP2);
+  }
+}
+
+// Bound by its streams (12 words per node in MODE 1).  Two wavefronts per SIMD
+// at least: left alone, the compiler hoists every factor load and takes up
+// to 256 registers at NP >= 9 (NP = 12, 1.67e7 nodes, plain: 640 us against
+// 427).  MODE 1 at 1.67e7 nodes, us before -> now: NP = 6 412 -> 300, NP = 8
+// 326 -> 269 (6.0 TB/s).
 template <int NP, int MODE, bool H1F, int H2M, int EPB_ = epb<NP>()>
-__global__ void __launch_bounds__(NP * NP * EPB_)
+__global__ void __launch_bounds__(NP * NP * EPB_,
+                                  min_waves((24 * NP + 16) * (NP + 1) * NP * EPB_, NP * NP * EPB_))
     k_axhelm(DMat<NP> Dm, const double *__restrict__ Dg, double *__restrict__ au,
              const double *__restrict__ uin, const double *__restrict__ g, int64_t gstride,
              const double *__restrict__ h1f, double h1s, const double *__restrict__ h2f,
@@ -133,31 +226,15 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
 
   double rho = 0.0;
   for (int64_t eb = blockIdx.x; eb * EPB < nel; eb += gridDim.x) {
-    const int64_t e = eb * EPB + le;
-    const bool valid = (le < EPB) && (e < nel);
-    const int64_t base = e * NP3 + ij;
-    double r_u[NP], r_au[NP];
+    // a slab past the last element works on the block's first one, unstored
+    const bool valid = EPB == 1 || eb * EPB + le < nel;
+    const int64_t base = (eb * EPB + (valid ? le : 0)) * NP3 + ij;
+    double r_u[NP], r_au[NP], r_m[NP];
+    column_in<NP, MODE>(r_u, base, valid, uin, r, dinv, pout, xacc, beta, alpha, first);
     __syncthreads();  // LDS reuse across element groups (and s_D fill)
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      double v = 0.0;
-      if (valid) {
-        const int64_t l = base + k * NP2;
-        if constexpr (MODE == 1) {
-          // add2s1: p = beta*p + z, z = r*d
-          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
-          stnt(v, pout + l);
-        } else if constexpr (MODE == 2) {
-          const double po = ldnt(uin + l);
-          v = beta * po + ldnt(r + l);
-          if (xacc) stnt(ldnt(xacc + l) + alpha * po, xacc + l);
-          stnt(v, pout + l);
-        } else {
-          v = ldnt(uin + l);
-        }
-      }
-      r_u[k] = v;
-      s_u[le][k * NP2 + ij] = v;
+      s_u[le][k * NP2 + ij] = r_u[k];
       r_au[k] = 0.0;
     }
     __syncthreads();
@@ -170,32 +247,28 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
         us += s_D[j][m] * s_u[le][k * NP2 + m * NP + i];
         ut += Dm.d[k + NP * m] * r_u[m];
       }
-      double wr = 0.0, ws = 0.0, wt = 0.0;
-      if (valid) {
-        const int64_t l = base + k * NP2;
-        const double G1 = ldnt(g + l), G2 = ldnt(g + gstride + l),
-                     G3 = ldnt(g + 2 * gstride + l);
-        const double G4 = ldnt(g + 3 * gstride + l), G5 = ldnt(g + 4 * gstride + l),
-                     G6 = ldnt(g + 5 * gstride + l);
-        wr = ur * G1;
-        ws = us * G2;
-        wt = ut * G3;
-        wr = wr + us * G4;
-        wr = wr + ut * G5;
-        ws = ws + ur * G4;
-        ws = ws + ut * G6;
-        wt = wt + ur * G5;
-        wt = wt + us * G6;
-        const double h1 = H1F ? ldnt(h1f + l) : h1s;
-        wr *= h1;
-        ws *= h1;
-        wt *= h1;
-      }
+      const int64_t l = base + k * NP2;
+      const double G1 = ldnt(g + l), G2 = ldnt(g + gstride + l),
+                   G3 = ldnt(g + 2 * gstride + l);
+      const double G4 = ldnt(g + 3 * gstride + l), G5 = ldnt(g + 4 * gstride + l),
+                   G6 = ldnt(g + 5 * gstride + l);
+      double wr = ur * G1, ws = us * G2, wt = ut * G3;
+      wr = wr + us * G4;
+      wr = wr + ut * G5;
+      ws = ws + ur * G4;
+      ws = ws + ut * G6;
+      wt = wt + ur * G5;
+      wt = wt + us * G6;
+      const double h1 = H1F ? ldnt(h1f + l) : h1s;
+      wr *= h1;
+      ws *= h1;
+      wt *= h1;
       s_wr[le][k * NP2 + ij] = wr;
       s_ws[le][k * NP2 + ij] = ws;
 #pragma unroll
       for (int kk = 0; kk < NP; ++kk) r_au[kk] += Dm.d[k + NP * kk] * wt;
     }
+    column_mass<NP, H2M>(r_m, base, h2f, h2s, bm1);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
@@ -205,12 +278,10 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
         ar += s_D[m][i] * s_wr[le][k * NP2 + j * NP + m];
         as += s_D[m][j] * s_ws[le][k * NP2 + m * NP + i];
       }
+      double a = ar + as + r_au[k];
+      if constexpr (H2M != 0) a = a + r_m[k] * r_u[k];
       if (valid) {
-        const int64_t l = base + k * NP2;
-        double a = ar + as + r_au[k];
-        if constexpr (H2M == 1) a = a + (h2s * ldnt(bm1 + l)) * r_u[k];
-        if constexpr (H2M == 2) a = a + (ldnt(h2f + l) * ldnt(bm1 + l)) * r_u[k];
-        stnt(a, au + l);
+        stnt(a, au + base + k * NP2);
         if constexpr (MODE == 1 || MODE == 2) rho += a * r_u[k];  // p . (A_L p), element-local
       }
     }
@@ -267,30 +338,12 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
   for (int t = tid; t < NP2; t += blockDim.x) s_D[t % NP][t / NP] = Dg[t];
   double rho = 0.0;
   for (int64_t eb = blockIdx.x; eb * EPB < nel; eb += gridDim.x) {
-    const int64_t e = eb * EPB + le;
-    const bool valid = (le < EPB) && (e < nel);
-    const int64_t base = e * (int64_t)(NP2 * NP) + ij;
-    double r_u[NP], r_au[NP], r_o[NP];
+    const bool valid = EPB == 1 || eb * EPB + le < nel;
+    const int64_t base = (eb * EPB + (valid ? le : 0)) * (int64_t)(NP2 * NP) + ij;
+    double r_u[NP], r_au[NP], r_o[NP], r_m[NP];
+    column_in<NP, MODE>(r_u, base, valid, uin, r, dinv, pout, xacc, beta, alpha, first);
 #pragma unroll
-    for (int k = 0; k < NP; ++k) {
-      double v = 0.0;
-      if (valid) {
-        const int64_t l = base + k * NP2;
-        if constexpr (MODE == 1) {
-          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
-          stnt(v, pout + l);
-        } else if constexpr (MODE == 2) {
-          const double po = ldnt(uin + l);
-          v = beta * po + ldnt(r + l);
-          if (xacc) stnt(ldnt(xacc + l) + alpha * po, xacc + l);
-          stnt(v, pout + l);
-        } else {
-          v = ldnt(uin + l);
-        }
-      }
-      r_u[k] = v;
-      r_au[k] = 0.0;
-    }
+    for (int k = 0; k < NP; ++k) r_au[k] = 0.0;
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       // one plane at a time: keeps the scheduler from hoisting the next
@@ -306,27 +359,22 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
         us += s_D[j][m] * s_u[le][m * NP + i];
         ut += Dm.d[k + NP * m] * r_u[m];
       }
-      double wr = 0.0, ws = 0.0, wt = 0.0;
-      if (valid) {
-        const int64_t l = base + k * NP2;
-        const double G1 = ldnt(g + l), G2 = ldnt(g + gstride + l),
-                     G3 = ldnt(g + 2 * gstride + l);
-        const double G4 = ldnt(g + 3 * gstride + l), G5 = ldnt(g + 4 * gstride + l),
-                     G6 = ldnt(g + 5 * gstride + l);
-        wr = ur * G1;
-        ws = us * G2;
-        wt = ut * G3;
-        wr = wr + us * G4;
-        wr = wr + ut * G5;
-        ws = ws + ur * G4;
-        ws = ws + ut * G6;
-        wt = wt + ur * G5;
-        wt = wt + us * G6;
-        const double h1 = H1F ? ldnt(h1f + l) : h1s;
-        wr *= h1;
-        ws *= h1;
-        wt *= h1;
-      }
+      const int64_t l = base + k * NP2;
+      const double G1 = ldnt(g + l), G2 = ldnt(g + gstride + l),
+                   G3 = ldnt(g + 2 * gstride + l);
+      const double G4 = ldnt(g + 3 * gstride + l), G5 = ldnt(g + 4 * gstride + l),
+                   G6 = ldnt(g + 5 * gstride + l);
+      double wr = ur * G1, ws = us * G2, wt = ut * G3;
+      wr = wr + us * G4;
+      wr = wr + ut * G5;
+      ws = ws + ur * G4;
+      ws = ws + ut * G6;
+      wt = wt + ur * G5;
+      wt = wt + us * G6;
+      const double h1 = H1F ? ldnt(h1f + l) : h1s;
+      wr *= h1;
+      ws *= h1;
+      wt *= h1;
       s_wr[le][ij] = wr;
       s_ws[le][ij] = ws;
 #pragma unroll
@@ -346,15 +394,15 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
 #pragma unroll
       for (int kk = 0; kk < NP; ++kk) asm volatile("" : "+v"(r_au[kk]));
     }
+    column_mass<NP, H2M>(r_m, base, h2f, h2s, bm1);
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      const int64_t l = base + k * NP2;
       double a = r_o[k] + r_au[k];
-      if constexpr (H2M == 1) a = a + (h2s * (valid ? ldnt(bm1 + l) : 0.0)) * r_u[k];
-      if constexpr (H2M == 2)
-        a = a + ((valid ? ldnt(h2f + l) : 0.0) * (valid ? ldnt(bm1 + l) : 0.0)) * r_u[k];
-      if (valid) stnt(a, au + l);
-      if constexpr (MODE == 1 || MODE == 2) rho += a * r_u[k];  // a = r_u = 0 off the mesh
+      if constexpr (H2M != 0) a = a + r_m[k] * r_u[k];
+      if (valid) {
+        stnt(a, au + base + k * NP2);
+        if constexpr (MODE == 1 || MODE == 2) rho += a * r_u[k];
+      }
     }
   }
   if constexpr (MODE == 1 || MODE == 2) {
@@ -395,7 +443,8 @@ constexpr int mx_threads() {
 }
 
 template <int NP, int MODE, bool H1F, int H2M>
-__global__ void __launch_bounds__(mx_threads<NP>())
+__global__ void __launch_bounds__(mx_threads<NP>(),
+                                  min_waves(24 * (NP | 1) * NP * NP, mx_threads<NP>()))
     k_axhelm_mx(DMat<NP> Dm, const double *__restrict__ Dg, double *__restrict__ au,
                 const double *__restrict__ uin, const double *__restrict__ g, int64_t gstride,
                 const double *__restrict__ h1f, double h1s, const double *__restrict__ h2f,
@@ -443,28 +492,14 @@ __global__ void __launch_bounds__(mx_threads<NP>())
   const int own_at = i + PJ * j;  // the owner's node in a plane of LDS
   double rho = 0.0;
   for (int64_t e = blockIdx.x; e < nel; e += gridDim.x) {
-    const int64_t base = e * NP3 + tid;
-    double r_u[NP], r_au[NP];
+    // threads without a column load the last one's, unstored
+    const int64_t base = e * NP3 + (own ? tid : NP2 - 1);
+    double r_u[NP], r_au[NP], r_m[NP];
+    column_in<NP, MODE>(r_u, base, own, uin, r, dinv, pout, xacc, beta, alpha, first);
     __syncthreads();  // the previous element's LDS reads are done
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      double v = 0.0;
-      if (own) {
-        const int64_t l = base + k * NP2;
-        if constexpr (MODE == 1) {
-          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
-          stnt(v, pout + l);
-        } else if constexpr (MODE == 2) {
-          const double po = ldnt(uin + l);
-          v = beta * po + ldnt(r + l);
-          if (xacc) stnt(ldnt(xacc + l) + alpha * po, xacc + l);
-          stnt(v, pout + l);
-        } else {
-          v = ldnt(uin + l);
-        }
-        s_u[k * PK + own_at] = v;
-      }
-      r_u[k] = v;
+      if (own) s_u[k * PK + own_at] = r_u[k];
       r_au[k] = 0.0;
     }
     __syncthreads();
@@ -551,14 +586,14 @@ __global__ void __launch_bounds__(mx_threads<NP>())
         if (lin && jj < NP) s_u[k * PK + PJ * jj + lr] = acc[v];
       }
     }
+    column_mass<NP, H2M>(r_m, base, h2f, h2s, bm1);
     __syncthreads();
     if (own) {
 #pragma unroll
       for (int k = 0; k < NP; ++k) {
         const int64_t l = base + k * NP2;
         double a = s_u[k * PK + own_at] + r_au[k];
-        if constexpr (H2M == 1) a = a + (h2s * ldnt(bm1 + l)) * r_u[k];
-        if constexpr (H2M == 2) a = a + (ldnt(h2f + l) * ldnt(bm1 + l)) * r_u[k];
+        if constexpr (H2M != 0) a = a + r_m[k] * r_u[k];
         stnt(a, au + l);
         if constexpr (MODE == 1 || MODE == 2) rho += a * r_u[k];
       }
@@ -580,9 +615,11 @@ __global__ void __launch_bounds__(mx_threads<NP>())
 // k_axhelm_pl), each wavefront forms ar + as of its plane, and the owners
 // keep those in registers until the t-direction sums are complete.  The
 // products, their layouts and the arithmetic order are those of
-// k_axhelm_mx, so the two give the same au bit for bit.
+// k_axhelm_mx, so the two give the same au bit for bit.  Register bound as
+// k_axhelm: MODE 1 at 1.67e7 nodes, us before -> now: NP = 10 503 -> 294 (the
+// fastest kernel before: 389), NP = 12 663 -> 341 (510; 4.7 TB/s).
 template <int NP, int MODE, bool H1F, int H2M>
-__global__ void __launch_bounds__(mx_threads<NP>())
+__global__ void __launch_bounds__(mx_threads<NP>(), 2)
     k_axhelm_mxp(DMat<NP> Dm, const double *__restrict__ Dg, double *__restrict__ au,
                  const double *__restrict__ uin, const double *__restrict__ g, int64_t gstride,
                  const double *__restrict__ h1f, double h1s, const double *__restrict__ h2f,
@@ -630,26 +667,11 @@ __global__ void __launch_bounds__(mx_threads<NP>())
   double *const wu = s_u + wv * PP, *const wwr = s_wr + wv * PP, *const wws = s_ws + wv * PP;
   double rho = 0.0;
   for (int64_t e = blockIdx.x; e < nel; e += gridDim.x) {
-    const int64_t base = e * NP3 + tid;
-    double r_u[NP], r_au[NP], r_o[NP];
+    const int64_t base = e * NP3 + (own ? tid : NP2 - 1);
+    double r_u[NP], r_au[NP], r_o[NP], r_m[NP];
+    column_in<NP, MODE>(r_u, base, own, uin, r, dinv, pout, xacc, beta, alpha, first);
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      double v = 0.0;
-      if (own) {
-        const int64_t l = base + k * NP2;
-        if constexpr (MODE == 1) {
-          v = (first ? 0.0 : beta * ldnt(uin + l)) + ldnt(dinv + l) * ldnt(r + l);
-          stnt(v, pout + l);
-        } else if constexpr (MODE == 2) {
-          const double po = ldnt(uin + l);
-          v = beta * po + ldnt(r + l);
-          if (xacc) stnt(ldnt(xacc + l) + alpha * po, xacc + l);
-          stnt(v, pout + l);
-        } else {
-          v = ldnt(uin + l);
-        }
-      }
-      r_u[k] = v;
       r_au[k] = 0.0;
       r_o[k] = 0.0;
     }
@@ -752,13 +774,13 @@ __global__ void __launch_bounds__(mx_threads<NP>())
           if (gq * G + q < NP) r_o[gq * G + q] = s_u[q * PP + own_at];
       }
     }
+    column_mass<NP, H2M>(r_m, base, h2f, h2s, bm1);
     if (own) {
 #pragma unroll
       for (int k = 0; k < NP; ++k) {
         const int64_t l = base + k * NP2;
         double a = r_o[k] + r_au[k];
-        if constexpr (H2M == 1) a = a + (h2s * ldnt(bm1 + l)) * r_u[k];
-        if constexpr (H2M == 2) a = a + (ldnt(h2f + l) * ldnt(bm1 + l)) * r_u[k];
+        if constexpr (H2M != 0) a = a + r_m[k] * r_u[k];
         stnt(a, au + l);
         if constexpr (MODE == 1 || MODE == 2) rho += a * r_u[k];
       }
@@ -783,9 +805,25 @@ struct AxhelmChoice {
   int variant_flex = 0;  // MODE 2
   bool tuned = false;
 };
+// Untuned (meshes of less than 2^20 nodes): per order the kernel that is the
+// fastest or near it at 6e4 to 9e5 nodes -- element-staged up to NP = 8, the
+// matrix cores beyond, staging the element (4) or groups of planes (5).  us
+// at 2.5e5 nodes, element-staged / matrix cores, CG-fused apply: NP = 8 13 /
+// 18 (4), 10 26 / 22 (5), 12 37 / 29 (5), 14 53 / 39 (4), 16 67 / 49 (5).
+constexpr AxhelmChoice axhelm_default(int np) {
+  const int v = np < 9 ? 0 : (np == 11 || (np >= 13 && np <= 15) ? 4 : 5);
+  return AxhelmChoice{v, 0, v, v, false};
+}
+struct AxhelmChoices {
+  AxhelmChoice c[kMaxNP + 1];
+  constexpr AxhelmChoices() : c() {
+    for (int np = 0; np <= kMaxNP; ++np) c[np] = axhelm_default(np);
+  }
+  AxhelmChoice &operator[](int np) { return c[np]; }
+};
 // by kind of coefficients (0: h1 and h2 both constant, 1: a field among them,
 // which adds one or two streams) and order
-inline AxhelmChoice g_axhelm_choice[2][kMaxNP + 1];
+inline AxhelmChoices g_axhelm_choice[2];
 inline int axhelm_kind(Coef h1, Coef h2) { return h1.uniform() && h2.uniform() ? 0 : 1; }
 
 // One launch of the axhelm kernel (element- or plane-staged, EPB slabs per
@@ -834,7 +872,11 @@ static int axhelm_go(const Mesh &m, const DMat<NP> &Dm, double *au, const double
     hipLaunchKernelGGL((k_axhelm<NP, MODE, H1F_, H2M_, EPB>), dim3(grid), block, 0, s, Dm,    \
                        m.Dd, au, u, m.g, m.n, h1.f, h1.s, h2.f, h2.s, m.bm1, m.nel, pout, r,   \
                        dinv, mult, st, rho_part, betap, xacc, alphap)
-  if (h1f) {
+  if constexpr (MODE == 3) {  // the mixed solver's: constant coefficients
+    NK_CHECK(!h1f && h2m != 2, NKH_ERR_ARG, "gated axhelm: constant h1 and h2 only");
+    if (h2m == 0) NK_LAUNCH(false, 0);
+    else NK_LAUNCH(false, 1);
+  } else if (h1f) {
     if (h2m == 0) NK_LAUNCH(true, 0);
     else if (h2m == 1) NK_LAUNCH(true, 1);
     else NK_LAUNCH(true, 2);
