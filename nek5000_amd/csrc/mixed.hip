@@ -223,8 +223,42 @@ __global__ void __launch_bounds__(256)
 // slab as the FP64 kernel.
 __device__ __forceinline__ float ldnt32(const float *q) { return __builtin_nontemporal_load(q); }
 
+// One thread's t-column of p, every load issued before the first value is
+// used, stored where `store` (column_in of the FP64 kernels; JAC at 9e6
+// nodes, us before -> now, the faster kernel of each order: lx1 = 6 138 -> 92,
+// 8 94 -> 76 (5.7 TB/s), 9 140 -> 97, 10 124 -> 105, 12 133 -> 122, 14 190 ->
+// 155).
+template <int NP, bool JAC>
+__device__ __forceinline__ void column_in32(float (&v)[NP], int64_t base, bool store, float *p,
+                                            const float *__restrict__ z,
+                                            const float *__restrict__ dd, float beta) {
+  constexpr int NP2 = NP * NP;
+  float a[NP], b[NP], c[NP];
+#pragma unroll
+  for (int k = 0; k < NP; ++k) a[k] = 0.0f;
+  if (!JAC || beta != 0.0f) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) a[k] = ldnt32(p + base + k * NP2);
+  }
+#pragma unroll
+  for (int k = 0; k < NP; ++k) b[k] = ldnt32(z + base + k * NP2);
+  if constexpr (JAC) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) c[k] = ldnt32(dd + base + k * NP2);
+  }
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    if constexpr (JAC) v[k] = c[k] * b[k] + beta * a[k];
+    else v[k] = beta * a[k] + b[k];
+  }
+  if (store) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) __builtin_nontemporal_store(v[k], p + base + k * NP2);
+  }
+}
+
 template <int NP, bool H2, bool JAC>
-__global__ void __launch_bounds__(NP * NP * epb<NP>())
+__global__ void __launch_bounds__(NP * NP * epb<NP>(), NP == 9 || NP == 10 ? 3 : 1)
     k_axhelm32(DMatF<NP> Dk, const double *__restrict__ Dg, float *__restrict__ w,
                float *__restrict__ p, const float *__restrict__ z, const float *__restrict__ dd,
                const float *__restrict__ g, int64_t gstride, float h1, float h2,
@@ -247,23 +281,15 @@ __global__ void __launch_bounds__(NP * NP * epb<NP>())
   for (int t = tid; t < NP2; t += blockDim.x) s_D[t % NP][t / NP] = (float)Dg[t];
   double den = 0.0;
   for (int64_t eb = blockIdx.x; eb * EPB < nel; eb += gridDim.x) {
-    const int64_t e = eb * EPB + le;
-    const bool valid = (le < EPB) && (e < nel);
-    const int64_t base = e * NP3 + ij;
-    float r_u[NP], r_au[NP];
+    // a slab past the last element works on the block's first one, unstored
+    const bool valid = EPB == 1 || eb * EPB + le < nel;
+    const int64_t base = (eb * EPB + (valid ? le : 0)) * NP3 + ij;
+    float r_u[NP], r_au[NP], r_m[NP];
+    column_in32<NP, JAC>(r_u, base, valid, p, z, dd, beta);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      float v = 0.0f;
-      if (valid) {
-        const int64_t l = base + k * NP2;
-        if constexpr (JAC)
-          v = ldnt32(dd + l) * ldnt32(z + l) + (beta != 0.0f ? beta * ldnt32(p + l) : 0.0f);
-        else v = beta * ldnt32(p + l) + ldnt32(z + l);
-        __builtin_nontemporal_store(v, p + l);
-      }
-      r_u[k] = v;
-      s_u[le][k * NP2 + ij] = v;
+      s_u[le][k * NP2 + ij] = r_u[k];
       r_au[k] = 0.0f;
     }
     __syncthreads();
@@ -276,21 +302,22 @@ __global__ void __launch_bounds__(NP * NP * epb<NP>())
         us += s_D[j][m] * s_u[le][k * NP2 + m * NP + i];
         ut += Dk.d[k + NP * m] * r_u[m];
       }
-      float wr = 0.0f, ws = 0.0f, wt = 0.0f;
-      if (valid) {
-        const int64_t l = base + k * NP2;
-        const float G1 = ldnt32(g + l), G2 = ldnt32(g + gstride + l),
-                    G3 = ldnt32(g + 2 * gstride + l);
-        const float G4 = ldnt32(g + 3 * gstride + l), G5 = ldnt32(g + 4 * gstride + l),
-                    G6 = ldnt32(g + 5 * gstride + l);
-        wr = h1 * (ur * G1 + us * G4 + ut * G5);
-        ws = h1 * (ur * G4 + us * G2 + ut * G6);
-        wt = h1 * (ur * G5 + us * G6 + ut * G3);
-      }
+      const int64_t l = base + k * NP2;
+      const float G1 = ldnt32(g + l), G2 = ldnt32(g + gstride + l),
+                  G3 = ldnt32(g + 2 * gstride + l);
+      const float G4 = ldnt32(g + 3 * gstride + l), G5 = ldnt32(g + 4 * gstride + l),
+                  G6 = ldnt32(g + 5 * gstride + l);
+      const float wr = h1 * (ur * G1 + us * G4 + ut * G5);
+      const float ws = h1 * (ur * G4 + us * G2 + ut * G6);
+      const float wt = h1 * (ur * G5 + us * G6 + ut * G3);
       s_wr[le][k * NP2 + ij] = wr;
       s_ws[le][k * NP2 + ij] = ws;
 #pragma unroll
       for (int kk = 0; kk < NP; ++kk) r_au[kk] += Dk.d[k + NP * kk] * wt;
+    }
+    if constexpr (H2) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) r_m[k] = h2 * ldnt32(bm1 + base + k * NP2);
     }
     __syncthreads();
 #pragma unroll
@@ -301,11 +328,10 @@ __global__ void __launch_bounds__(NP * NP * epb<NP>())
         ar += s_D[m][i] * s_wr[le][k * NP2 + j * NP + m];
         as += s_D[m][j] * s_ws[le][k * NP2 + m * NP + i];
       }
+      float a = ar + as + r_au[k];
+      if constexpr (H2) a = a + r_m[k] * r_u[k];
       if (valid) {
-        const int64_t l = base + k * NP2;
-        float a = ar + as + r_au[k];
-        if constexpr (H2) a = a + (h2 * ldnt32(bm1 + l)) * r_u[k];
-        __builtin_nontemporal_store(a, w + l);
+        __builtin_nontemporal_store(a, w + base + k * NP2);
         den += (double)a * (double)r_u[k];
       }
     }
@@ -323,11 +349,12 @@ __global__ void __launch_bounds__(NP * NP * epb<NP>())
 // t-direction terms, the factors and the epilogue as in k_axhelm32.  Lane l
 // of a product holds A[l%16][4c + l/16] and B[4c + l/16][l%16] of chunk c and
 // gets D[4(l/16)+v][l%16] in register v (the FP32 layout, checked on
-// gfx950).  Results agree with k_axhelm32 to FP32 rounding.
+// gfx950).  Results agree with k_axhelm32 to FP32 rounding.  Registers held
+// to two wavefronts per SIMD as in k_axhelm_mxp.
 typedef float nk_f4 __attribute__((ext_vector_type(4)));
 
 template <int NP, bool H2, bool JAC>
-__global__ void __launch_bounds__(mx_threads<NP>())
+__global__ void __launch_bounds__(mx_threads<NP>(), 2)
     k_axhelm32_mxp(DMatF<NP> Dk, const double *__restrict__ Dg, float *__restrict__ w,
                    float *__restrict__ p, const float *__restrict__ z,
                    const float *__restrict__ dd, const float *__restrict__ g, int64_t gstride,
@@ -362,19 +389,12 @@ __global__ void __launch_bounds__(mx_threads<NP>())
   float *const wu = s_u + wv * PP, *const wwr = s_wr + wv * PP, *const wws = s_ws + wv * PP;
   double den = 0.0;
   for (int64_t e = blockIdx.x; e < nel; e += gridDim.x) {
-    const int64_t base = e * NP3 + tid;
-    float r_u[NP], r_au[NP], r_o[NP];
+    // threads without a column load the last one's, unstored
+    const int64_t base = e * NP3 + (own ? tid : NP2 - 1);
+    float r_u[NP], r_au[NP], r_o[NP], r_m[NP];
+    column_in32<NP, JAC>(r_u, base, own, p, z, dd, beta);
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      float v = 0.0f;
-      if (own) {
-        const int64_t l = base + k * NP2;
-        if constexpr (JAC)
-          v = ldnt32(dd + l) * ldnt32(z + l) + (beta != 0.0f ? beta * ldnt32(p + l) : 0.0f);
-        else v = beta * ldnt32(p + l) + ldnt32(z + l);
-        __builtin_nontemporal_store(v, p + l);
-      }
-      r_u[k] = v;
       r_au[k] = 0.0f;
       r_o[k] = 0.0f;
     }
@@ -466,12 +486,16 @@ __global__ void __launch_bounds__(mx_threads<NP>())
           if (gq * G + q < NP) r_o[gq * G + q] = s_u[q * PP + own_at];
       }
     }
+    if constexpr (H2) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) r_m[k] = h2 * ldnt32(bm1 + base + k * NP2);
+    }
     if (own) {
 #pragma unroll
       for (int k = 0; k < NP; ++k) {
         const int64_t l = base + k * NP2;
         float a = r_o[k] + r_au[k];
-        if constexpr (H2) a = a + (h2 * ldnt32(bm1 + l)) * r_u[k];
+        if constexpr (H2) a = a + r_m[k] * r_u[k];
         __builtin_nontemporal_store(a, w + l);
         den += (double)a * (double)r_u[k];
       }
@@ -483,13 +507,11 @@ __global__ void __launch_bounds__(mx_threads<NP>())
 
 // Kernel of the FP32 operator per order: 0 vector FMA (k_axhelm32), 1 the
 // matrix cores (k_axhelm32_mxp, lx1 = 8..16); nkh_axhelm32_set_variant fixes
-// it.  Defaults from 100 mixed Jacobi-PCG iterations per kernel on boxes of
-// about 5e7 unique DOF (MI355X, GDOF*iter/s vector -> matrix cores): lx1 = 8
-// 30.9 -> 31.6 (and the mixed flexible CG at E = 64^3 122.9-123.3 -> 122.1-
-// 122.8 ms per solve), 11 30.3 -> 32.0, 14 26.2 -> 27.3, 15 25.4 -> 28.1;
-// the other orders are faster with vector FMA or within 1 % (lx1 = 12:
-// 32.3 -> 29.0).
-int g_ax32_variant[kMaxNP + 1] = {0, 0, 0, 0, 0, 0, 0, 0, 1, 0, 0, 1, 0, 0, 1, 1, 0};
+// it.  Defaults: the faster one at 9e6 nodes, us vector / matrix cores, JAC
+// and flexible CG: lx1 = 8 76 / 79 and 64 / 70, 9 97 / 108 and 85 / 98, 10
+// 135 / 105 and 90 / 93, 12 185 / 123 and 109 / 115, 14 230 / 155 and 214 /
+// 146, 16 197 / 149 and 158 / 123.
+int g_ax32_variant[kMaxNP + 1] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 1};
 
 template <int NP, bool JAC>
 static int axhelm32_dispatch(const Mesh &m, float *w, float *p, const float *z, const float *dd,
