@@ -325,9 +325,8 @@ typedef struct {
 } nkh_batch_solve;
 /* hmholtz.f:2-69 + the Jacobi branch of cggo (:611-846) for every solve of
    the batch (non-PRES names): the set-up of each solve in order, then all
-   solves iterate together -- eight steady-state iterations of the whole
-   batch (each solve's launches on its own stream) are captured once in a
-   hipGraph and replayed until every solve has stopped.  Iterates and
+   solves iterate together, each on its own stream, until every one has
+   stopped.  Iterates and
    results equal those of nkd_hmholtz on each solve (prm->precision 0 or
    2).  res: nb results; *graph_launches (optional): iterations enqueued
    for the slowest solve. */

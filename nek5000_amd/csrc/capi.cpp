@@ -512,6 +512,7 @@ static void mesh_release(Mesh *m) {
                   (void *)m->st, (void *)m->red, (void *)m->g32, (void *)m->bm1_32,
                   (void *)m->undeformed})
     if (p) (void)hipFree(p);
+  if (m->box) (void)hipHostFree(m->box);
   delete m;
 }
 

@@ -16,9 +16,8 @@
 // (mask*QQ^T w, p)_mult = sum_l p_l w_l exactly in exact arithmetic.  The
 // solve checks those conditions once and otherwise runs the unfused
 // sequence (axhelm, dssum, mask, dot).
-// Scalars stay on the device (CgState); the host enqueues iterations ahead
-// and reads the state back every few iterations.  Kernels of iterations past
-// the exit return immediately.
+// Scalars stay on the device (CgState); the kernel of the exit test reports
+// them to the host.  Kernels past the exit return immediately.
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -90,7 +89,7 @@ __global__ void __launch_bounds__(256)
             const double *__restrict__ mask, const double *__restrict__ mult, double *f,
             int mask_f, const double *__restrict__ binv, const double *__restrict__ other,
             uint8_t *__restrict__ code, int64_t n, int np, double *__restrict__ part,
-            double *__restrict__ groups) {
+            double *__restrict__ groups, int *__restrict__ left) {
   __shared__ double sb[4][kNF];
   __shared__ uint8_t s_in[kMaxNP * kMaxNP * kMaxNP];
   const int np3 = np * np * np;
@@ -98,7 +97,10 @@ __global__ void __launch_bounds__(256)
     const int i = q % np, j = (q / np) % np, k = q / (np * np);
     s_in[q] = i > 0 && i < np - 1 && j > 0 && j < np - 1 && k > 0 && k < np - 1;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) *groups = 0.0;  // gs_prepare runs after this
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // for the kernels after this one
+    *groups = 0.0;
+    *left = kNF;
+  }
   __syncthreads();
   double v[kNF];
 #pragma unroll
@@ -155,9 +157,11 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// block q: result q over the count partials
+// block q: result q over the count partials; the last block to end reports
+// the results and the group check to the host (left counts the blocks to go)
 __global__ void __launch_bounds__(256)
-    k_facts_final(const double *__restrict__ part, int count, double *__restrict__ out) {
+    k_facts_final(const double *__restrict__ part, int count, double *__restrict__ out,
+                  int *__restrict__ left, BoxRef rep) {
   __shared__ double sb[4];
   const int q = blockIdx.x, op = fact_op(q);
   double v = fact_start(op);
@@ -170,6 +174,12 @@ __global__ void __launch_bounds__(256)
     double t = sb[0];
     for (int w = 1; w < 4; ++w) t = fact_join(op, t, sb[w]);
     out[q] = t;
+    if (rep.b) {
+      rep.b->v[q] = t;
+      if (q == 0) rep.b->v[kNF] = out[kNF];
+      __threadfence_system();
+      if (atomicSub(left, 1) == 1) box_report(rep);
+    }
   }
 }
 
@@ -217,7 +227,8 @@ __global__ void __launch_bounds__(256)
               double *__restrict__ d, const double *__restrict__ mult,
               const double *__restrict__ binv, double *__restrict__ dm,
               double *__restrict__ bm, int plain_norm, int64_t n, double *__restrict__ part1,
-              double *__restrict__ part2) {
+              double *__restrict__ part2, CgState init, CgState *__restrict__ st) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *st = init;
   double s1 = 0.0, s2 = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -291,13 +302,15 @@ __global__ void __launch_bounds__(256)
   block_store2(s1, s2, part1, part2);
 }
 
-__global__ void __launch_bounds__(kScalThreads)
-    k_cg_scalars1(CgState *__restrict__ st, const double *__restrict__ part1,
-                  const double *__restrict__ part2, int nparts, double *__restrict__ hist) {
-  if (st->done) return;
-  const double s1 = block_sum_array(part1, nparts);
-  const double s2 = block_sum_array(part2, nparts);
-  if (threadIdx.x != 0) return;
+// the state to the host (a solve that is done changes it no more)
+__device__ __forceinline__ void state_report(const CgState *st, const BoxRef &rep) {
+  if (!rep.b) return;
+  *reinterpret_cast<CgState *>(rep.b->v) = *st;
+  box_report(rep);
+}
+static_assert(sizeof(CgState) <= sizeof(HostBox::v), "a report holds a state");
+
+__device__ void cg_scalars1(CgState *st, double s1, double s2, double *hist) {
   st->pending = 0;
   const int iter = st->iter + 1;
   st->iter = iter;
@@ -327,9 +340,25 @@ __global__ void __launch_bounds__(kScalThreads)
 }
 
 __global__ void __launch_bounds__(kScalThreads)
-    k_cg_scalars2(CgState *__restrict__ st, const double *__restrict__ rp1, int n1,
-                  const double *__restrict__ rp2, int n2, double *__restrict__ hist) {
+    k_cg_scalars1(CgState *__restrict__ st, const double *__restrict__ part1,
+                  const double *__restrict__ part2, int nparts, double *__restrict__ hist,
+                  BoxRef rep) {
   if (st->done) return;
+  const double s1 = block_sum_array(part1, nparts);
+  const double s2 = block_sum_array(part2, nparts);
+  if (threadIdx.x != 0) return;
+  cg_scalars1(st, s1, s2, hist);
+  state_report(st, rep);
+}
+
+__global__ void __launch_bounds__(kScalThreads)
+    k_cg_scalars2(CgState *__restrict__ st, const double *__restrict__ rp1, int n1,
+                  const double *__restrict__ rp2, int n2, double *__restrict__ hist,
+                  BoxRef rep) {
+  if (st->done) {  // the solve's last kernel
+    if (threadIdx.x == 0) box_report(rep);
+    return;
+  }
   const double a = block_sum_array(rp1, n1);
   const double b = (n2 > 0) ? block_sum_array(rp2, n2) : 0.0;
   if (threadIdx.x != 0) return;
@@ -544,13 +573,7 @@ __global__ void __launch_bounds__(256)
 
 // refresh, part 3: the true residual's norm decides the exit; otherwise the
 // iteration continues from it with the same search direction
-__global__ void __launch_bounds__(kScalThreads)
-    k_mcg_scalars1b(McgState *__restrict__ ms, const double *__restrict__ part1,
-                    const double *__restrict__ part2, int nparts, double *__restrict__ hist) {
-  if (ms->gate.done) return;
-  const double s1 = block_sum_array(part1, nparts);
-  const double s2 = block_sum_array(part2, nparts);
-  if (threadIdx.x != 0) return;
+__device__ void mcg_scalars1b(McgState *ms, double s1, double s2, double *hist) {
   CgState *st = &ms->cg;
   ms->gate.done = 1;
   ms->nrefresh += 1;
@@ -578,6 +601,22 @@ __global__ void __launch_bounds__(kScalThreads)
   st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
 }
 
+// (reports the state whether a refresh ran or not)
+__global__ void __launch_bounds__(kScalThreads)
+    k_mcg_scalars1b(McgState *__restrict__ ms, const double *__restrict__ part1,
+                    const double *__restrict__ part2, int nparts, double *__restrict__ hist,
+                    BoxRef rep) {
+  if (ms->gate.done) {
+    if (threadIdx.x == 0) state_report(&ms->cg, rep);
+    return;
+  }
+  const double s1 = block_sum_array(part1, nparts);
+  const double s2 = block_sum_array(part2, nparts);
+  if (threadIdx.x != 0) return;
+  mcg_scalars1b(ms, s1, s2, hist);
+  state_report(&ms->cg, rep);
+}
+
 // x = 0, xs = 0, r = f (rounded), and 1/d (d the assembled diagonal), its
 // product with mult and binv*mult (or mult) in FP32; the first iteration's
 // partial sums
@@ -586,7 +625,9 @@ __global__ void __launch_bounds__(256)
                float *__restrict__ d32, float *__restrict__ dm, float *__restrict__ bm,
                const double *__restrict__ f, const double *__restrict__ d,
                const double *__restrict__ mult, const double *__restrict__ binv, int plain_norm,
-               int64_t n, double *__restrict__ part1, double *__restrict__ part2) {
+               int64_t n, double *__restrict__ part1, double *__restrict__ part2, McgState init,
+               McgState *__restrict__ ms) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *ms = init;
   double s1 = 0.0, s2 = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -619,7 +660,40 @@ int ensure_small(Mesh &m) {
   // room for the mixed-precision solve's state (a CgState first)
   if (!m.st) NK_HIP(hipMalloc(&m.st, sizeof(McgState)));
   if (!m.red) NK_HIP(hipMalloc(&m.red, sizeof(double) * kRedSize));
+  if (!m.box) NK_TRY(box_alloc(&m.box));
   return NKH_OK;
+}
+
+int box_alloc(HostBox **b) {
+  NK_HIP(hipHostMalloc(reinterpret_cast<void **>(b), sizeof(HostBox),
+                       hipHostMallocMapped | hipHostMallocCoherent));
+  std::memset(static_cast<void *>(*b), 0, sizeof(HostBox));
+  return NKH_OK;
+}
+
+namespace {
+__global__ void k_box_report(BoxRef r) { box_report(r); }
+}  // namespace
+
+int box_join(const BoxRef &r, hipStream_t s) {
+  hipLaunchKernelGGL(k_box_report, dim3(1), dim3(1), 0, s, r);
+  NK_HIP(hipGetLastError());
+  return box_wait(r, s);
+}
+
+int box_wait(const BoxRef &r, hipStream_t s) {
+  for (int64_t spin = 1;; ++spin) {
+    if (__atomic_load_n(&r.b->seq, __ATOMIC_ACQUIRE) >= r.seq) return NKH_OK;
+    if (spin % 8192 == 0) {  // every 50 us or so
+      const hipError_t e = hipStreamQuery(s);
+      if (e == hipErrorNotReady) continue;
+      NK_HIP(e);
+      NK_CHECK(__atomic_load_n(&r.b->seq, __ATOMIC_ACQUIRE) >= r.seq, NKH_ERR_STATE,
+               "a solve's kernels ended without their report");
+      return NKH_OK;
+    }
+    __builtin_ia32_pause();
+  }
 }
 
 int ensure_workspace(Mesh &m) {
@@ -640,16 +714,17 @@ int ensure_workspace(Mesh &m) {
 // at red + kRedOut, the group flags of mask in flag.
 static int enqueue_facts(Mesh &m, const double *h1, const double *h2, const double *mask,
                          const double *mult, double *f, const FactsAsk &ask, double *red,
-                         uint8_t *flag, hipStream_t s) {
+                         uint8_t *flag, const BoxRef &rep, hipStream_t s) {
   static_assert(kNF * kRedBlocks <= kRedRho2, "the partial sums take the dots' place");
   double *part = red + kRedPart1, *res = red + kRedOut;
+  int *left = reinterpret_cast<int *>(res + kNF + 1);
   const int64_t per = 1024;  // nodes per block, up to the fixed grid
   const int nb = (int)std::min<int64_t>(std::max<int64_t>((m.n + per - 1) / per, 1), kRedBlocks);
   hipLaunchKernelGGL(k_facts, dim3(nb), dim3(256), 0, s, h1, h2, mask, mult, f,
                      ask.mask_f ? 1 : 0, ask.chk ? m.binv : nullptr, ask.other_mask, ask.code,
-                     m.n, m.np, part, res + kNF);
+                     m.n, m.np, part, res + kNF, left);
   NK_TRY(gs_prepare(m.gs, mask, mult, flag, res + kNF, s));
-  hipLaunchKernelGGL(k_facts_final, dim3(kNF), dim3(256), 0, s, part, nb, res);
+  hipLaunchKernelGGL(k_facts_final, dim3(kNF), dim3(256), 0, s, part, nb, res, left, rep);
   NK_HIP(hipGetLastError());
   return NKH_OK;
 }
@@ -682,7 +757,13 @@ int gather_facts(Mesh &m, const double *h1, const double *h2, const double *mask
                  hipStream_t s) {
   NK_TRY(ensure_small(m));
   if (!m.gs.flag && m.gs.ngroups > 0) NK_HIP(hipMalloc(&m.gs.flag, (size_t)m.gs.ngroups));
-  NK_TRY(enqueue_facts(m, h1, h2, mask, mult, f, ask, m.red, m.gs.flag, s));
+  const BoxRef rep = m.next_report();
+  NK_TRY(enqueue_facts(m, h1, h2, mask, mult, f, ask, m.red, m.gs.flag, rep, s));
+  if (rep.b) {
+    NK_TRY(box_wait(rep, s));
+    *out = read_facts(m, h1, h2, rep.b->v);
+    return NKH_OK;
+  }
   double h[kNF + 1];
   NK_HIP(hipMemcpyAsync(h, m.red + kRedOut, sizeof(h), hipMemcpyDeviceToHost, s));
   NK_HIP(hipStreamSynchronize(s));
@@ -741,7 +822,7 @@ int run_chktcg1(Mesh &m, double *tol, const SolveFacts &facts) {
 }
 
 // One Jacobi-PCG solve whose iterations can be enqueued one at a time (the
-// single solve below, and the batch of solves captured in a graph).
+// single solve below, and the batch of solves).
 struct CgRun {
   Mesh *m = nullptr;
   double *x = nullptr, *r = nullptr, *w = nullptr, *p = nullptr, *d = nullptr, *dm = nullptr,
@@ -754,6 +835,17 @@ struct CgRun {
   bool fused = false, vec_ok = false, trivial = false;
   int niter = 0, launched = 0, ax_grid_parts = 0;
   double *hist = nullptr;
+  // An iteration makes two reports: the state after its exit test, and the
+  // end of its last kernel if the solve is done (a solve returns only when
+  // nothing of it is left to run).
+  HostBox *box = nullptr;  // null: no reports
+  BoxRef last;             // the second report of the iteration enqueued last
+  BoxRef exit_test() const { return BoxRef{box, last.seq - 1}; }
+  int wait(CgState *hs, hipStream_t s) const {
+    NK_TRY(box_wait(exit_test(), s));
+    std::memcpy(hs, box->v, sizeof(CgState));
+    return hs->done ? box_wait(last, s) : NKH_OK;
+  }
 
   // hmholtz.f:611-720 up to the loop: preconditioner, r = f, null-space check,
   // choice of the fused iteration, device state.  ws: 6 n doubles, red:
@@ -792,17 +884,6 @@ struct CgRun {
     // the operator's kernel choice for this order (w is scratch until then)
     NK_TRY(axhelm_autotune(mesh, w, f, h1, h2, s));
     NK_TRY(setprec_sum(mesh, d, h1, h2, s));
-    hipLaunchKernelGGL(k_cg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, r, f, d, mult,
-                       mesh.binv, dm, bm, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
-                       red + kRedPart2);
-    NK_HIP(hipGetLastError());
-    // Fused iteration (rho inside axhelm, mask inside the assembly) when its
-    // conditions hold and f is zero where masked.
-    fused = facts.fused() && facts.fmasked == 0.0;
-    flag = mesh.gs.flag;
-    ax_grid_parts = axhelm_cg_grid(mesh);
-    auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    vec_ok = al16(x) && al16(r) && al16(p) && al16(w) && al16(dm) && al16(bm);
     CgState h{};
     h.rtz1 = 1.0;
     h.tol = tol;
@@ -812,7 +893,17 @@ struct CgRun {
     h.maxit = niter;
     h.istep = prm.istep;
     h.param18 = prm.param18;
-    NK_HIP(hipMemcpyAsync(st, &h, sizeof(CgState), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_cg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, r, f, d, mult,
+                       mesh.binv, dm, bm, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
+                       red + kRedPart2, h, st);
+    NK_HIP(hipGetLastError());
+    // Fused iteration (rho inside axhelm, mask inside the assembly) when its
+    // conditions hold and f is zero where masked.
+    fused = facts.fused() && facts.fmasked == 0.0;
+    flag = mesh.gs.flag;
+    ax_grid_parts = axhelm_cg_grid(mesh);
+    auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    vec_ok = al16(x) && al16(r) && al16(p) && al16(w) && al16(dm) && al16(bm);
     hist = nullptr;
     if (want_hist) {
       hist = red + kRedHist;
@@ -833,8 +924,9 @@ struct CgRun {
     if (launched > 0)  // (the first iteration's sums come from k_cg_init)
       hipLaunchKernelGGL((vec_ok ? k_cg_update_dots<true> : k_cg_update_dots<false>), dim3(ub),
                          dim3(256), 0, s, x, r, p, w, dm, bm, n, st, part1, part2);
+    last = BoxRef{box, last.seq + 2};
     hipLaunchKernelGGL(k_cg_scalars1, dim3(1), dim3(kScalThreads), 0, s, st, part1, part2, ub,
-                       hist);
+                       hist, exit_test());
     if (fused) {
       if (ev) NK_HIP(hipEventRecord(ev[0], s));
       NK_TRY(launch_axhelm_cg(*m, w, p, r, d, h1, h2, mult, st, rho1, s));
@@ -842,7 +934,7 @@ struct CgRun {
       NK_TRY(gs_assemble(m->gs, w, st, s, flag));
       if (ev) NK_HIP(hipEventRecord(ev[2], s));
       hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st, rho1,
-                         ax_grid_parts, rho2, 0, hist);
+                         ax_grid_parts, rho2, 0, hist, last);
     } else {
       NK_TRY(launch_axhelm_cg(*m, w, p, r, d, h1, h2, mult, st, nullptr, s));
       NK_TRY(gs_op(m->gs, w, 0, s));
@@ -850,7 +942,7 @@ struct CgRun {
       hipLaunchKernelGGL(k_dot3_guarded, dim3(kRedBlocks), dim3(256), 0, s, w, p, mult, n, st,
                          rho1);
       hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st, rho1, kRedBlocks,
-                         rho2, 0, hist);
+                         rho2, 0, hist, last);
     }
     NK_HIP(hipGetLastError());
     ++launched;
@@ -888,6 +980,17 @@ struct McgRun {
   bool trivial = false, vec_ok = false, fused = true;
   int niter = 0, launched = 0, ax_grid_parts = 0;
   double *hist = nullptr;
+  // An iteration makes two reports: the state after its exit test, and the
+  // end of its last kernel if the solve is done (a solve returns only when
+  // nothing of it is left to run).
+  HostBox *box = nullptr;  // null: no reports
+  BoxRef last;             // the second report of the iteration enqueued last
+  BoxRef exit_test() const { return BoxRef{box, last.seq - 1}; }
+  int wait(CgState *hs, hipStream_t s) const {
+    NK_TRY(box_wait(exit_test(), s));
+    std::memcpy(hs, box->v, sizeof(CgState));
+    return hs->done ? box_wait(last, s) : NKH_OK;
+  }
 
   int begin(Mesh &mesh, double *ws, double *red_, void *st_, double *x_, const double *f_,
             const SolveFacts &facts, const double *mask, const double *mult, double tin,
@@ -931,14 +1034,6 @@ struct McgRun {
     flag = mesh.gs.flag;
     NK_TRY(axhelm_autotune(mesh, ax, f, h1, h2, s));  // the refreshes' operator
     NK_TRY(setprec_sum(mesh, ax, h1, h2, s));  // the diagonal (FP64) in the ax slot
-    hipLaunchKernelGGL(k_mcg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, r, d, dm, bm, f,
-                       ax, mult, mesh.binv, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
-                       red + kRedPart2);
-    NK_HIP(hipGetLastError());
-    NK_TRY(ensure_geom32(mesh, s));
-    ax_grid_parts = axhelm_cg_grid(mesh);
-    auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    vec_ok = al16(r) && al16(p) && al16(w) && al16(xs) && al16(dm) && al16(bm);
     McgState h{};
     h.cg.rtz1 = 1.0;
     h.cg.tol = tol;
@@ -949,7 +1044,14 @@ struct McgRun {
     h.cg.istep = prm.istep;
     h.cg.param18 = prm.param18;
     h.gate.done = 1;
-    NK_HIP(hipMemcpyAsync(ms, &h, sizeof(McgState), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_mcg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, r, d, dm, bm, f,
+                       ax, mult, mesh.binv, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
+                       red + kRedPart2, h, ms);
+    NK_HIP(hipGetLastError());
+    NK_TRY(ensure_geom32(mesh, s));
+    ax_grid_parts = axhelm_cg_grid(mesh);
+    auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    vec_ok = al16(r) && al16(p) && al16(w) && al16(xs) && al16(dm) && al16(bm);
     hist = nullptr;
     if (want_hist) {
       hist = red + kRedHist;
@@ -978,15 +1080,16 @@ struct McgRun {
     NK_TRY(gs_assemble(m->gs, ax, gate, s, flag, rb));
     hipLaunchKernelGGL(k_mcg_resid, dim3(rb), dim3(256), 0, s, r, f, ax, dm, bm, n, gate, part1,
                        part2);
+    last = BoxRef{box, last.seq + 2};
     hipLaunchKernelGGL(k_mcg_scalars1b, dim3(1), dim3(kScalThreads), 0, s, ms, part1, part2, rb,
-                       hist);
+                       hist, exit_test());
     if (ev) NK_HIP(hipEventRecord(ev[0], s));
     NK_TRY(launch_axhelm32_jac(*m, w, p, r, d, (float)h1.s, (float)h2.s, st, rho1, s));
     if (ev) NK_HIP(hipEventRecord(ev[1], s));
     NK_TRY(gs_assemble(m->gs, w, st, s, flag));
     if (ev) NK_HIP(hipEventRecord(ev[2], s));
     hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st, rho1,
-                       ax_grid_parts, rho2, 0, hist);
+                       ax_grid_parts, rho2, 0, hist, last);
     NK_HIP(hipGetLastError());
     ++launched;
     return NKH_OK;
@@ -1027,7 +1130,8 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
     return NKH_OK;
   }
   CgState hs{};
-  int check_every = 1;
+  run.box = m.box;
+  run.last.seq = m.box_seq;
   // CTIMER mirror: event pairs around axhelm and gs of every launched iteration
   const bool timed = allow_timers && timers().on;
   const int niter = run.niter;
@@ -1042,15 +1146,21 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
     NK_HIP(hipEventCreate(&t_solve1));
     NK_HIP(hipEventRecord(t_solve0, s));
   }
+  // Each iteration's exit test reports to the host, which enqueues the next
+  // iteration while the operator of this one runs.  Without a report (the
+  // allocation-free solve) the state is copied back, later on every fourth
+  // iteration.
   while (true) {
     NK_TRY(run.enqueue(s, timed ? &ev[4 * run.launched] : nullptr));
-    if (run.launched % check_every == 0 || run.launched > niter) {
+    if (run.box) {
+      m.box_seq = run.last.seq;
+      NK_TRY(run.wait(&hs, s));
+    } else if (run.launched < 8 || run.launched % 4 == 0 || run.launched > niter) {
       NK_HIP(hipMemcpyAsync(&hs, run.st, sizeof(CgState), hipMemcpyDeviceToHost, s));
       NK_HIP(hipStreamSynchronize(s));
-      if (hs.done) break;
-      NK_CHECK(run.launched <= niter + 1, NKH_ERR_STATE, "cggo: state machine did not terminate");
-      if (run.launched >= 8) check_every = 4;
     }
+    if (hs.done) break;
+    NK_CHECK(run.launched <= niter + 1, NKH_ERR_STATE, "cggo: state machine did not terminate");
   }
   if (timed) {
     NK_HIP(hipEventRecord(t_solve1, s));
@@ -1145,6 +1255,7 @@ int run_cggo_noalloc(Mesh &m, double *x, const double *f, const double *h1, cons
   // a view of the mesh whose solve buffers are the scratch: the geometry
   // and gather-scatter map are the mesh's own, nothing of it is changed
   Mesh v = m;
+  v.box = nullptr;
   v.ws = sp;
   v.ws_doubles = kNoAllocWs;
   v.red = sp + kNoAllocWs;
@@ -1159,18 +1270,14 @@ int run_cggo_noalloc(Mesh &m, double *x, const double *f, const double *h1, cons
 
 // ---------------------------------------------------------------------------
 // Batched Jacobi-PCG: several hmholtz solves (different meshes, h1/h2,
-// masks, sizes; the same lx1 or not) iterate together.  Each solve keeps its
-// own work space, state and gs group flags; kGraphIters steady-state
-// iterations of all of them -- each solve's launches on its own stream,
-// forked from and joined to a library stream once per replay -- are
-// captured once in a hipGraph and replayed until every solve has stopped (a
-// finished solve's kernels return at once).  No memset is recorded in the
-// graph.
+// masks, sizes; the same lx1 or not) iterate together, each with its own work
+// space, state, gs group flags and stream.  The host enqueues the next
+// iteration of whichever solve has reported its exit test, so that the solves
+// run side by side and none waits for another.  (A captured graph of eight
+// iterations of all of them, built on every call, took longer to build than
+// small solves take to run: five solves of 560 to 1,320 elements 3.3 ms per
+// call with it.)
 // ---------------------------------------------------------------------------
-// iterations per replay of the batch graph (the host reads the states after
-// each replay)
-constexpr int kGraphIters = 8;
-
 struct CgBatch {
   int nb = 0;
   std::vector<int> mesh;
@@ -1180,16 +1287,12 @@ struct CgBatch {
   std::vector<int64_t> nflag;
   std::vector<hipStream_t> streams;
   std::vector<hipEvent_t> ev;  // fork + one join per solve
-  // the graph is captured and launched on a library stream (capture is not
-  // allowed on the caller's stream when that is the null stream), ordered
-  // after and before the caller's stream by ev_sync
-  hipStream_t cap = nullptr;
-  hipEvent_t ev_sync = nullptr;
+  std::vector<HostBox *> box;
+  std::vector<unsigned long long> seq;  // reports so far
   void release() {
-    if (cap) (void)hipStreamDestroy(cap);
-    if (ev_sync) (void)hipEventDestroy(ev_sync);
-    cap = nullptr;
-    ev_sync = nullptr;
+    for (HostBox *q : box)
+      if (q) (void)hipHostFree(q);
+    box.clear();
     for (double *q : ws) (void)hipFree(q);
     for (double *q : red) (void)hipFree(q);
     for (CgState *q : st) (void)hipFree(q);
@@ -1247,6 +1350,10 @@ int batch_create(int nb, const int *meshes, int *id) {
     B->flag.push_back(fl);
     B->nflag.push_back(m->gs.ngroups);
     B->streams.push_back(q);
+    B->box.push_back(nullptr);
+    B->seq.push_back(0);
+    const int rc = box_alloc(&B->box.back());
+    if (rc != NKH_OK) return fail(rc);
   }
   for (int k = 0; k <= nb; ++k) {
     hipEvent_t e;
@@ -1255,11 +1362,6 @@ int batch_create(int nb, const int *meshes, int *id) {
       return fail(NKH_ERR_HIP);
     }
     B->ev.push_back(e);
-  }
-  if (hipStreamCreateWithFlags(&B->cap, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&B->ev_sync, hipEventDisableTiming) != hipSuccess) {
-    set_error("nkh_batch_create: stream creation failed");
-    return fail(NKH_ERR_HIP);
   }
   g_batches.push_back(B);
   *id = (int)g_batches.size() - 1;
@@ -1288,7 +1390,7 @@ int batch_facts(int id, const nkh_batch_solve *solves, bool chk, SolveFacts *out
   NK_CHECK(id >= 0 && id < (int)g_batches.size() && g_batches[(size_t)id], NKH_ERR_ARG,
            "batch: bad handle %d", id);
   CgBatch &B = *g_batches[(size_t)id];
-  std::vector<double> h((size_t)B.nb * (kNF + 1));
+  std::vector<BoxRef> rep((size_t)B.nb);
   FactsAsk ask;
   ask.mask_f = true;
   ask.chk = chk;
@@ -1298,15 +1400,15 @@ int batch_facts(int id, const nkh_batch_solve *solves, bool chk, SolveFacts *out
     NK_CHECK(m->gs.ngroups == B.nflag[(size_t)k], NKH_ERR_STATE,
              "batch: the gather-scatter map of solve %d changed", k);
     const nkh_batch_solve &q = solves[k];
+    rep[(size_t)k] = BoxRef{B.box[(size_t)k], ++B.seq[(size_t)k]};
     NK_TRY(enqueue_facts(*m, q.h1, q.h2, q.mask, q.mult, q.rhs, ask, B.red[(size_t)k],
-                         B.flag[(size_t)k], s));
-    NK_HIP(hipMemcpyAsync(&h[(size_t)k * (kNF + 1)], B.red[(size_t)k] + kRedOut,
-                          sizeof(double) * (kNF + 1), hipMemcpyDeviceToHost, s));
+                         B.flag[(size_t)k], rep[(size_t)k], s));
   }
-  NK_HIP(hipStreamSynchronize(s));
-  for (int k = 0; k < B.nb; ++k)
+  for (int k = 0; k < B.nb; ++k) {
+    NK_TRY(box_wait(rep[(size_t)k], s));
     out[k] = read_facts(*get_mesh(B.mesh[(size_t)k]), solves[k].h1, solves[k].h2,
-                        &h[(size_t)k * (kNF + 1)]);
+                        B.box[(size_t)k]->v);
+  }
   return NKH_OK;
 }
 
@@ -1331,75 +1433,54 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
     if (m->gs.ngroups > 0) runs[(size_t)k].flag = B.flag[(size_t)k];
     active.push_back(k);
   }
-  // the first iteration (no pending update) eagerly, then the graph; all of
-  // it on the batch's own stream c, after the set-up on s
-  hipStream_t c = B.cap;
-  NK_HIP(hipEventRecord(B.ev_sync, s));
-  NK_HIP(hipStreamWaitEvent(c, B.ev_sync, 0));
-  auto fork_join = [&](auto &&body) -> int {
-    NK_HIP(hipEventRecord(B.ev[0], c));
-    for (int k : active) {
-      hipStream_t q = B.streams[(size_t)k];
-      NK_HIP(hipStreamWaitEvent(q, B.ev[0], 0));
-      NK_TRY(body(k, q));
-      NK_HIP(hipEventRecord(B.ev[(size_t)k + 1], q));
-    }
-    for (int k : active) NK_HIP(hipStreamWaitEvent(c, B.ev[(size_t)k + 1], 0));
-    return NKH_OK;
-  };
+  // every solve on its own stream, after the set-up on s
   int launches = 0;
   if (!active.empty()) {
-    NK_TRY(fork_join([&](int k, hipStream_t q) { return runs[(size_t)k].enqueue(q); }));
-    launches = 1;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    // the graph: kGraphIters iterations of every solve, each solve on its own
-    // stream (solves do not wait for each other between iterations)
-    NK_HIP(hipStreamBeginCapture(c, hipStreamCaptureModeThreadLocal));
-    const int rc_cap = fork_join([&](int k, hipStream_t q) {
-      for (int it = 0; it < kGraphIters; ++it) NK_TRY(runs[(size_t)k].enqueue(q));
-      return NKH_OK;
-    });
-    const hipError_t end = hipStreamEndCapture(c, &graph);
-    NK_TRY(rc_cap);
-    NK_HIP(end);
-    NK_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    int niter_max = 0;
-    for (int k : active) niter_max = std::max(niter_max, runs[(size_t)k].niter);
-    std::vector<CgState> hs((size_t)B.nb);
+    NK_HIP(hipEventRecord(B.ev[0], s));
     int rc = NKH_OK;
-    while (true) {
-      if (hipGraphLaunch(exec, c) != hipSuccess) {
-        set_error("batch: graph launch failed");
-        rc = NKH_ERR_HIP;
-        break;
-      }
-      launches += kGraphIters;
-      {
-        for (int k : active)
-          (void)hipMemcpyAsync(&hs[(size_t)k], B.st[(size_t)k], sizeof(CgState),
-                               hipMemcpyDeviceToHost, c);
-        if (hipStreamSynchronize(c) != hipSuccess) {
-          set_error("batch: state read-back failed");
-          rc = NKH_ERR_HIP;
-          break;
+    std::vector<int> open;
+    for (int k : active) {
+      Run &run = runs[(size_t)k];
+      run.box = B.box[(size_t)k];
+      run.last.seq = B.seq[(size_t)k];
+      NK_HIP(hipStreamWaitEvent(B.streams[(size_t)k], B.ev[0], 0));
+      if (rc == NKH_OK) rc = run.enqueue(B.streams[(size_t)k]);
+      B.seq[(size_t)k] = run.last.seq;
+      open.push_back(k);
+    }
+    // round robin over the solves that have not ended: their report is read,
+    // then their next iteration enqueued
+    while (rc == NKH_OK && !open.empty()) {
+      std::vector<int> next;
+      for (int k : open) {
+        Run &run = runs[(size_t)k];
+        hipStream_t q = B.streams[(size_t)k];
+        CgState hs;
+        if ((rc = run.wait(&hs, q)) != NKH_OK) break;
+        if (hs.done) {
+          run.result(hs, &res[k]);
+          continue;
         }
-        bool all = true;
-        for (int k : active) all = all && hs[(size_t)k].done;
-        if (all) break;
-        if (launches > niter_max + kGraphIters) {
-          set_error("batch: state machines did not terminate");
+        if (run.launched > run.niter + 1) {
+          set_error("batch: a state machine did not terminate");
           rc = NKH_ERR_STATE;
           break;
         }
+        if ((rc = run.enqueue(q)) != NKH_OK) break;
+        B.seq[(size_t)k] = run.last.seq;
+        next.push_back(k);
       }
+      open.swap(next);
     }
-    (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
+    // the caller's stream goes on after every solve's, also after an error
+    // (which leaves work in flight)
+    for (int k : active) {
+      if (rc != NKH_OK) (void)hipStreamSynchronize(B.streams[(size_t)k]);
+      launches = std::max(launches, runs[(size_t)k].launched);
+      (void)hipEventRecord(B.ev[(size_t)k + 1], B.streams[(size_t)k]);
+      (void)hipStreamWaitEvent(s, B.ev[(size_t)k + 1], 0);
+    }
     NK_TRY(rc);
-    NK_HIP(hipEventRecord(B.ev_sync, c));
-    NK_HIP(hipStreamWaitEvent(s, B.ev_sync, 0));
-    for (int k : active) runs[(size_t)k].result(hs[(size_t)k], &res[k]);
   }
   for (int k = 0; k < B.nb; ++k)
     if (runs[(size_t)k].trivial) runs[(size_t)k].result(CgState{}, &res[k]);

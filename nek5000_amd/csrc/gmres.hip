@@ -3,7 +3,7 @@
 //
 // Krylov vectors V (m+1) and preconditioned vectors Z (m) stay in HBM; the
 // small Hessenberg problem (Givens rotations, back substitution) runs on the
-// host from the Gram-Schmidt coefficients read back each step.  Dots are
+// host from the Gram-Schmidt coefficients each step reports.  Dots are
 // fixed-grid partial sums reduced in a fixed order.  ml = mu = 1 in the
 // reference (uzawa_gmres_split, gmres.f:252-271), so there is no scaling.
 #include <algorithm>
@@ -30,12 +30,6 @@ __device__ __forceinline__ void store_part(double a, double *part) {
   __syncthreads();
   if (threadIdx.x == 0) part[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
   __syncthreads();
-}
-
-// w = v * mgmask (h1mg_solve masks its right-hand side in place)
-__global__ void k_gm_copy_mask(double *__restrict__ w, const double *__restrict__ v,
-                               const double *__restrict__ mask, int64_t n) {
-  NK_LOOP(i, n) w[i] = v[i] * mask[i];
 }
 
 // r = res - mask*w; partial sum r*r*wt   (r = res - A x with ax's mask)
@@ -77,8 +71,10 @@ __global__ void __launch_bounds__(256)
     if (c < cnt) store_part(acc[c], part + (int64_t)(i0 + c) * kGmBlocks);
 }
 
-// out[i] = fixed-order sum of the kGmBlocks partials of dot i (block i)
-__global__ void __launch_bounds__(256) k_gm_final(const double *part, double *out) {
+// out[i] = fixed-order sum of the kGmBlocks partials of dot i (block i); with
+// a report (one block), that sum and the nh doubles h before it
+__global__ void __launch_bounds__(256)
+    k_gm_final(const double *part, double *out, const double *h, int nh, BoxRef rep) {
   __shared__ double sa[4];
   const double *p = part + (int64_t)blockIdx.x * kGmBlocks;
   double a = 0.0;
@@ -87,7 +83,13 @@ __global__ void __launch_bounds__(256) k_gm_final(const double *part, double *ou
   if ((threadIdx.x & 63) == 0) sa[threadIdx.x >> 6] = a;
   __syncthreads();
   if (threadIdx.x == 0) out[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
+  if (rep.b && threadIdx.x == 0) {
+    for (int i = 0; i < nh; ++i) rep.b->v[i] = h[i];
+    rep.b->v[nh] = out[blockIdx.x];
+    box_report(rep);
+  }
 }
+static_assert(kGmresM + 1 <= (int)(sizeof(HostBox::v) / sizeof(double)), "a report holds a step");
 
 // w = w - h_i v_i for i = 0..j-1 in order (add2s2), then partial w*w*wt
 __global__ void __launch_bounds__(256)
@@ -104,18 +106,29 @@ __global__ void __launch_bounds__(256)
   store_part(a, part);
 }
 
-// v = w * s (cmult2)
-__global__ void k_gm_scale(double *__restrict__ v, const double *__restrict__ w, double s,
-                           int64_t n) {
-  NK_LOOP(i, n) v[i] = w[i] * s;
+// v = u / sqrt(*a2) (cmult2: the next Krylov vector), w = v * mgmask (the
+// right-hand side that h1mg_solve masks in place).  It needs no host: the
+// step's report is on its way meanwhile.
+__global__ void __launch_bounds__(256)
+    k_gm_next(double *__restrict__ v, double *w, const double *u, const double *__restrict__ a2,
+              const double *__restrict__ mask, int64_t n) {
+  const double s = 1.0 / sqrt(*a2);
+  NK_LOOP(i, n) {
+    const double vi = u[i] * s;
+    v[i] = vi;
+    w[i] = vi * mask[i];
+  }
 }
 
+struct GmCoef {
+  double c[kGmresM];
+};
 // x = x + c_i z_i for i = 0..j-1 in order
-__global__ void k_gm_xupd(double *__restrict__ x, const double *__restrict__ Z,
-                          const double *__restrict__ c, int j, int64_t n) {
+__global__ void k_gm_xupd(double *__restrict__ x, const double *__restrict__ Z, GmCoef c, int j,
+                          int64_t n) {
   NK_LOOP(q, n) {
     double xq = x[q];
-    for (int i = 0; i < j; ++i) xq = xq + c[i] * Z[(int64_t)i * n + q];
+    for (int i = 0; i < j; ++i) xq = xq + c.c[i] * Z[(int64_t)i * n + q];
     x[q] = xq;
   }
 }
@@ -145,7 +158,8 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
     NK_TRY(mg_dalloc(&mg.gsm, 2 * (M + 2)));
   }
   double *V = mg.gV, *Z = mg.gZ, *x = mg.gx, *r = mg.gr, *w = mg.gw, *part = mg.gpart;
-  double *dh = mg.gsm, *dc = mg.gsm + (M + 2);
+  double *dh = mg.gsm, *da2 = mg.gsm + (M + 2);  // h(1..j); the squared norm after them
+  NK_TRY(ensure_small(m));
   const double *mgmask = mg.lev[mg.lmax].mask;
   const dim3 G(kGmBlocks), B(256);
   const double norm_fac = 1.0 / std::sqrt(m.vol);
@@ -156,14 +170,14 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
   if (prm.param21 > 0 && tolps > std::fabs(prm.param21)) tolps = std::fabs(prm.param21);
   if (prm.istep == 0) tolps = 1.e-4;
   double tolpss = tolps;
-  std::vector<double> H((size_t)M * M, 0.0), gam(M + 1, 0.0), c(M, 0.0), sn(M, 0.0), hv(M + 2);
+  std::vector<double> H((size_t)M * M, 0.0), gam(M + 1, 0.0), c(M, 0.0), sn(M, 0.0);
   auto HH = [&](int i, int jj) -> double & { return H[(size_t)i + (size_t)M * jj]; };
-  auto dot_final = [&](int count, double *host) -> int {
-    hipLaunchKernelGGL(k_gm_final, dim3(count), B, 0, s, part, dh);
-    NK_HIP(hipGetLastError());
-    NK_HIP(hipMemcpyAsync(host, dh, sizeof(double) * count, hipMemcpyDeviceToHost, s));
-    NK_HIP(hipStreamSynchronize(s));
-    return NKH_OK;
+  // the squared norm's partials to *da2, and with the nh coefficients of dh
+  // to the host (wait by box_wait)
+  auto norm_report = [&](int nh) -> BoxRef {
+    const BoxRef rep = m.next_report();
+    hipLaunchKernelGGL(k_gm_final, dim3(1), B, 0, s, part, da2, dh, nh, rep);
+    return rep;
   };
   hipLaunchKernelGGL(k_gm_zero, dim3(mg_grid(n)), B, 0, s, x, n);
   double div0 = 0.0, rnorm = 0.0;
@@ -176,20 +190,20 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
       NK_TRY(gs_op(m.gs, w, 0, s));
     }
     hipLaunchKernelGGL(k_gm_resid, G, B, 0, s, r, res, w, mask, wt, n, iter == 0 ? 1 : 0, part);
-    double g2;
-    NK_TRY(dot_final(1, &g2));
-    gam[0] = std::sqrt(g2);
+    const BoxRef rep0 = norm_report(0);
+    hipLaunchKernelGGL(k_gm_next, dim3(mg_grid(n)), B, 0, s, V, w, r, da2, mgmask, n);
+    NK_HIP(hipGetLastError());
+    NK_TRY(box_wait(rep0, s));
+    gam[0] = std::sqrt(rep0.b->v[0]);
     if (iter == 0) {
       div0 = gam[0] * norm_fac;
       if (prm.param21 < 0) tolpss = std::fabs(prm.param21) * div0;
     }
     rnorm = 0.0;
     if (gam[0] == 0.0) break;
-    hipLaunchKernelGGL(k_gm_scale, dim3(mg_grid(n)), B, 0, s, V, r, 1.0 / gam[0], n);
     for (j = 1; j <= M; ++j) {
       iter += 1;
-      double *vj = V + (int64_t)(j - 1) * n, *zj = Z + (int64_t)(j - 1) * n;
-      hipLaunchKernelGGL(k_gm_copy_mask, dim3(mg_grid(n)), B, 0, s, w, vj, mgmask, n);
+      double *zj = Z + (int64_t)(j - 1) * n;
       NK_TRY(mg_solve(m, zj, w, s, prm.param40, prm.precision));
       if (nullsp) NK_TRY(mg_ortho(mg, zj, n, s));  // gmres.f:427
       NK_TRY(launch_axhelm(m, w, zj, h1, h2, s));
@@ -200,13 +214,16 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
         hipLaunchKernelGGL(k_gm_dots, G, B, 0, s, w, mask, i0 == 0 ? 1 : 0, V, n, i0, cnt, wt,
                            part);
       }
-      NK_HIP(hipGetLastError());
-      NK_TRY(dot_final(j, hv.data()));
-      for (int i = 1; i <= j; ++i) HH(i - 1, j - 1) = hv[(size_t)(i - 1)];
-      // dh still holds h(1..j) on the device
+      hipLaunchKernelGGL(k_gm_final, dim3(j), B, 0, s, part, dh, nullptr, 0, BoxRef{});
       hipLaunchKernelGGL(k_gm_orth, G, B, 0, s, w, V, dh, j, wt, n, part);
-      double a2;
-      NK_TRY(dot_final(1, &a2));
+      const BoxRef rep = norm_report(j);
+      if (j < M)  // (not read if this step is the last)
+        hipLaunchKernelGGL(k_gm_next, dim3(mg_grid(n)), B, 0, s, V + (int64_t)j * n, w, w, da2,
+                           mgmask, n);
+      NK_HIP(hipGetLastError());
+      NK_TRY(box_wait(rep, s));
+      for (int i = 1; i <= j; ++i) HH(i - 1, j - 1) = rep.b->v[i - 1];
+      const double a2 = rep.b->v[j];
       for (int i = 1; i <= j - 1; ++i) {  // previous Givens rotations
         const double temp = HH(i - 1, j - 1);
         HH(i - 1, j - 1) = c[i - 1] * temp + sn[i - 1] * HH(i, j - 1);
@@ -232,8 +249,6 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
         break;
       }
       if (j == M) break;  // restart
-      hipLaunchKernelGGL(k_gm_scale, dim3(mg_grid(n)), B, 0, s, V + (int64_t)j * n, w,
-                         1.0 / alpha, n);
     }
     if (j > M) j = M;
     // back substitution c = H^-1 gamma; x += sum c_i z_i (gmres.f:518-529)
@@ -242,14 +257,15 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
       for (int i = j; i >= k + 1; --i) temp = temp - HH(k - 1, i - 1) * c[i - 1];
       c[k - 1] = temp / HH(k - 1, k - 1);
     }
-    NK_HIP(hipMemcpyAsync(dc, c.data(), sizeof(double) * j, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_gm_xupd, dim3(mg_grid(n)), B, 0, s, x, Z, dc, j, n);
+    GmCoef cj{};
+    std::copy(c.begin(), c.begin() + j, cj.c);
+    hipLaunchKernelGGL(k_gm_xupd, dim3(mg_grid(n)), B, 0, s, x, Z, cj, j, n);
     NK_HIP(hipGetLastError());
   }
   // res = x (copy, gmres.f:535), orthogonalised against the null space (:534)
   NK_HIP(hipMemcpyAsync(res, x, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   if (nullsp) NK_TRY(mg_ortho(mg, res, n, s));
-  NK_HIP(hipStreamSynchronize(s));
+  NK_TRY(box_join(m.next_report(), s));
   if (out) {
     out->niter = iter;
     out->converged = rnorm < tolpss || gam[0] == 0.0;

@@ -1523,15 +1523,19 @@ __global__ void k_fcg_xfin(double *__restrict__ x, const double *__restrict__ p,
   }
 }
 
-__global__ void __launch_bounds__(256) k_fcg_rnorm(FcgState *st, const double *part, double vol) {
+__global__ void __launch_bounds__(256) k_fcg_rnorm(FcgState *st, const double *part, double vol,
+                                                   BoxRef rep) {
   const double t = final_sum(part);
   if (threadIdx.x == 0) {
     const double rn = sqrt(t / vol);
     st->rnorm = rn;
     st->iter += 1;
     if (rn < st->tolpss) st->done = 1;
+    *reinterpret_cast<FcgState *>(rep.b->v) = *st;
+    box_report(rep);
   }
 }
+static_assert(sizeof(FcgState) <= sizeof(HostBox::v), "a report holds a state");
 
 }  // namespace
 
@@ -1582,6 +1586,7 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
   // assembly, when the conditions for that identity hold (p = beta p + z
   // is continuous and zero where pmask is when pmask is the fine mask)
   const bool fused = !differ && facts.fused();
+  NK_TRY(ensure_small(m));
   double *rho_part = m.red + kRedRho1;
   const int nrho = axhelm_cg_grid(m);
   hipLaunchKernelGGL(k_fcg_init, g, b, 0, s, r, res, p, wt, mgmask, n, pa);
@@ -1627,19 +1632,17 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
       hipLaunchKernelGGL(k_fcg_update<uint8_t>, g, b, 0, s, res, r, p, w, wtc, mg.fst, n, pa);
     else
       hipLaunchKernelGGL(k_fcg_update<double>, g, b, 0, s, res, r, p, w, wt, mg.fst, n, pa);
-    hipLaunchKernelGGL(k_fcg_rnorm, dim3(1), b, 0, s, mg.fst, pa, m.vol);
+    const BoxRef rep = m.next_report();
+    hipLaunchKernelGGL(k_fcg_rnorm, dim3(1), b, 0, s, mg.fst, pa, m.vol, rep);
     if (hipGetLastError() != hipSuccess) {
       set_error("hmh_flex_cg: kernel launch failed");
       rc = NKH_ERR_HIP;
       break;
     }
-    if (hipMemcpyAsync(&hs, mg.fst, sizeof(FcgState), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess) {
-      set_error("hmh_flex_cg: state read-back failed");
-      rc = NKH_ERR_HIP;
-      break;
-    }
+    if ((rc = box_wait(rep, s)) != NKH_OK) break;
+    std::memcpy(&hs, rep.b->v, sizeof(FcgState));
     if (tm.on) {
+      (void)hipStreamSynchronize(s);
       float a = 0.f, c = 0.f;
       (void)hipEventElapsedTime(&a, ev[0], ev[1]);
       (void)hipEventElapsedTime(&c, ev[1], ev[2]);

@@ -11,6 +11,7 @@
 // outer tolerance), so two or three outer steps reach 1e-8.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "element_kernels.h"
@@ -170,13 +171,26 @@ __global__ void __launch_bounds__(256)
   part1(a, part);
 }
 
-__global__ void __launch_bounds__(256) k_mx_rnorm(MxState *st, const double *part, double vol) {
+__global__ void __launch_bounds__(256) k_mx_rnorm(MxState *st, const double *part, double vol,
+                                                  BoxRef rep) {
   const double t = fsum(part, kMxBlocks);
   if (threadIdx.x == 0) {
     const double rn = sqrt(t / vol);
     st->rnorm = rn;
     st->iter += 1;
     if (rn < st->tol) st->done = 1;
+    *reinterpret_cast<MxState *>(rep.b->v) = *st;
+    box_report(rep);
+  }
+}
+static_assert(sizeof(MxState) <= sizeof(HostBox::v), "a report holds a state");
+
+// the sum of the kMxBlocks partials, reported to the host
+__global__ void __launch_bounds__(256) k_mx_sum(const double *part, BoxRef rep) {
+  const double t = fsum(part, kMxBlocks);
+  if (threadIdx.x == 0) {
+    rep.b->v[0] = t;
+    box_report(rep);
   }
 }
 
@@ -633,6 +647,7 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
            "mixed-precision solve: h1 and h2 must be uniform");
   Mg &mg = *m.mg;
   hipStream_t s = cur_stream();
+  NK_TRY(ensure_small(m));
   const int64_t n = m.n;
   const double *mgmask = mg.lev[mg.lmax].mask;
   // the inner solver needs the identities of the fused FP64 path: pmask
@@ -668,12 +683,11 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
   NK_HIP(hipMemcpyAsync(b64, res, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   hipLaunchKernelGGL(k_mx_init, G, B, 0, s, r64, x64, b64, mgmask, wt, n, pc);
   auto host_sum = [&](double *part, double *v) -> int {
-    std::vector<double> h(kMxBlocks);
-    NK_HIP(hipMemcpyAsync(h.data(), part, sizeof(double) * kMxBlocks, hipMemcpyDeviceToHost, s));
-    NK_HIP(hipStreamSynchronize(s));
-    double a = 0.0;
-    for (double x : h) a += x;
-    *v = a;
+    const BoxRef rep = m.next_report();
+    hipLaunchKernelGGL(k_mx_sum, dim3(1), B, 0, s, part, rep);
+    NK_HIP(hipGetLastError());
+    NK_TRY(box_wait(rep, s));
+    *v = rep.b->v[0];
     return NKH_OK;
   };
   double t0;
@@ -707,10 +721,11 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
       else
         hipLaunchKernelGGL(k_mx_update<float>, G, B, 0, s, mg.xx, mg.xr, mg.xp, mg.xw, mg.xwt,
                            st, n, pa);
-      hipLaunchKernelGGL(k_mx_rnorm, dim3(1), B, 0, s, st, pa, m.vol);
+      const BoxRef rep = m.next_report();
+      hipLaunchKernelGGL(k_mx_rnorm, dim3(1), B, 0, s, st, pa, m.vol, rep);
       NK_HIP(hipGetLastError());
-      NK_HIP(hipMemcpyAsync(&hs, st, sizeof(MxState), hipMemcpyDeviceToHost, s));
-      NK_HIP(hipStreamSynchronize(s));
+      NK_TRY(box_wait(rep, s));
+      std::memcpy(&hs, rep.b->v, sizeof(MxState));
       if (rnorm_history) rnorm_history[total] = hs.rnorm;
       total += 1;
       if (hs.done) break;
@@ -728,7 +743,7 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
   NK_HIP(hipMemcpyAsync(res, x64, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   // hmholtz.f:2272: orthogonalise the solution against the null space
   if (mg_null_space_on(mg, h2)) NK_TRY(mg_ortho(mg, res, n, s));
-  NK_HIP(hipStreamSynchronize(s));
+  NK_TRY(box_join(m.next_report(), s));
   if (out) {
     out->niter = total;
     out->converged = rn < tolpss;

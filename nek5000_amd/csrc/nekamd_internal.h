@@ -100,6 +100,32 @@ struct CgState {
   int param18;
 };
 
+// Host memory that kernels report to: the thread that holds a result writes
+// it to v and then the report's number to seq, where the host, waiting for
+// that number, finds it a few microseconds later (a copy and a stream
+// synchronization leave the GPU idle for about 40 us; MI355X).
+struct HostBox {
+  unsigned long long seq;
+  unsigned long long pad[7];
+  double v[56];
+};
+// one report: its place and number (b null: none is made)
+struct BoxRef {
+  HostBox *b = nullptr;
+  unsigned long long seq = 0;
+};
+__device__ __forceinline__ void box_report(const BoxRef &r) {
+  if (!r.b) return;
+  __threadfence_system();
+  __hip_atomic_store(&r.b->seq, r.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+int box_alloc(HostBox **b);  // zeroed; freed by hipHostFree
+// Wait until r is reported by a kernel enqueued on s; an error of the stream,
+// or its end without the report, ends the wait.
+int box_wait(const BoxRef &r, hipStream_t s);
+// Wait for everything enqueued on s (a report from a kernel of its own).
+int box_join(const BoxRef &r, hipStream_t s);
+
 struct Mg;  // multigrid hierarchy (hsmg.hip)
 
 struct Mesh {
@@ -123,6 +149,9 @@ struct Mesh {
   size_t ws_doubles = 0;
   CgState *st = nullptr;       // device
   double *red = nullptr;       // device, partial sums
+  HostBox *box = nullptr;      // the solves' reports to the host, and their count
+  unsigned long long box_seq = 0;
+  BoxRef next_report() { return BoxRef{box, box ? ++box_seq : 0}; }
   Mg *mg = nullptr;            // H1 multigrid hierarchy (nkh_mg_setup)
   // FP32 copies of g and bm1 for the single-precision operator (built on
   // first use, rebuilt when geom_version moves)

@@ -393,7 +393,8 @@ class Batch:
 
     def hmholtz(self, solves, maxit, params=None):
         """solves: list of dicts u, rhs, h1, h2, mask, mult, tli (tensors on
-        the GPU).  Returns (list of result dicts, graph launches)."""
+        the GPU).  Returns (list of result dicts, iterations enqueued for the
+        slowest solve)."""
         nb = len(self.fields)
         assert len(solves) == nb
         arr = (_lib.NkhBatchSolve * nb)()
