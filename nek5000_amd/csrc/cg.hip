@@ -5,12 +5,13 @@
 //     z = r*d ; rtz1 = (z,r)_mult ; rbn2 = sqrt((r,r)_{binv*mult}/vol)
 //     exit test ; beta ; p = z + beta p ; w = A p ; dssum(w) ; w *= mask
 //     rho = (w,p)_mult ; alpha ; x += alpha p ; r -= alpha w
-// runs as five launches:
-//     k_cg_update_dots : x/r update of the previous iteration + both dots
-//     k_cg_scalars1    : one block: sums the dot partials, exit test, beta
+// runs as three launches:
+//     k_cg_update_dots : x/r update of the previous iteration + both dots;
+//                        in its last block the exit test and beta
 //     axhelm (MODE 1)  : p update fused in, w = A_L p, rho = sum p.w
-//     gs_assemble      : w <- mask * dssum(w)
-//     k_cg_scalars2    : one block: rho, alpha
+//     gs_assemble_step : w <- mask * dssum(w); in a block of its own alpha
+// (With the two scalar steps as kernels of their own 336 elements, lx1 8, took
+// 420 us a solve, now 347; 9e6 nodes 7250, now 7180.)
 // rho is taken before the assembly: with p continuous and zero where the
 // mask is, and mult summing to one over each group of shared nodes,
 // (mask*QQ^T w, p)_mult = sum_l p_l w_l exactly in exact arithmetic.  The
@@ -23,6 +24,7 @@
 #include <vector>
 
 #include "nekamd_internal.h"
+#include "tails.h"
 
 namespace nekamd {
 
@@ -52,10 +54,14 @@ __device__ __forceinline__ void block_store2(double a, double b, double *pa, dou
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    pa[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
-    pb[blockIdx.x] = ((sbb[0] + sbb[1]) + sbb[2]) + sbb[3];
+    leave(pa + blockIdx.x, ((sa[0] + sa[1]) + sa[2]) + sa[3]);
+    leave(pb + blockIdx.x, ((sbb[0] + sbb[1]) + sbb[2]) + sbb[3]);
   }
 }
+
+// last_block's counters of a solve
+static_assert(kCounterDoubles <= kRedBlocks, "their place in red");
+inline int *counters(double *red) { return reinterpret_cast<int *>(red + kRedCount); }
 
 // Grid of the update-and-dots kernels: about 2048 nodes per block, at most
 // kUpdBlocks -- a launch costs about 10 ns per block, which dominates small
@@ -227,8 +233,12 @@ __global__ void __launch_bounds__(256)
               double *__restrict__ d, const double *__restrict__ mult,
               const double *__restrict__ binv, double *__restrict__ dm,
               double *__restrict__ bm, int plain_norm, int64_t n, double *__restrict__ part1,
-              double *__restrict__ part2, CgState init, CgState *__restrict__ st) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *st = init;
+              double *__restrict__ part2, CgState init, CgState *__restrict__ st,
+              int *__restrict__ cnt) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) *st = init;
+    clear_counters(cnt);
+  }
   double s1 = 0.0, s2 = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -246,16 +256,53 @@ __global__ void __launch_bounds__(256)
   block_store2(s1, s2, part1, part2);
 }
 
+// the state to the host (a solve that is done changes it no more)
+__device__ __forceinline__ void state_report(const CgState *st, const BoxRef &rep) {
+  if (!rep.b) return;
+  *reinterpret_cast<CgState *>(rep.b->v) = *st;
+  box_report(rep);
+}
+static_assert(sizeof(CgState) <= sizeof(HostBox::v), "a report holds a state");
+
+__device__ void cg_scalars1(CgState *st, double s1, double s2, double *hist) {
+  const int iter = st->iter + 1;
+  st->iter = iter;
+  if (iter > st->maxit) {  // loop exhausted (hmholtz.f:817: niter = iter-1)
+    st->done = 1;
+    st->niter = st->maxit;
+    return;
+  }
+  st->rtz2 = st->rtz1;
+  st->rtz1 = s1;
+  const double rbn2 = sqrt(s2 / st->vol);
+  st->rbn2 = rbn2;
+  if (iter == 1) st->rbn0 = rbn2;
+  if (st->param22 < 0) st->tol = fabs(st->param22) * st->rbn0;
+  if (st->tin < 0) st->tol = fabs(st->tin) * st->rbn0;
+  if (hist) {
+    hist[5 * (iter - 1) + 0] = rbn2;
+    hist[5 * (iter - 1) + 1] = s1;
+  }
+  if (rbn2 <= st->tol && (iter > 1 || st->istep <= 5)) {
+    st->done = 1;
+    st->converged = 1;
+    st->niter = iter - 1;
+    return;
+  }
+  st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
+}
+
 // x += alpha p ; r -= alpha w (the update of the previous iteration) ; partial
 // sums of (d*r)*r*mult and binv*mult*r*r (vlsc3 / vlsc32, hmholtz.f:754-759).
-// VEC: 16-byte loads of node pairs (all six arrays 16-byte aligned).
+// VEC: 16-byte loads of node pairs (all six arrays 16-byte aligned).  The last
+// block makes the iteration's exit test and beta and reports to the host.
 template <bool VEC>
 __global__ void __launch_bounds__(256)
     k_cg_update_dots(double *__restrict__ x, double *__restrict__ r,
                      const double *__restrict__ p, const double *__restrict__ w,
                      const double *__restrict__ dm, const double *__restrict__ bm, int64_t n,
-                     const CgState *__restrict__ st, double *__restrict__ part1,
-                     double *__restrict__ part2) {
+                     CgState *st, double *part1, double *part2, int *cnt, double *hist,
+                     BoxRef rep) {
   if (st->done) return;
   const double alpha = st->alpha;
   double s1 = 0.0, s2 = 0.0;
@@ -300,78 +347,36 @@ __global__ void __launch_bounds__(256)
     s2 += bm[i] * rr;
   }
   block_store2(s1, s2, part1, part2);
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[2];
+  sum_left(part1, part2 - part1, gridDim.x, t);
+  if (threadIdx.x != 0) return;
+  cg_scalars1(st, t[0], t[1], hist);
+  state_report(st, rep);
 }
 
-// the state to the host (a solve that is done changes it no more)
-__device__ __forceinline__ void state_report(const CgState *st, const BoxRef &rep) {
-  if (!rep.b) return;
-  *reinterpret_cast<CgState *>(rep.b->v) = *st;
-  box_report(rep);
-}
-static_assert(sizeof(CgState) <= sizeof(HostBox::v), "a report holds a state");
-
-__device__ void cg_scalars1(CgState *st, double s1, double s2, double *hist) {
-  st->pending = 0;
-  const int iter = st->iter + 1;
-  st->iter = iter;
-  if (iter > st->maxit) {  // loop exhausted (hmholtz.f:817: niter = iter-1)
-    st->done = 1;
-    st->niter = st->maxit;
-    return;
-  }
-  st->rtz2 = st->rtz1;
-  st->rtz1 = s1;
-  const double rbn2 = sqrt(s2 / st->vol);
-  st->rbn2 = rbn2;
-  if (iter == 1) st->rbn0 = rbn2;
-  if (st->param22 < 0) st->tol = fabs(st->param22) * st->rbn0;
-  if (st->tin < 0) st->tol = fabs(st->tin) * st->rbn0;
-  if (hist) {
-    hist[5 * (iter - 1) + 0] = rbn2;
-    hist[5 * (iter - 1) + 1] = s1;
-  }
-  if (rbn2 <= st->tol && (iter > 1 || st->istep <= 5)) {
-    st->done = 1;
-    st->converged = 1;
-    st->niter = iter - 1;
-    return;
-  }
-  st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
-}
-
+// the first iteration's, after k_cg_init
 __global__ void __launch_bounds__(kScalThreads)
     k_cg_scalars1(CgState *__restrict__ st, const double *__restrict__ part1,
                   const double *__restrict__ part2, int nparts, double *__restrict__ hist,
                   BoxRef rep) {
   if (st->done) return;
-  const double s1 = block_sum_array(part1, nparts);
-  const double s2 = block_sum_array(part2, nparts);
+  double t[2];
+  sum_left(part1, part2 - part1, nparts, t);
   if (threadIdx.x != 0) return;
-  cg_scalars1(st, s1, s2, hist);
+  cg_scalars1(st, t[0], t[1], hist);
   state_report(st, rep);
 }
 
+// rho and alpha (the general path; the fused one has them in the assembly)
 __global__ void __launch_bounds__(kScalThreads)
-    k_cg_scalars2(CgState *__restrict__ st, const double *__restrict__ rp1, int n1,
-                  const double *__restrict__ rp2, int n2, double *__restrict__ hist,
-                  BoxRef rep) {
-  if (st->done) {  // the solve's last kernel
-    if (threadIdx.x == 0) box_report(rep);
-    return;
-  }
-  const double a = block_sum_array(rp1, n1);
-  const double b = (n2 > 0) ? block_sum_array(rp2, n2) : 0.0;
-  if (threadIdx.x != 0) return;
-  const double rho = a + b;
-  st->rho = rho;
-  st->alpha = st->rtz1 / rho;
-  st->pending = 1;
-  if (hist) {
-    const int it = st->iter;
-    hist[5 * (it - 1) + 2] = rho;
-    hist[5 * (it - 1) + 3] = st->alpha;
-    hist[5 * (it - 1) + 4] = st->beta;
-  }
+    k_cg_scalars2(CgState *__restrict__ st, StepLength step, BoxRef last) {
+  if (!st->done) step_length(step);
+  else if (threadIdx.x == 0) box_report(last);  // the solve's last kernel
+}
+// rho = the count partials of the operator, alpha = rtz1 / rho
+inline StepLength step_of(CgState *st, const double *part, int count, double *hist) {
+  return StepLength{part, count, &st->rtz1, &st->rho, &st->alpha, hist, &st->beta, &st->iter};
 }
 
 // rho over all nodes (used when ids are not zero exactly at interiors):
@@ -439,14 +444,54 @@ inline int refresh_blocks(int64_t n) {
   return (int)(b < 64 ? 64 : (b > kRefreshBlocks ? kRefreshBlocks : b));
 }
 
-// xs += alpha p ; r -= alpha w (FP32) ; FP64 partials of dm*r*r and bm*r*r
+// as cg_scalars1, but a refresh of the residual is requested instead of
+// ending the solve or when the iterated residual fell by kRefresh
+__device__ void mcg_scalars1(McgState *ms, double s1, double s2, double *hist) {
+  CgState *st = &ms->cg;
+  const int iter = st->iter + 1;
+  st->iter = iter;
+  if (iter > st->maxit) {  // loop exhausted: fold the correction into x
+    ms->final = 2;
+    ms->gate.done = 0;
+    return;
+  }
+  st->rtz2 = st->rtz1;
+  st->rtz1 = s1;
+  const double rbn2 = sqrt(s2 / st->vol);
+  st->rbn2 = rbn2;
+  if (iter == 1) {
+    st->rbn0 = rbn2;
+    ms->rmax = rbn2;
+  }
+  if (st->param22 < 0) st->tol = fabs(st->param22) * st->rbn0;
+  if (st->tin < 0) st->tol = fabs(st->tin) * st->rbn0;
+  if (hist) {
+    hist[5 * (iter - 1) + 0] = rbn2;
+    hist[5 * (iter - 1) + 1] = s1;
+  }
+  if (rbn2 <= st->tol && (iter > 1 || st->istep <= 5)) {
+    ms->final = 1;
+    ms->gate.done = 0;
+    return;
+  }
+  if (rbn2 < kRefresh * ms->rmax) {
+    ms->final = 0;
+    ms->gate.done = 0;
+    return;
+  }
+  if (rbn2 > ms->rmax) ms->rmax = rbn2;
+  st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
+}
+
+// xs += alpha p ; r -= alpha w (FP32) ; FP64 partials of dm*r*r and bm*r*r;
+// the iteration's tests in the last block
 template <bool VEC>
 __global__ void __launch_bounds__(256)
     k_mcg_update_dots(float *__restrict__ xs, float *__restrict__ r,
                       const float *__restrict__ p, const float *__restrict__ w,
                       const float *__restrict__ dm, const float *__restrict__ bm, int64_t n,
-                      const CgState *__restrict__ st, double *__restrict__ part1,
-                      double *__restrict__ part2) {
+                      McgState *ms, double *part1, double *part2, int *cnt, double *hist) {
+  CgState *st = &ms->cg;
   if (st->done) return;
   const float alpha = (float)st->alpha;
   double s1 = 0.0, s2 = 0.0;
@@ -493,51 +538,21 @@ __global__ void __launch_bounds__(256)
     s2 += bm[i] * q;
   }
   block_store2(s1, s2, part1, part2);
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[2];
+  sum_left(part1, part2 - part1, gridDim.x, t);
+  if (threadIdx.x != 0) return;
+  mcg_scalars1(ms, t[0], t[1], hist);
 }
 
-// as k_cg_scalars1, but a refresh of the residual is requested instead of
-// ending the solve or when the iterated residual fell by kRefresh
+// the first iteration's, after k_mcg_init
 __global__ void __launch_bounds__(kScalThreads)
     k_mcg_scalars1(McgState *__restrict__ ms, const double *__restrict__ part1,
                    const double *__restrict__ part2, int nparts, double *__restrict__ hist) {
-  CgState *st = &ms->cg;
-  if (st->done) return;
-  const double s1 = block_sum_array(part1, nparts);
-  const double s2 = block_sum_array(part2, nparts);
-  if (threadIdx.x != 0) return;
-  const int iter = st->iter + 1;
-  st->iter = iter;
-  if (iter > st->maxit) {  // loop exhausted: fold the correction into x
-    ms->final = 2;
-    ms->gate.done = 0;
-    return;
-  }
-  st->rtz2 = st->rtz1;
-  st->rtz1 = s1;
-  const double rbn2 = sqrt(s2 / st->vol);
-  st->rbn2 = rbn2;
-  if (iter == 1) {
-    st->rbn0 = rbn2;
-    ms->rmax = rbn2;
-  }
-  if (st->param22 < 0) st->tol = fabs(st->param22) * st->rbn0;
-  if (st->tin < 0) st->tol = fabs(st->tin) * st->rbn0;
-  if (hist) {
-    hist[5 * (iter - 1) + 0] = rbn2;
-    hist[5 * (iter - 1) + 1] = s1;
-  }
-  if (rbn2 <= st->tol && (iter > 1 || st->istep <= 5)) {
-    ms->final = 1;
-    ms->gate.done = 0;
-    return;
-  }
-  if (rbn2 < kRefresh * ms->rmax) {
-    ms->final = 0;
-    ms->gate.done = 0;
-    return;
-  }
-  if (rbn2 > ms->rmax) ms->rmax = rbn2;
-  st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
+  if (ms->cg.done) return;
+  double t[2];
+  sum_left(part1, part2 - part1, nparts, t);
+  if (threadIdx.x == 0) mcg_scalars1(ms, t[0], t[1], hist);
 }
 
 // refresh, part 1: x += xs (FP64), xs = 0
@@ -549,26 +564,6 @@ __global__ void k_mcg_fold(double *__restrict__ x, float *__restrict__ xs, int64
     x[i] = x[i] + (double)xs[i];
     xs[i] = 0.0f;
   }
-}
-
-// refresh, part 2 (after ax = mask*QQ^T A_L x): r = f - ax in FP64, stored
-// rounded; partials of dm*r32^2 (the iteration's rtz) and bm*r^2 (FP64 norm)
-__global__ void __launch_bounds__(256)
-    k_mcg_resid(float *__restrict__ r32, const double *__restrict__ f,
-                const double *__restrict__ ax, const float *__restrict__ dm,
-                const float *__restrict__ bm, int64_t n, const CgState *__restrict__ gate,
-                double *__restrict__ part1, double *__restrict__ part2) {
-  if (gate->done) return;
-  double s1 = 0.0, s2 = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double ri = f[i] - ax[i];
-    const float rf = (float)ri;
-    r32[i] = rf;
-    s1 += dm[i] * ((double)rf * rf);
-    s2 += bm[i] * (ri * ri);
-  }
-  block_store2(s1, s2, part1, part2);
 }
 
 // refresh, part 3: the true residual's norm decides the exit; otherwise the
@@ -601,19 +596,34 @@ __device__ void mcg_scalars1b(McgState *ms, double s1, double s2, double *hist) 
   st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
 }
 
-// (reports the state whether a refresh ran or not)
-__global__ void __launch_bounds__(kScalThreads)
-    k_mcg_scalars1b(McgState *__restrict__ ms, const double *__restrict__ part1,
-                    const double *__restrict__ part2, int nparts, double *__restrict__ hist,
-                    BoxRef rep) {
+// refresh, part 2 (after ax = mask*QQ^T A_L x): r = f - ax in FP64, stored
+// rounded; partials of dm*r32^2 (the iteration's rtz) and bm*r^2 (FP64 norm);
+// part 3 in the last block.  The state is reported whether a refresh runs or
+// not.
+__global__ void __launch_bounds__(256)
+    k_mcg_resid(float *__restrict__ r32, const double *__restrict__ f,
+                const double *__restrict__ ax, const float *__restrict__ dm,
+                const float *__restrict__ bm, int64_t n, McgState *ms, double *part1,
+                double *part2, int *cnt, double *hist, BoxRef rep) {
   if (ms->gate.done) {
-    if (threadIdx.x == 0) state_report(&ms->cg, rep);
+    if (blockIdx.x == 0 && threadIdx.x == 0) state_report(&ms->cg, rep);
     return;
   }
-  const double s1 = block_sum_array(part1, nparts);
-  const double s2 = block_sum_array(part2, nparts);
+  double s1 = 0.0, s2 = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const double ri = f[i] - ax[i];
+    const float rf = (float)ri;
+    r32[i] = rf;
+    s1 += dm[i] * ((double)rf * rf);
+    s2 += bm[i] * (ri * ri);
+  }
+  block_store2(s1, s2, part1, part2);
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[2];
+  sum_left(part1, part2 - part1, gridDim.x, t);
   if (threadIdx.x != 0) return;
-  mcg_scalars1b(ms, s1, s2, hist);
+  mcg_scalars1b(ms, t[0], t[1], hist);
   state_report(&ms->cg, rep);
 }
 
@@ -626,8 +636,11 @@ __global__ void __launch_bounds__(256)
                const double *__restrict__ f, const double *__restrict__ d,
                const double *__restrict__ mult, const double *__restrict__ binv, int plain_norm,
                int64_t n, double *__restrict__ part1, double *__restrict__ part2, McgState init,
-               McgState *__restrict__ ms) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *ms = init;
+               McgState *__restrict__ ms, int *__restrict__ cnt) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) *ms = init;
+    clear_counters(cnt);
+  }
   double s1 = 0.0, s2 = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -715,7 +728,7 @@ int ensure_workspace(Mesh &m) {
 static int enqueue_facts(Mesh &m, const double *h1, const double *h2, const double *mask,
                          const double *mult, double *f, const FactsAsk &ask, double *red,
                          uint8_t *flag, const BoxRef &rep, hipStream_t s) {
-  static_assert(kNF * kRedBlocks <= kRedRho2, "the partial sums take the dots' place");
+  static_assert(kNF * kRedBlocks <= kRedCount, "the partial sums take the dots' place");
   double *part = red + kRedPart1, *res = red + kRedOut;
   int *left = reinterpret_cast<int *>(res + kNF + 1);
   const int64_t per = 1024;  // nodes per block, up to the fixed grid
@@ -895,7 +908,7 @@ struct CgRun {
     h.param18 = prm.param18;
     hipLaunchKernelGGL(k_cg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, r, f, d, mult,
                        mesh.binv, dm, bm, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
-                       red + kRedPart2, h, st);
+                       red + kRedPart2, h, st, counters(red));
     NK_HIP(hipGetLastError());
     // Fused iteration (rho inside axhelm, mask inside the assembly) when its
     // conditions hold and f is zero where masked.
@@ -918,31 +931,31 @@ struct CgRun {
   // and the assembly
   int enqueue(hipStream_t s, hipEvent_t *ev = nullptr) {
     const int64_t n = m->n;
-    double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1,
-           *rho2 = red + kRedRho2;
+    double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1;
     const int ub = upd_blocks(n);
-    if (launched > 0)  // (the first iteration's sums come from k_cg_init)
-      hipLaunchKernelGGL((vec_ok ? k_cg_update_dots<true> : k_cg_update_dots<false>), dim3(ub),
-                         dim3(256), 0, s, x, r, p, w, dm, bm, n, st, part1, part2);
     last = BoxRef{box, last.seq + 2};
-    hipLaunchKernelGGL(k_cg_scalars1, dim3(1), dim3(kScalThreads), 0, s, st, part1, part2, ub,
-                       hist, exit_test());
+    if (launched > 0)
+      hipLaunchKernelGGL((vec_ok ? k_cg_update_dots<true> : k_cg_update_dots<false>), dim3(ub),
+                         dim3(256), 0, s, x, r, p, w, dm, bm, n, st, part1, part2,
+                         counters(red), hist, exit_test());
+    else  // (the first iteration's sums come from k_cg_init)
+      hipLaunchKernelGGL(k_cg_scalars1, dim3(1), dim3(kScalThreads), 0, s, st, part1, part2, ub,
+                         hist, exit_test());
     if (fused) {
       if (ev) NK_HIP(hipEventRecord(ev[0], s));
       NK_TRY(launch_axhelm_cg(*m, w, p, r, d, h1, h2, mult, st, rho1, s));
       if (ev) NK_HIP(hipEventRecord(ev[1], s));
-      NK_TRY(gs_assemble(m->gs, w, st, s, flag));
+      NK_TRY(gs_assemble_step(m->gs, w, st, s, flag, step_of(st, rho1, ax_grid_parts, hist),
+                              last));
       if (ev) NK_HIP(hipEventRecord(ev[2], s));
-      hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st, rho1,
-                         ax_grid_parts, rho2, 0, hist, last);
     } else {
       NK_TRY(launch_axhelm_cg(*m, w, p, r, d, h1, h2, mult, st, nullptr, s));
       NK_TRY(gs_op(m->gs, w, 0, s));
       hipLaunchKernelGGL(k_mask_guarded, dim3(grid_for(n)), dim3(256), 0, s, w, mask, n, st);
       hipLaunchKernelGGL(k_dot3_guarded, dim3(kRedBlocks), dim3(256), 0, s, w, p, mult, n, st,
                          rho1);
-      hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st, rho1, kRedBlocks,
-                         rho2, 0, hist, last);
+      hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st,
+                         step_of(st, rho1, kRedBlocks, hist), last);
     }
     NK_HIP(hipGetLastError());
     ++launched;
@@ -1046,7 +1059,7 @@ struct McgRun {
     h.gate.done = 1;
     hipLaunchKernelGGL(k_mcg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, r, d, dm, bm, f,
                        ax, mult, mesh.binv, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
-                       red + kRedPart2, h, ms);
+                       red + kRedPart2, h, ms, counters(red));
     NK_HIP(hipGetLastError());
     NK_TRY(ensure_geom32(mesh, s));
     ax_grid_parts = axhelm_cg_grid(mesh);
@@ -1064,32 +1077,30 @@ struct McgRun {
 
   int enqueue(hipStream_t s, hipEvent_t *ev = nullptr) {
     const int64_t n = m->n;
-    double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1,
-           *rho2 = red + kRedRho2;
+    double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1;
     const int ub = upd_blocks(n);
-    if (launched > 0)  // (the first iteration's sums come from k_mcg_init)
+    if (launched > 0)
       hipLaunchKernelGGL((vec_ok ? k_mcg_update_dots<true> : k_mcg_update_dots<false>), dim3(ub),
-                         dim3(256), 0, s, xs, r, p, w, dm, bm, n, st, part1, part2);
-    hipLaunchKernelGGL(k_mcg_scalars1, dim3(1), dim3(kScalThreads), 0, s, ms, part1, part2, ub,
-                       hist);
+                         dim3(256), 0, s, xs, r, p, w, dm, bm, n, ms, part1, part2,
+                         counters(red), hist);
+    else  // (the first iteration's sums come from k_mcg_init)
+      hipLaunchKernelGGL(k_mcg_scalars1, dim3(1), dim3(kScalThreads), 0, s, ms, part1, part2, ub,
+                         hist);
     // the refresh (its kernels return at once while the gate is closed)
     const CgState *gate = &ms->gate;
     const int rb = refresh_blocks(n);
     hipLaunchKernelGGL(k_mcg_fold, dim3(rb), dim3(256), 0, s, x, xs, n, gate);
     NK_TRY(launch_axhelm_gated(*m, ax, x, h1, h2, gate, s));
     NK_TRY(gs_assemble(m->gs, ax, gate, s, flag, rb));
-    hipLaunchKernelGGL(k_mcg_resid, dim3(rb), dim3(256), 0, s, r, f, ax, dm, bm, n, gate, part1,
-                       part2);
     last = BoxRef{box, last.seq + 2};
-    hipLaunchKernelGGL(k_mcg_scalars1b, dim3(1), dim3(kScalThreads), 0, s, ms, part1, part2, rb,
-                       hist, exit_test());
+    hipLaunchKernelGGL(k_mcg_resid, dim3(rb), dim3(256), 0, s, r, f, ax, dm, bm, n, ms, part1,
+                       part2, counters(red), hist, exit_test());
     if (ev) NK_HIP(hipEventRecord(ev[0], s));
     NK_TRY(launch_axhelm32_jac(*m, w, p, r, d, (float)h1.s, (float)h2.s, st, rho1, s));
     if (ev) NK_HIP(hipEventRecord(ev[1], s));
-    NK_TRY(gs_assemble(m->gs, w, st, s, flag));
+    NK_TRY(gs_assemble_step(m->gs, w, st, s, flag, step_of(st, rho1, ax_grid_parts, hist),
+                            last));
     if (ev) NK_HIP(hipEventRecord(ev[2], s));
-    hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st, rho1,
-                       ax_grid_parts, rho2, 0, hist, last);
     NK_HIP(hipGetLastError());
     ++launched;
     return NKH_OK;

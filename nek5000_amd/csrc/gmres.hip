@@ -11,99 +11,153 @@
 #include <vector>
 
 #include "hsmg.h"
+#include "tails.h"
 
 namespace nekamd {
 
 namespace {
 
-constexpr int kGmBlocks = 2048;
+constexpr int kGmBlocks = 2048;  // room for the partials of one sum (dot_blocks)
 constexpr int kDotChunk = 8;
+// last_block's counters: a set for each chunk of products, one for the norms
+constexpr int kCounters = (kGmresM + kDotChunk - 1) / kDotChunk + 1;
+constexpr int kCounterInts = 2 * kCounterDoubles;
 
 #define NK_LOOP(i, n)                                                          \
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < (n); \
        i += (int64_t)gridDim.x * blockDim.x)
 
-__device__ __forceinline__ void store_part(double a, double *part) {
+// *out = the sum over the grid of a, and in the last block that and the nh
+// doubles h before it to the host
+__device__ __forceinline__ void norm_and_report(double a, double *part, int *cnt, double *out,
+                                                const double *h, int nh, const BoxRef &rep) {
   __shared__ double sa[4];
   for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
   if ((threadIdx.x & 63) == 0) sa[threadIdx.x >> 6] = a;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
-  __syncthreads();
+  if (threadIdx.x == 0) leave(part + blockIdx.x, ((sa[0] + sa[1]) + sa[2]) + sa[3]);
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[1];
+  sum_left(part, 0, gridDim.x, t);
+  if (threadIdx.x != 0) return;
+  *out = t[0];
+  for (int i = 0; i < nh; ++i) rep.b->v[i] = h[i];
+  rep.b->v[nh] = t[0];
+  box_report(rep);
 }
+static_assert(kGmresM + 1 <= (int)(sizeof(HostBox::v) / sizeof(double)), "a report holds a step");
 
-// r = res - mask*w; partial sum r*r*wt   (r = res - A x with ax's mask)
+// r = res - mask*w; *a2 = sum r*r*wt, reported   (r = res - A x with ax's mask)
 __global__ void __launch_bounds__(256)
     k_gm_resid(double *__restrict__ r, const double *__restrict__ res,
                const double *__restrict__ w, const double *__restrict__ mask,
-               const double *__restrict__ wt, int64_t n, int first, double *part) {
+               const double *__restrict__ wt, int64_t n, int first, double *part, int *cnt,
+               double *a2, BoxRef rep) {
   double a = 0.0;
   NK_LOOP(i, n) {
     const double ri = first ? res[i] : res[i] - w[i] * mask[i];
     r[i] = ri;
     a += (ri * ri) * wt[i];
   }
-  store_part(a, part);
+  norm_and_report(a, part, cnt, a2, nullptr, 0, rep);
 }
 
-// w *= mask (ax's pmask), then partial sums of (w*v_i)*wt for i in
-// [i0, i0+cnt) (vlsc3, gmres.f:466)
-__global__ void __launch_bounds__(256)
-    k_gm_dots(double *__restrict__ w, const double *__restrict__ mask, int apply_mask,
-              const double *__restrict__ V, int64_t n, int i0, int cnt,
-              const double *__restrict__ wt, double *part) {
-  double acc[kDotChunk];
-#pragma unroll
-  for (int c = 0; c < kDotChunk; ++c) acc[c] = 0.0;
+// h_c = sum (mask*w v_c)*wt for the C vectors v at V (vlsc3, gmres.f:466)
+template <int C>
+__device__ __forceinline__ void gm_dots(const double *__restrict__ w,
+                                        const double *__restrict__ mask,
+                                        const double *__restrict__ V, int64_t n,
+                                        const double *__restrict__ wt, double *part, int *cnt,
+                                        double *h, double (*sw)[4]) {
+  double acc[C] = {};
   NK_LOOP(q, n) {
-    double wq = w[q];
-    if (apply_mask) {
-      wq = wq * mask[q];
-      w[q] = wq;
-    }
-    const double wv = wt[q];
+    double v[C];
 #pragma unroll
-    for (int c = 0; c < kDotChunk; ++c)
-      if (c < cnt) acc[c] += (wq * V[(int64_t)(i0 + c) * n + q]) * wv;
+    for (int c = 0; c < C; ++c) v[c] = V[(int64_t)c * n + q];
+    const double wq = w[q] * mask[q], wv = wt[q];
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] += (wq * v[c]) * wv;
   }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
-  for (int c = 0; c < kDotChunk; ++c)
-    if (c < cnt) store_part(acc[c], part + (int64_t)(i0 + c) * kGmBlocks);
-}
-
-// out[i] = fixed-order sum of the kGmBlocks partials of dot i (block i); with
-// a report (one block), that sum and the nh doubles h before it
-__global__ void __launch_bounds__(256)
-    k_gm_final(const double *part, double *out, const double *h, int nh, BoxRef rep) {
-  __shared__ double sa[4];
-  const double *p = part + (int64_t)blockIdx.x * kGmBlocks;
-  double a = 0.0;
-  for (int q = threadIdx.x; q < kGmBlocks; q += blockDim.x) a += p[q];
-  for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-  if ((threadIdx.x & 63) == 0) sa[threadIdx.x >> 6] = a;
+  for (int c = 0; c < C; ++c) {
+    double a = acc[c];
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
+    if (lane == 0) sw[c][wave] = a;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
-  if (rep.b && threadIdx.x == 0) {
-    for (int i = 0; i < nh; ++i) rep.b->v[i] = h[i];
-    rep.b->v[nh] = out[blockIdx.x];
-    box_report(rep);
+  const int t = threadIdx.x;
+  if (t < C)
+    leave(part + (int64_t)t * kGmBlocks + blockIdx.x, ((sw[t][0] + sw[t][1]) + sw[t][2]) + sw[t][3]);
+  if (!last_block(cnt, gridDim.x)) return;
+  for (int c = wave; c < C; c += 4) {
+    const double *p = part + (int64_t)c * kGmBlocks;
+    double b[4] = {};
+    int q = lane;
+    for (; q + 192 < (int)gridDim.x; q += 256) {
+      double l[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) l[u] = left(p + q + 64 * u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) b[u] += l[u];
+    }
+    for (; q < (int)gridDim.x; q += 64) b[0] += left(p + q);
+    double a = (b[0] + b[1]) + (b[2] + b[3]);
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
+    if (lane == 0) h[c] = a;
   }
 }
-static_assert(kGmresM + 1 <= (int)(sizeof(HostBox::v) / sizeof(double)), "a report holds a step");
 
-// w = w - h_i v_i for i = 0..j-1 in order (add2s2), then partial w*w*wt
+// Chunk blockIdx.y of the j products, kDotChunk of them a chunk (each reads w,
+// mask and wt once); cnt: a set of counters a chunk.  The last block of a chunk adds
+// up its products, a wavefront each.
 __global__ void __launch_bounds__(256)
-    k_gm_orth(double *__restrict__ w, const double *__restrict__ V,
-              const double *__restrict__ h, int j, const double *__restrict__ wt, int64_t n,
-              double *part) {
+    k_gm_dots(const double *__restrict__ w, const double *__restrict__ mask,
+              const double *__restrict__ V, int64_t n, int j, const double *__restrict__ wt,
+              double *part, int *cnt, double *h) {
+  __shared__ double sw[kDotChunk][4];
+  const int i0 = blockIdx.y * kDotChunk;
+  V += (int64_t)i0 * n;
+  part += (int64_t)i0 * kGmBlocks;
+  h += i0;
+  cnt += blockIdx.y * kCounterInts;
+  switch (j - i0) {
+    case 1: return gm_dots<1>(w, mask, V, n, wt, part, cnt, h, sw);
+    case 2: return gm_dots<2>(w, mask, V, n, wt, part, cnt, h, sw);
+    case 3: return gm_dots<3>(w, mask, V, n, wt, part, cnt, h, sw);
+    case 4: return gm_dots<4>(w, mask, V, n, wt, part, cnt, h, sw);
+    case 5: return gm_dots<5>(w, mask, V, n, wt, part, cnt, h, sw);
+    case 6: return gm_dots<6>(w, mask, V, n, wt, part, cnt, h, sw);
+    case 7: return gm_dots<7>(w, mask, V, n, wt, part, cnt, h, sw);
+    default: return gm_dots<8>(w, mask, V, n, wt, part, cnt, h, sw);
+  }
+}
+static_assert(kDotChunk == 8, "the cases of k_gm_dots");
+
+// w = mask*w - h_i v_i for i = 0..j-1 in order (add2s2), then *a2 = sum w*w*wt,
+// reported with h
+__global__ void __launch_bounds__(256)
+    k_gm_orth(double *__restrict__ w, const double *__restrict__ mask,
+              const double *__restrict__ V, const double *__restrict__ h, int j,
+              const double *__restrict__ wt, int64_t n, double *part, int *cnt, double *a2,
+              BoxRef rep) {
   double a = 0.0;
   NK_LOOP(q, n) {
-    double wq = w[q];
-    for (int i = 0; i < j; ++i) wq = wq + (-h[i]) * V[(int64_t)i * n + q];
+    double wq = w[q] * mask[q];
+    const double wv = wt[q];
+    int i = 0;
+    for (; i + 4 <= j; i += 4) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = V[(int64_t)(i + u) * n + q];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) wq = wq + (-h[i + u]) * v[u];
+    }
+    for (; i < j; ++i) wq = wq + (-h[i]) * V[(int64_t)i * n + q];
     w[q] = wq;
-    a += (wq * wq) * wt[q];
+    a += (wq * wq) * wv;
   }
-  store_part(a, part);
+  norm_and_report(a, part, cnt, a2, h, j, rep);
 }
 
 // v = u / sqrt(*a2) (cmult2: the next Krylov vector), w = v * mgmask (the
@@ -133,7 +187,10 @@ __global__ void k_gm_xupd(double *__restrict__ x, const double *__restrict__ Z, 
   }
 }
 
-__global__ void k_gm_zero(double *__restrict__ x, int64_t n) {
+// x = 0, and the counters of the kernels that end in last_block
+__global__ void k_gm_zero(double *__restrict__ x, int64_t n, int *__restrict__ cnt) {
+  if (blockIdx.x == 0)
+    for (int k = 0; k < kCounters; ++k) clear_counters(cnt + k * kCounterInts);
   NK_LOOP(i, n) x[i] = 0.0;
 }
 
@@ -155,13 +212,16 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
     NK_TRY(mg_dalloc(&mg.gZ, (int64_t)M * n));
     for (double **p : {&mg.gx, &mg.gr, &mg.gw}) NK_TRY(mg_dalloc(p, n));
     NK_TRY(mg_dalloc(&mg.gpart, (int64_t)(M + 2) * kGmBlocks));
-    NK_TRY(mg_dalloc(&mg.gsm, 2 * (M + 2)));
+    NK_TRY(mg_dalloc(&mg.gsm, 2 * (M + 2) + kCounters * kCounterDoubles));
   }
   double *V = mg.gV, *Z = mg.gZ, *x = mg.gx, *r = mg.gr, *w = mg.gw, *part = mg.gpart;
-  double *dh = mg.gsm, *da2 = mg.gsm + (M + 2);  // h(1..j); the squared norm after them
+  // h(1..j), the squared norm after them, the counters
+  double *dh = mg.gsm, *da2 = mg.gsm + (M + 2);
+  int *cnt = reinterpret_cast<int *>(mg.gsm + 2 * (M + 2));
+  int *ncnt = cnt + (kCounters - 1) * kCounterInts;
   NK_TRY(ensure_small(m));
   const double *mgmask = mg.lev[mg.lmax].mask;
-  const dim3 G(kGmBlocks), B(256);
+  const dim3 G(dot_blocks(n)), B(256);
   const double norm_fac = 1.0 / std::sqrt(m.vol);
   const bool nullsp = mg_null_space_on(mg, h2);
   // hmholtz.f-style tolerance (gmres.f:352-356)
@@ -172,14 +232,7 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
   double tolpss = tolps;
   std::vector<double> H((size_t)M * M, 0.0), gam(M + 1, 0.0), c(M, 0.0), sn(M, 0.0);
   auto HH = [&](int i, int jj) -> double & { return H[(size_t)i + (size_t)M * jj]; };
-  // the squared norm's partials to *da2, and with the nh coefficients of dh
-  // to the host (wait by box_wait)
-  auto norm_report = [&](int nh) -> BoxRef {
-    const BoxRef rep = m.next_report();
-    hipLaunchKernelGGL(k_gm_final, dim3(1), B, 0, s, part, da2, dh, nh, rep);
-    return rep;
-  };
-  hipLaunchKernelGGL(k_gm_zero, dim3(mg_grid(n)), B, 0, s, x, n);
+  hipLaunchKernelGGL(k_gm_zero, dim3(mg_grid(n)), B, 0, s, x, n, cnt);
   double div0 = 0.0, rnorm = 0.0;
   int iter = 0, j = 0;
   bool iconv = false;
@@ -189,8 +242,9 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
       NK_TRY(launch_axhelm(m, w, x, h1, h2, s));
       NK_TRY(gs_op(m.gs, w, 0, s));
     }
-    hipLaunchKernelGGL(k_gm_resid, G, B, 0, s, r, res, w, mask, wt, n, iter == 0 ? 1 : 0, part);
-    const BoxRef rep0 = norm_report(0);
+    const BoxRef rep0 = m.next_report();
+    hipLaunchKernelGGL(k_gm_resid, G, B, 0, s, r, res, w, mask, wt, n, iter == 0 ? 1 : 0, part,
+                       ncnt, da2, rep0);
     hipLaunchKernelGGL(k_gm_next, dim3(mg_grid(n)), B, 0, s, V, w, r, da2, mgmask, n);
     NK_HIP(hipGetLastError());
     NK_TRY(box_wait(rep0, s));
@@ -209,14 +263,10 @@ int run_gmres(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
       NK_TRY(launch_axhelm(m, w, zj, h1, h2, s));
       NK_TRY(gs_op(m.gs, w, 0, s));
       // classical Gram-Schmidt, one pass (gmres.f:464-474)
-      for (int i0 = 0; i0 < j; i0 += kDotChunk) {
-        const int cnt = std::min(kDotChunk, j - i0);
-        hipLaunchKernelGGL(k_gm_dots, G, B, 0, s, w, mask, i0 == 0 ? 1 : 0, V, n, i0, cnt, wt,
-                           part);
-      }
-      hipLaunchKernelGGL(k_gm_final, dim3(j), B, 0, s, part, dh, nullptr, 0, BoxRef{});
-      hipLaunchKernelGGL(k_gm_orth, G, B, 0, s, w, V, dh, j, wt, n, part);
-      const BoxRef rep = norm_report(j);
+      hipLaunchKernelGGL(k_gm_dots, dim3(G.x, (j + kDotChunk - 1) / kDotChunk), B, 0, s, w, mask,
+                         V, n, j, wt, part, cnt, dh);
+      const BoxRef rep = m.next_report();
+      hipLaunchKernelGGL(k_gm_orth, G, B, 0, s, w, mask, V, dh, j, wt, n, part, ncnt, da2, rep);
       if (j < M)  // (not read if this step is the last)
         hipLaunchKernelGGL(k_gm_next, dim3(mg_grid(n)), B, 0, s, V + (int64_t)j * n, w, w, da2,
                            mgmask, n);

@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "nekamd_internal.h"
+#include "tails.h"
 
 namespace nekamd {
 
@@ -185,8 +186,9 @@ __device__ __forceinline__ double gs_combine(double a, double b) {
 // (workgroups are dealt to the 8 XCDs round-robin) take neighbouring
 // packets and share their L2 lines.  Wavefront-uniform (held in a scalar
 // register, so the packet's descriptors are scalar loads).
-__device__ __forceinline__ int pk_index() {
-  const int nb = gridDim.x, b = blockIdx.x;
+// The first `first` blocks (a multiple of 8) do other work.
+__device__ __forceinline__ int pk_index(int first = 0) {
+  const int nb = gridDim.x - first, b = blockIdx.x - first;
   const int lb = (b % 8) * (nb / 8) + b / 8;
   return __builtin_amdgcn_readfirstlane(lb * 4 + (int)(threadIdx.x >> 6));
 }
@@ -316,9 +318,17 @@ __global__ void __launch_bounds__(256)
     k_gs_assemble_pk(T *__restrict__ w, const int32_t *__restrict__ pk_m,
                      const int32_t *__restrict__ pk_g, const uint64_t *__restrict__ pk_head,
                      const int32_t *__restrict__ idx, const uint8_t *__restrict__ flag,
-                     int64_t npk, const CgState *__restrict__ st) {
-  if (st && st->done) return;
-  const int p = pk_index();
+                     int64_t npk, const CgState *__restrict__ st, int first, StepLength step,
+                     BoxRef last) {
+  const bool done = st && st->done;
+  if ((int)blockIdx.x < first) {  // block 0: the step length, or the end of the solve
+    if (blockIdx.x != 0) return;
+    if (!done) step_length(step);
+    else if (threadIdx.x == 0) box_report(last);
+    return;
+  }
+  if (done) return;
+  const int p = pk_index(first);
   if (p >= npk) return;
   const PkLane L = pk_lane(pk_m, pk_head, idx, p);
   const T v = L.act ? w[L.node] : T(0);
@@ -475,7 +485,8 @@ static int gs_assemble_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s
   const uint8_t *fl = flag ? flag : gs.flag;
   if (gs.npk > 0)
     hipLaunchKernelGGL(k_gs_assemble_pk<T>, dim3(pk_blocks(gs.npk)), dim3(256), 0, s, w,
-                       gs.pk_m, gs.pk_g, gs.pk_head, gs.idx, fl, gs.npk, st);
+                       gs.pk_m, gs.pk_g, gs.pk_head, gs.idx, fl, gs.npk, st, 0, StepLength{},
+                       BoxRef{});
   const int64_t nbig = gs.ngroups - gs.gpk;
   if (nbig > 0) {
     const int nb = nblocks > 0 ? nblocks : gs_blocks(nbig);
@@ -485,6 +496,43 @@ static int gs_assemble_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s
   }
   NK_HIP(hipGetLastError());
   return NKH_OK;
+}
+
+__global__ void __launch_bounds__(1024)
+    k_gs_step(const CgState *__restrict__ st, StepLength step, BoxRef last) {
+  if (!(st && st->done)) step_length(step);
+  else if (threadIdx.x == 0) box_report(last);
+}
+
+// The step length rides in the packet kernel as 8 blocks ahead of the
+// packets' (one works; 8 keep the packets' XCDs): it needs the operator's
+// partial sums only, and takes less than the assembly beside it (3.4 us and a
+// gap of 4 to 9 us as a kernel of its own on 560 elements, lx1 8).  Groups
+// beyond the packets' size (over 64 members) have a kernel after the packets',
+// and the step length its own after that.
+template <typename T>
+static int gs_assemble_step_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s,
+                              const uint8_t *flag, const StepLength &a, const BoxRef &last) {
+  if (gs.npk > 0 && gs.ngroups == gs.gpk) {
+    hipLaunchKernelGGL(k_gs_assemble_pk<T>, dim3(pk_blocks(gs.npk) + 8), dim3(256), 0, s, w,
+                       gs.pk_m, gs.pk_g, gs.pk_head, gs.idx, flag ? flag : gs.flag, gs.npk, st,
+                       8, a, last);
+  } else {
+    NK_TRY(gs_assemble_t(gs, w, st, s, flag));
+    hipLaunchKernelGGL(k_gs_step, dim3(1), dim3(1024), 0, s, st, a, last);
+  }
+  NK_HIP(hipGetLastError());
+  return NKH_OK;
+}
+
+int gs_assemble_step(const GsMap &gs, double *w, const CgState *st, hipStream_t s,
+                     const uint8_t *flag, const StepLength &a, const BoxRef &last) {
+  return gs_assemble_step_t(gs, w, st, s, flag, a, last);
+}
+
+int gs_assemble_step(const GsMap &gs, float *w, const CgState *st, hipStream_t s,
+                     const uint8_t *flag, const StepLength &a, const BoxRef &last) {
+  return gs_assemble_step_t(gs, w, st, s, flag, a, last);
 }
 
 int gs_assemble(const GsMap &gs, double *w, const CgState *st, hipStream_t s,

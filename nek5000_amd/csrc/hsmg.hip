@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "hsmg.h"
+#include "tails.h"
 
 namespace nekamd {
 
@@ -1321,7 +1322,7 @@ __device__ __forceinline__ void block_part(double a, double *part) {
   for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
   if ((threadIdx.x & 63) == 0) sa[threadIdx.x >> 6] = a;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
+  if (threadIdx.x == 0) leave(part + blockIdx.x, ((sa[0] + sa[1]) + sa[2]) + sa[3]);
 }
 
 __device__ __forceinline__ void block_part2(double a, double b, double *pa, double *pb) {
@@ -1336,8 +1337,8 @@ __device__ __forceinline__ void block_part2(double a, double b, double *pa, doub
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    pa[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
-    pb[blockIdx.x] = ((sb[0] + sb[1]) + sb[2]) + sb[3];
+    leave(pa + blockIdx.x, ((sa[0] + sa[1]) + sa[2]) + sa[3]);
+    leave(pb + blockIdx.x, ((sb[0] + sb[1]) + sb[2]) + sb[3]);
   }
 }
 
@@ -1377,7 +1378,9 @@ __global__ void __launch_bounds__(256)
 }
 
 __global__ void __launch_bounds__(256)
-    k_fcg_start(FcgState *st, const double *part, double vol, double param21, double tolps) {
+    k_fcg_start(FcgState *st, const double *part, double vol, double param21, double tolps,
+                int *cnt) {
+  clear_counters(cnt);
   const double t = final_sum(part);
   if (threadIdx.x == 0) {
     const double div0 = sqrt(t / vol);
@@ -1408,12 +1411,12 @@ __device__ __forceinline__ double wt_at(const uint8_t *__restrict__ c, int64_t i
 // previous residual r1 and forms rho2 = -glsc3(z,wt,r1-r) (hmholtz.f:2236-
 // 2241); r1 - r is the last update alpha*w exactly in exact arithmetic (w
 // still holds that iteration's A p), so rho2 = -alpha*glsc3(z,wt,w) without
-// the extra vector.
+// the extra vector.  beta in the last block.
 template <typename WT>
 __global__ void __launch_bounds__(256)
     k_fcg_dots(const double *__restrict__ z, const double *__restrict__ r,
                const double *__restrict__ w, const WT *__restrict__ wt, int64_t n,
-               double *pa, double *pb) {
+               double *pa, double *pb, int *cnt, FcgState *st) {
   double a = 0.0, b = 0.0;
   NK_GRID_LOOP(i, n) {
     const double zw = z[i] * wt_at(wt, i);
@@ -1421,18 +1424,15 @@ __global__ void __launch_bounds__(256)
     b += zw * w[i];
   }
   block_part2(a, b, pa, pb);
-}
-
-__global__ void __launch_bounds__(256) k_fcg_beta(FcgState *st, const double *pa, const double *pb) {
-  const double a = final_sum(pa);
-  const double b = final_sum(pb);
-  if (threadIdx.x == 0) {
-    st->rho0 = st->rho1;
-    st->rho1 = a;
-    // first iteration: r1 = 0, so rho2 = glsc3(z,wt,r); p = 0 then anyway
-    st->rho2 = (st->iter == 0) ? a : -st->alpha * b;
-    st->beta = st->rho2 / st->rho0;
-  }
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[2];
+  sum_left(pa, pb - pa, gridDim.x, t);
+  if (threadIdx.x != 0) return;
+  st->rho0 = st->rho1;
+  st->rho1 = t[0];
+  // first iteration: r1 = 0, so rho2 = glsc3(z,wt,r); p = 0 then anyway
+  st->rho2 = (st->iter == 0) ? t[0] : -st->alpha * t[1];
+  st->beta = st->rho2 / st->rho0;
 }
 
 // add2s1: p = beta*p + z
@@ -1456,16 +1456,6 @@ __global__ void __launch_bounds__(256)
   block_part(a, part);
 }
 
-// den from the count rho partials of the fused axhelm; alpha
-// one block of 1024 threads (the fused axhelm leaves up to 65536 partials)
-__global__ void __launch_bounds__(1024) k_fcg_alpha_n(FcgState *st, const double *part, int count) {
-  const double t = block_sum_partials(part, count);
-  if (threadIdx.x == 0) {
-    st->den = t;
-    st->alpha = st->rho1 / t;
-  }
-}
-
 __global__ void __launch_bounds__(256) k_fcg_alpha(FcgState *st, const double *part) {
   const double t = final_sum(part);
   if (threadIdx.x == 0) {
@@ -1474,12 +1464,30 @@ __global__ void __launch_bounds__(256) k_fcg_alpha(FcgState *st, const double *p
   }
 }
 
+// the block's part of sum r*r*wt; in the last block the residual's norm, the
+// exit test and the report of the state
+__device__ __forceinline__ void fcg_rnorm(double a, double *part, int *cnt, FcgState *st, double vol,
+                                          const BoxRef &rep) {
+  block_part(a, part);
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[1];
+  sum_left(part, 0, gridDim.x, t);
+  if (threadIdx.x != 0) return;
+  const double rn = sqrt(t[0] / vol);
+  st->rnorm = rn;
+  st->iter += 1;
+  if (rn < st->tolpss) st->done = 1;
+  *reinterpret_cast<FcgState *>(rep.b->v) = *st;
+  box_report(rep);
+}
+static_assert(sizeof(FcgState) <= sizeof(HostBox::v), "a report holds a state");
+
 // res += alpha p; r -= alpha w; partial sum r*r*wt
 template <typename WT>
 __global__ void __launch_bounds__(256)
     k_fcg_update(double *__restrict__ res, double *__restrict__ r, const double *__restrict__ p,
-                 const double *__restrict__ w, const WT *__restrict__ wt, const FcgState *st,
-                 int64_t n, double *part) {
+                 const double *__restrict__ w, const WT *__restrict__ wt, FcgState *st,
+                 int64_t n, double *part, int *cnt, double vol, BoxRef rep) {
   const double alpha = st->alpha;
   double a = 0.0;
   // streaming: every word is touched once, hence the nontemporal hints
@@ -1492,7 +1500,7 @@ __global__ void __launch_bounds__(256)
     __builtin_nontemporal_store(ri, r + i);
     a = a + ri * ri * wt_at(wt, i);
   }
-  block_part(a, part);
+  fcg_rnorm(a, part, cnt, st, vol, rep);
 }
 
 // r -= alpha w; partial sum r*r*wt (the fused path: x += alpha p is done by
@@ -1500,7 +1508,8 @@ __global__ void __launch_bounds__(256)
 template <typename WT>
 __global__ void __launch_bounds__(256)
     k_fcg_update_r(double *__restrict__ r, const double *__restrict__ w,
-                   const WT *__restrict__ wt, const FcgState *st, int64_t n, double *part) {
+                   const WT *__restrict__ wt, FcgState *st, int64_t n, double *part,
+                   int *cnt, double vol, BoxRef rep) {
   const double alpha = st->alpha;
   double a = 0.0;
   NK_GRID_LOOP(i, n) {
@@ -1509,7 +1518,7 @@ __global__ void __launch_bounds__(256)
     __builtin_nontemporal_store(ri, r + i);
     a = a + ri * ri * wt_at(wt, i);
   }
-  block_part(a, part);
+  fcg_rnorm(a, part, cnt, st, vol, rep);
 }
 
 // the last iteration's x += alpha p
@@ -1523,19 +1532,6 @@ __global__ void k_fcg_xfin(double *__restrict__ x, const double *__restrict__ p,
   }
 }
 
-__global__ void __launch_bounds__(256) k_fcg_rnorm(FcgState *st, const double *part, double vol,
-                                                   BoxRef rep) {
-  const double t = final_sum(part);
-  if (threadIdx.x == 0) {
-    const double rn = sqrt(t / vol);
-    st->rnorm = rn;
-    st->iter += 1;
-    if (rn < st->tolpss) st->done = 1;
-    *reinterpret_cast<FcgState *>(rep.b->v) = *st;
-    box_report(rep);
-  }
-}
-static_assert(sizeof(FcgState) <= sizeof(HostBox::v), "a report holds a state");
 
 }  // namespace
 
@@ -1562,11 +1558,12 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
   // (the mixed solver allocates fr..fw on its own, so each piece is checked)
   if (!mg.fr)
     for (double **p : {&mg.fr, &mg.fp, &mg.fz, &mg.fw}) NK_TRY(mg_dalloc(p, n));
-  if (!mg.fpart) NK_TRY(mg_dalloc(&mg.fpart, 3 * kFcgBlocks));
+  if (!mg.fpart) NK_TRY(mg_dalloc(&mg.fpart, 2 * kFcgBlocks + kCounterDoubles));
   if (!mg.fst) NK_HIP(hipMalloc(&mg.fst, sizeof(FcgState)));
   const double *mgmask = mg.lev[mg.lmax].mask;
   double *r = mg.fr, *p = mg.fp, *z = mg.fz, *w = mg.fw;
   double *pa = mg.fpart, *pb = mg.fpart + kFcgBlocks;
+  int *cnt = reinterpret_cast<int *>(mg.fpart + 2 * kFcgBlocks);
   // the operator's kernel choice for this order (w is scratch until the
   // first apply of the iteration)
   NK_TRY(axhelm_autotune(m, w, res, h1, h2, s));
@@ -1575,7 +1572,7 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
   NK_TRY(run_chktcg1(m, &tolps, facts));
   if (prm.param21 > 0 && tolps > std::fabs(prm.param21)) tolps = std::fabs(prm.param21);
   if (prm.istep == 0) tolps = 1.e-4;
-  const dim3 g(kFcgBlocks), b(256);
+  const dim3 g(kFcgBlocks), gd(dot_blocks(n)), b(256);
   // r stays masked by the update (w carries pmask) when pmask is the
   // multigrid's fine mask; otherwise it is masked again before every V-cycle
   // as h1mg_solve does
@@ -1588,9 +1585,12 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
   const bool fused = !differ && facts.fused();
   NK_TRY(ensure_small(m));
   double *rho_part = m.red + kRedRho1;
-  const int nrho = axhelm_cg_grid(m);
+  // den = the partials the fused axhelm leaves, alpha = rho1 / den
+  const StepLength step{rho_part, axhelm_cg_grid(m), &mg.fst->rho1, &mg.fst->den,
+                        &mg.fst->alpha, nullptr, nullptr, nullptr};
   hipLaunchKernelGGL(k_fcg_init, g, b, 0, s, r, res, p, wt, mgmask, n, pa);
-  hipLaunchKernelGGL(k_fcg_start, dim3(1), b, 0, s, mg.fst, pa, m.vol, prm.param21, tolps);
+  hipLaunchKernelGGL(k_fcg_start, dim3(1), b, 0, s, mg.fst, pa, m.vol, prm.param21, tolps,
+                     cnt);
   NK_HIP(hipGetLastError());
   Timers &tm = timers();
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -1600,20 +1600,21 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
   int iter = 0;
   int rc = NKH_OK;
   for (int k = 1; k <= maxit; ++k) {
+    const BoxRef rep = m.next_report();
     if (differ && (rc = mul_inplace(r, mgmask, n, s)) != NKH_OK) break;
     if ((rc = mg_solve(m, z, r, s, prm.param40, prm.precision)) != NKH_OK) break;
-    if (wtc) hipLaunchKernelGGL(k_fcg_dots<uint8_t>, g, b, 0, s, z, r, w, wtc, n, pa, pb);
-    else hipLaunchKernelGGL(k_fcg_dots<double>, g, b, 0, s, z, r, w, wt, n, pa, pb);
-    hipLaunchKernelGGL(k_fcg_beta, dim3(1), b, 0, s, mg.fst, pa, pb);
+    if (wtc) hipLaunchKernelGGL(k_fcg_dots<uint8_t>, gd, b, 0, s, z, r, w, wtc, n, pa, pb,
+                         cnt, mg.fst);
+    else hipLaunchKernelGGL(k_fcg_dots<double>, gd, b, 0, s, z, r, w, wt, n, pa, pb,
+                         cnt, mg.fst);
     if (fused) {
       if (tm.on) (void)hipEventRecord(ev[0], s);
       if ((rc = launch_axhelm_flex(m, w, p, z, h1, h2, &mg.fst->beta, rho_part, s, res,
                                    &mg.fst->alpha)) != NKH_OK)
         break;
       if (tm.on) (void)hipEventRecord(ev[1], s);
-      if ((rc = gs_assemble(m.gs, w, nullptr, s)) != NKH_OK) break;
+      if ((rc = gs_assemble_step(m.gs, w, nullptr, s, nullptr, step, BoxRef{})) != NKH_OK) break;
       if (tm.on) (void)hipEventRecord(ev[2], s);
-      hipLaunchKernelGGL(k_fcg_alpha_n, dim3(1), dim3(1024), 0, s, mg.fst, rho_part, nrho);
     } else {
       hipLaunchKernelGGL(k_fcg_p, dim3(mg_grid(n)), b, 0, s, p, z, mg.fst, n);
       if (tm.on) (void)hipEventRecord(ev[0], s);
@@ -1625,15 +1626,17 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
       hipLaunchKernelGGL(k_fcg_alpha, dim3(1), b, 0, s, mg.fst, pa);
     }
     if (fused && wtc)
-      hipLaunchKernelGGL(k_fcg_update_r<uint8_t>, g, b, 0, s, r, w, wtc, mg.fst, n, pa);
+      hipLaunchKernelGGL(k_fcg_update_r<uint8_t>, gd, b, 0, s, r, w, wtc, mg.fst, n, pa, cnt,
+                         m.vol, rep);
     else if (fused)
-      hipLaunchKernelGGL(k_fcg_update_r<double>, g, b, 0, s, r, w, wt, mg.fst, n, pa);
+      hipLaunchKernelGGL(k_fcg_update_r<double>, gd, b, 0, s, r, w, wt, mg.fst, n, pa, cnt,
+                         m.vol, rep);
     else if (wtc)
-      hipLaunchKernelGGL(k_fcg_update<uint8_t>, g, b, 0, s, res, r, p, w, wtc, mg.fst, n, pa);
+      hipLaunchKernelGGL(k_fcg_update<uint8_t>, gd, b, 0, s, res, r, p, w, wtc, mg.fst, n, pa,
+                         cnt, m.vol, rep);
     else
-      hipLaunchKernelGGL(k_fcg_update<double>, g, b, 0, s, res, r, p, w, wt, mg.fst, n, pa);
-    const BoxRef rep = m.next_report();
-    hipLaunchKernelGGL(k_fcg_rnorm, dim3(1), b, 0, s, mg.fst, pa, m.vol, rep);
+      hipLaunchKernelGGL(k_fcg_update<double>, gd, b, 0, s, res, r, p, w, wt, mg.fst, n, pa,
+                         cnt, m.vol, rep);
     if (hipGetLastError() != hipSuccess) {
       set_error("hmh_flex_cg: kernel launch failed");
       rc = NKH_ERR_HIP;

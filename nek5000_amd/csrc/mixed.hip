@@ -16,6 +16,7 @@
 
 #include "element_kernels.h"
 #include "hsmg.h"
+#include "tails.h"
 
 namespace nekamd {
 
@@ -39,7 +40,7 @@ __device__ __forceinline__ void part1(double a, double *part) {
   for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
   if ((threadIdx.x & 63) == 0) sa[threadIdx.x >> 6] = a;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = ((sa[0] + sa[1]) + sa[2]) + sa[3];
+  if (threadIdx.x == 0) leave(part + blockIdx.x, ((sa[0] + sa[1]) + sa[2]) + sa[3]);
   __syncthreads();
 }
 
@@ -74,7 +75,9 @@ __global__ void k_mx_start(float *__restrict__ r, float *__restrict__ x, float *
   }
 }
 
-__global__ void k_mx_state(MxState *st, double tol) {
+__global__ void __launch_bounds__(64) k_mx_state(MxState *st, double tol, int *cnt) {
+  clear_counters(cnt);
+  if (threadIdx.x != 0) return;
   st->rho1 = 1.0;
   st->iter = 0;
   st->done = 0;
@@ -89,12 +92,12 @@ __device__ __forceinline__ float wt32(const uint8_t *__restrict__ c, int64_t i) 
 }
 
 // partials of sum z*wt*r and sum z*wt*w in FP64 (rho1 and the rho2 term,
-// as the FP64 solver: rho2 = -alpha sum z*wt*w_prev)
+// as the FP64 solver: rho2 = -alpha sum z*wt*w_prev); beta in the last block
 template <typename WT>
 __global__ void __launch_bounds__(256)
     k_mx_dots(const float *__restrict__ z, const float *__restrict__ r,
               const float *__restrict__ w, const WT *__restrict__ wt, int64_t n, double *pa,
-              double *pb) {
+              double *pb, int *cnt, MxState *st) {
   double a = 0.0, b = 0.0;
   NK_LOOP(i, n) {
     const double zw = (double)z[i] * (double)wt32(wt, i);
@@ -103,34 +106,23 @@ __global__ void __launch_bounds__(256)
   }
   part1(a, pa);
   part1(b, pb);
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[2];
+  sum_left(pa, pb - pa, gridDim.x, t);
+  if (threadIdx.x != 0) return;
+  st->rho0 = st->rho1;
+  st->rho1 = t[0];
+  st->rho2 = (st->iter == 0) ? t[0] : -st->alpha * t[1];
+  st->beta = st->rho2 / st->rho0;
 }
 
-__global__ void __launch_bounds__(256) k_mx_beta(MxState *st, const double *pa, const double *pb) {
-  const double a = fsum(pa, kMxBlocks);
-  const double b = fsum(pb, kMxBlocks);
-  if (threadIdx.x == 0) {
-    st->rho0 = st->rho1;
-    st->rho1 = a;
-    st->rho2 = (st->iter == 0) ? a : -st->alpha * b;
-    st->beta = st->rho2 / st->rho0;
-  }
-}
-
-// one block of 1024 threads (the fused axhelm leaves up to 65536 partials)
-__global__ void __launch_bounds__(1024) k_mx_alpha(MxState *st, const double *part, int count) {
-  const double t = block_sum_partials(part, count);
-  if (threadIdx.x == 0) {
-    st->den = t;
-    st->alpha = st->rho1 / t;
-  }
-}
-
-// x += alpha p; r -= alpha w; partial sum r*r*wt (FP64)
+// x += alpha p; r -= alpha w; partial sum r*r*wt (FP64); the norm, the exit
+// test and the report in the last block
 template <typename WT>
 __global__ void __launch_bounds__(256)
     k_mx_update(float *__restrict__ x, float *__restrict__ r, const float *__restrict__ p,
-                const float *__restrict__ w, const WT *__restrict__ wt, const MxState *st,
-                int64_t n, double *part) {
+                const float *__restrict__ w, const WT *__restrict__ wt, MxState *st,
+                int64_t n, double *part, int *cnt, double vol, BoxRef rep) {
   // 4 nodes per step with nontemporal hints (the vectors are separate
   // 256-byte aligned allocations), the tail node by node
   typedef float v4 __attribute__((ext_vector_type(4)));
@@ -169,20 +161,18 @@ __global__ void __launch_bounds__(256)
     a += (double)ri * (double)ri * (double)wt32(wt, i);
   }
   part1(a, part);
+  if (!last_block(cnt, gridDim.x)) return;
+  double t[1];
+  sum_left(part, 0, gridDim.x, t);
+  if (threadIdx.x != 0) return;
+  const double rn = sqrt(t[0] / vol);
+  st->rnorm = rn;
+  st->iter += 1;
+  if (rn < st->tol) st->done = 1;
+  *reinterpret_cast<MxState *>(rep.b->v) = *st;
+  box_report(rep);
 }
 
-__global__ void __launch_bounds__(256) k_mx_rnorm(MxState *st, const double *part, double vol,
-                                                  BoxRef rep) {
-  const double t = fsum(part, kMxBlocks);
-  if (threadIdx.x == 0) {
-    const double rn = sqrt(t / vol);
-    st->rnorm = rn;
-    st->iter += 1;
-    if (rn < st->tol) st->done = 1;
-    *reinterpret_cast<MxState *>(rep.b->v) = *st;
-    box_report(rep);
-  }
-}
 static_assert(sizeof(MxState) <= sizeof(HostBox::v), "a report holds a state");
 
 // the sum of the kMxBlocks partials, reported to the host
@@ -659,12 +649,12 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
            "mixed-precision solve: the pressure mask must be the multigrid's fine mask");
   if (!mg.xr) {
     for (float **p : {&mg.xr, &mg.xp, &mg.xz, &mg.xw, &mg.xx, &mg.xwt}) NK_TRY(falloc(p, n));
-    NK_TRY(mg_dalloc(&mg.xpart, 3 * kMxBlocks + kAxBlocks));
+    NK_TRY(mg_dalloc(&mg.xpart, 3 * kMxBlocks + kAxBlocks + kCounterDoubles));
     NK_HIP(hipMalloc(&mg.xst, sizeof(MxState)));
   }
   if (!mg.fr)
     for (double **p : {&mg.fr, &mg.fp, &mg.fz, &mg.fw}) NK_TRY(mg_dalloc(p, n));
-  const dim3 G(kMxBlocks), B(256);
+  const dim3 G(kMxBlocks), Gd(dot_blocks(n)), B(256);
   NK_TRY(ensure_geom32(m, s));
   // the weights as count bytes where every one is 1/count (1 B instead of 4
   // per node in the inner dots and update)
@@ -673,7 +663,9 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
   MxState *st = (MxState *)mg.xst;
   double *pa = mg.xpart, *pb = mg.xpart + kMxBlocks, *pc = mg.xpart + 2 * kMxBlocks;
   double *den_part = mg.xpart + 3 * kMxBlocks;
-  const int nden = axhelm_cg_grid(m);
+  int *cnt = reinterpret_cast<int *>(den_part + kAxBlocks);
+  const StepLength step{den_part, axhelm_cg_grid(m), &st->rho1, &st->den,
+                        &st->alpha, nullptr, nullptr, nullptr};
   double *r64 = mg.fr, *x64 = mg.fp, *b64 = mg.fz, *ax = mg.fw;
   // tolerance as hmh_flex_cg (hmholtz.f:2205-2220)
   double tolps = 0.0;
@@ -701,28 +693,27 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
   for (int outer = 0; outer < kMaxOuter && rn >= tolpss && total < maxit; ++outer) {
     const double itol = std::max(kInnerRtol * rn, 0.5 * tolpss);
     hipLaunchKernelGGL(k_mx_start, dim3(mg_grid(n)), B, 0, s, mg.xr, mg.xx, mg.xp, r64, n);
-    hipLaunchKernelGGL(k_mx_state, dim3(1), dim3(1), 0, s, st, itol);
+    hipLaunchKernelGGL(k_mx_state, dim3(1), dim3(64), 0, s, st, itol, cnt);
     NK_HIP(hipGetLastError());
     while (total < maxit) {
       // the inner V-cycles' coarse problem: one AMG V-cycle for param40 = 1,
       // else the coarse solve (crs_mode 2: 0.1 relative where it is the AMG-PCG)
       NK_TRY(mg_solve32(m, mg.xz, mg.xr, s, prm.param40 == 1 ? 1 : 2));
       if (wtc)
-        hipLaunchKernelGGL(k_mx_dots<uint8_t>, G, B, 0, s, mg.xz, mg.xr, mg.xw, wtc, n, pa, pb);
+        hipLaunchKernelGGL(k_mx_dots<uint8_t>, Gd, B, 0, s, mg.xz, mg.xr, mg.xw, wtc, n, pa, pb,
+                           cnt, st);
       else
-        hipLaunchKernelGGL(k_mx_dots<float>, G, B, 0, s, mg.xz, mg.xr, mg.xw, mg.xwt, n, pa, pb);
-      hipLaunchKernelGGL(k_mx_beta, dim3(1), B, 0, s, st, pa, pb);
+        hipLaunchKernelGGL(k_mx_dots<float>, Gd, B, 0, s, mg.xz, mg.xr, mg.xw, mg.xwt, n, pa, pb,
+                           cnt, st);
       NK_TRY(launch_axhelm32_flex(m, mg.xw, mg.xp, mg.xz, h1f, h2f, st, den_part, s));
-      NK_TRY(gs_assemble(m.gs, mg.xw, nullptr, s));
-      hipLaunchKernelGGL(k_mx_alpha, dim3(1), dim3(1024), 0, s, st, den_part, nden);
-      if (wtc)
-        hipLaunchKernelGGL(k_mx_update<uint8_t>, G, B, 0, s, mg.xx, mg.xr, mg.xp, mg.xw, wtc, st,
-                           n, pa);
-      else
-        hipLaunchKernelGGL(k_mx_update<float>, G, B, 0, s, mg.xx, mg.xr, mg.xp, mg.xw, mg.xwt,
-                           st, n, pa);
+      NK_TRY(gs_assemble_step(m.gs, mg.xw, nullptr, s, nullptr, step, BoxRef{}));
       const BoxRef rep = m.next_report();
-      hipLaunchKernelGGL(k_mx_rnorm, dim3(1), B, 0, s, st, pa, m.vol, rep);
+      if (wtc)
+        hipLaunchKernelGGL(k_mx_update<uint8_t>, Gd, B, 0, s, mg.xx, mg.xr, mg.xp, mg.xw, wtc, st,
+                           n, pa, cnt, m.vol, rep);
+      else
+        hipLaunchKernelGGL(k_mx_update<float>, Gd, B, 0, s, mg.xx, mg.xr, mg.xp, mg.xw, mg.xwt,
+                           st, n, pa, cnt, m.vol, rep);
       NK_HIP(hipGetLastError());
       NK_TRY(box_wait(rep, s));
       std::memcpy(&hs, rep.b->v, sizeof(MxState));

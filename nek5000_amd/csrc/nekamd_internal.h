@@ -27,8 +27,8 @@ constexpr int kUpdBlocks = 16384;
 // Layout of Mesh::red (doubles).
 constexpr int kRedPart1 = 0;                         // (z,r) partials
 constexpr int kRedPart2 = kUpdBlocks;                // (r,r)_binv partials
-constexpr int kRedRho2 = 2 * kUpdBlocks;             // rho partials (unfused path)
-constexpr int kRedScratch = kRedRho2 + kRedBlocks;   // setup reductions
+constexpr int kRedCount = 2 * kUpdBlocks;            // counters (last_block)
+constexpr int kRedScratch = kRedCount + kRedBlocks;   // setup reductions
 constexpr int kRedOut = kRedScratch + kRedBlocks;    // 64 result slots
 constexpr int kRedRho1 = kRedOut + 64;               // rho partials of axhelm
 constexpr int kRedHist = kRedRho1 + kAxBlocks;       // 5*kMaxCgIter history
@@ -95,7 +95,6 @@ struct CgState {
   int done;
   int niter;
   int converged;
-  int pending;    // x/r update of the previous iteration not yet applied
   int istep;
   int param18;
 };
