@@ -12,7 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libnekamd.so")
 OBJ = os.path.join(HERE, "_objs")
 # (the axhelm instantiations take longest and are compiled first)
-SOURCES = ["axhelm_cg.hip", "axhelm_flex.hip", "axhelm.hip", "axhelm_gated.hip", "hsmg.hip",
+SOURCES = ["axhelm_cg.hip", "axhelm_flex.hip", "axhelm.hip", "hsmg.hip",
            "capi.cpp", "kernels.hip", "gs.hip", "cg.hip",
            "hsmg_setup.hip", "coarse.hip", "coarse_direct.hip",
            "gmres.hip", "proj.hip", "adjoint.hip", "mesh_io.cpp", "mixed.hip"]

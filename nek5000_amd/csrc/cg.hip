@@ -11,7 +11,7 @@
 //     axhelm (MODE 1)  : p update fused in, w = A_L p, rho = sum p.w
 //     gs_assemble_step : w <- mask * dssum(w); in a block of its own alpha
 // (With the two scalar steps as kernels of their own 336 elements, lx1 8, took
-// 420 us a solve, now 347; 9e6 nodes 7250, now 7180.)
+// 420 us a solve, now 347; 1.68e7 nodes 7250, now 7180.)
 // rho is taken before the assembly: with p continuous and zero where the
 // mask is, and mult summing to one over each group of shared nodes,
 // (mask*QQ^T w, p)_mult = sum_l p_l w_l exactly in exact arithmetic.  The
@@ -262,7 +262,9 @@ __device__ __forceinline__ void state_report(const CgState *st, const BoxRef &re
   *reinterpret_cast<CgState *>(rep.b->v) = *st;
   box_report(rep);
 }
-static_assert(sizeof(CgState) <= sizeof(HostBox::v), "a report holds a state");
+// (of a mixed solve: the iteration's state, and whether a refresh is due)
+constexpr int kBoxDue = (int)(sizeof(HostBox::v) / sizeof(double)) - 1;
+static_assert(sizeof(CgState) <= sizeof(double) * kBoxDue, "a report holds a state");
 
 __device__ void cg_scalars1(CgState *st, double s1, double s2, double *hist) {
   const int iter = st->iter + 1;
@@ -417,7 +419,8 @@ __global__ void k_mask_guarded(double *__restrict__ w, const double *__restrict_
 // Sleijpen & van der Vorst 1996; Clark et al. 2010 for single/double CG).
 struct McgState {
   CgState cg;    // the iteration (read back by the host as a CgState)
-  CgState gate;  // gate.done == 0 while a refresh is due (gates its kernels)
+  CgState gate;  // beta, and done: no operator now (the solve ended, or due)
+  int due;       // a refresh is asked for
   double rmax;   // largest iterated residual norm since the last refresh
   int final;     // 1: iterated residual met the tolerance; 2: maxit reached
   int nrefresh;
@@ -433,15 +436,10 @@ struct McgState {
 // and 1e-6 gain nothing more and let the solution drift further (up to
 // 9e-9 relative from the FP64 solve at 1e-6, 4e-11 at 1e-4).
 constexpr double kRefresh = 1e-4;
-// grid of the refresh kernels: they run every pass of a captured loop and
-// mostly return at once, at a cost that grows with the number of blocks
-// (about 10 ns each), so it scales with the field: 64Ki nodes per block,
-// 64 to 2048 blocks (a multiple of 8, as the assembly's XCD mapping needs)
-constexpr int kRefreshBlocks = 2048;
-inline int refresh_blocks(int64_t n) {
-  int64_t b = (n + 65535) / 65536;
-  b = (b + 7) / 8 * 8;
-  return (int)(b < 64 ? 64 : (b > kRefreshBlocks ? kRefreshBlocks : b));
+__device__ __forceinline__ void state_report(const McgState *ms, const BoxRef &rep) {
+  if (!rep.b) return;
+  rep.b->v[kBoxDue] = ms->due;
+  state_report(&ms->cg, rep);
 }
 
 // as cg_scalars1, but a refresh of the residual is requested instead of
@@ -452,7 +450,7 @@ __device__ void mcg_scalars1(McgState *ms, double s1, double s2, double *hist) {
   st->iter = iter;
   if (iter > st->maxit) {  // loop exhausted: fold the correction into x
     ms->final = 2;
-    ms->gate.done = 0;
+    ms->due = ms->gate.done = 1;
     return;
   }
   st->rtz2 = st->rtz1;
@@ -471,16 +469,16 @@ __device__ void mcg_scalars1(McgState *ms, double s1, double s2, double *hist) {
   }
   if (rbn2 <= st->tol && (iter > 1 || st->istep <= 5)) {
     ms->final = 1;
-    ms->gate.done = 0;
+    ms->due = ms->gate.done = 1;
     return;
   }
   if (rbn2 < kRefresh * ms->rmax) {
     ms->final = 0;
-    ms->gate.done = 0;
+    ms->due = ms->gate.done = 1;
     return;
   }
   if (rbn2 > ms->rmax) ms->rmax = rbn2;
-  st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
+  ms->gate.beta = st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
 }
 
 // xs += alpha p ; r -= alpha w (FP32) ; FP64 partials of dm*r*r and bm*r*r;
@@ -490,7 +488,8 @@ __global__ void __launch_bounds__(256)
     k_mcg_update_dots(float *__restrict__ xs, float *__restrict__ r,
                       const float *__restrict__ p, const float *__restrict__ w,
                       const float *__restrict__ dm, const float *__restrict__ bm, int64_t n,
-                      McgState *ms, double *part1, double *part2, int *cnt, double *hist) {
+                      McgState *ms, double *part1, double *part2, int *cnt, double *hist,
+                      BoxRef rep) {
   CgState *st = &ms->cg;
   if (st->done) return;
   const float alpha = (float)st->alpha;
@@ -543,22 +542,25 @@ __global__ void __launch_bounds__(256)
   sum_left(part1, part2 - part1, gridDim.x, t);
   if (threadIdx.x != 0) return;
   mcg_scalars1(ms, t[0], t[1], hist);
+  state_report(ms, rep);
 }
 
 // the first iteration's, after k_mcg_init
 __global__ void __launch_bounds__(kScalThreads)
     k_mcg_scalars1(McgState *__restrict__ ms, const double *__restrict__ part1,
-                   const double *__restrict__ part2, int nparts, double *__restrict__ hist) {
+                   const double *__restrict__ part2, int nparts, double *__restrict__ hist,
+                   BoxRef rep) {
   if (ms->cg.done) return;
   double t[2];
   sum_left(part1, part2 - part1, nparts, t);
-  if (threadIdx.x == 0) mcg_scalars1(ms, t[0], t[1], hist);
+  if (threadIdx.x != 0) return;
+  mcg_scalars1(ms, t[0], t[1], hist);
+  state_report(ms, rep);
 }
 
 // refresh, part 1: x += xs (FP64), xs = 0
-__global__ void k_mcg_fold(double *__restrict__ x, float *__restrict__ xs, int64_t n,
-                           const CgState *__restrict__ gate) {
-  if (gate->done) return;
+__global__ void k_mcg_fold(double *__restrict__ x, float *__restrict__ xs, int64_t n) {
+#pragma unroll 4
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     x[i] = x[i] + (double)xs[i];
@@ -570,7 +572,7 @@ __global__ void k_mcg_fold(double *__restrict__ x, float *__restrict__ xs, int64
 // iteration continues from it with the same search direction
 __device__ void mcg_scalars1b(McgState *ms, double s1, double s2, double *hist) {
   CgState *st = &ms->cg;
-  ms->gate.done = 1;
+  ms->due = 0;
   ms->nrefresh += 1;
   const double rbn2 = sqrt(s2 / st->vol);
   st->rbn2 = rbn2;
@@ -593,23 +595,20 @@ __device__ void mcg_scalars1b(McgState *ms, double s1, double s2, double *hist) 
   }
   ms->final = 0;
   ms->rmax = rbn2;
-  st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
+  ms->gate.done = 0;
+  ms->gate.beta = st->beta = (iter == 1) ? 0.0 : st->rtz1 / st->rtz2;
 }
 
 // refresh, part 2 (after ax = mask*QQ^T A_L x): r = f - ax in FP64, stored
 // rounded; partials of dm*r32^2 (the iteration's rtz) and bm*r^2 (FP64 norm);
-// part 3 in the last block.  The state is reported whether a refresh runs or
-// not.
+// part 3 and the report in the last block.
 __global__ void __launch_bounds__(256)
     k_mcg_resid(float *__restrict__ r32, const double *__restrict__ f,
                 const double *__restrict__ ax, const float *__restrict__ dm,
                 const float *__restrict__ bm, int64_t n, McgState *ms, double *part1,
                 double *part2, int *cnt, double *hist, BoxRef rep) {
-  if (ms->gate.done) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) state_report(&ms->cg, rep);
-    return;
-  }
   double s1 = 0.0, s2 = 0.0;
+#pragma unroll 4
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const double ri = f[i] - ax[i];
@@ -624,7 +623,7 @@ __global__ void __launch_bounds__(256)
   sum_left(part1, part2 - part1, gridDim.x, t);
   if (threadIdx.x != 0) return;
   mcg_scalars1b(ms, t[0], t[1], hist);
-  state_report(&ms->cg, rep);
+  state_report(ms, rep);
 }
 
 // x = 0, xs = 0, r = f (rounded), and 1/d (d the assembled diagonal), its
@@ -854,7 +853,7 @@ struct CgRun {
   HostBox *box = nullptr;  // null: no reports
   BoxRef last;             // the second report of the iteration enqueued last
   BoxRef exit_test() const { return BoxRef{box, last.seq - 1}; }
-  int wait(CgState *hs, hipStream_t s) const {
+  int wait(CgState *hs, hipStream_t s) {
     NK_TRY(box_wait(exit_test(), s));
     std::memcpy(hs, box->v, sizeof(CgState));
     return hs->done ? box_wait(last, s) : NKH_OK;
@@ -927,6 +926,11 @@ struct CgRun {
     return NKH_OK;
   }
 
+  template <class Ev>
+  int go_on(hipStream_t s, Ev &&ev) {
+    return enqueue(s, ev(launched));
+  }
+
   // one iteration's launches on s; ev (optional, 3 events) brackets axhelm
   // and the assembly
   int enqueue(hipStream_t s, hipEvent_t *ev = nullptr) {
@@ -996,12 +1000,14 @@ struct McgRun {
   // An iteration makes two reports: the state after its exit test, and the
   // end of its last kernel if the solve is done (a solve returns only when
   // nothing of it is left to run).
-  HostBox *box = nullptr;  // null: no reports
+  HostBox *box = nullptr;
+  bool due = false;  // the last report asked for a refresh
   BoxRef last;             // the second report of the iteration enqueued last
   BoxRef exit_test() const { return BoxRef{box, last.seq - 1}; }
-  int wait(CgState *hs, hipStream_t s) const {
+  int wait(CgState *hs, hipStream_t s) {
     NK_TRY(box_wait(exit_test(), s));
     std::memcpy(hs, box->v, sizeof(CgState));
+    due = box->v[kBoxDue] != 0.0;
     return hs->done ? box_wait(last, s) : NKH_OK;
   }
 
@@ -1056,7 +1062,6 @@ struct McgRun {
     h.cg.maxit = niter;
     h.cg.istep = prm.istep;
     h.cg.param18 = prm.param18;
-    h.gate.done = 1;
     hipLaunchKernelGGL(k_mcg_init, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, r, d, dm, bm, f,
                        ax, mult, mesh.binv, prm.param18 == 1 ? 1 : 0, n, red + kRedPart1,
                        red + kRedPart2, h, ms, counters(red));
@@ -1075,34 +1080,57 @@ struct McgRun {
     return NKH_OK;
   }
 
+  // what follows the last report: a refresh if it asked for one, or the next
+  // iteration; ev(k): the events of iteration k
+  template <class Ev>
+  int go_on(hipStream_t s, Ev &&ev) {
+    return due ? refresh(s, ev(launched - 1)) : enqueue(s, ev(launched));
+  }
+
+  // One iteration's launches on s.  Its operator returns at once when the
+  // tests of the iteration ask for a refresh: the host, told so, enqueues that
+  // and the operator again (refresh()).
   int enqueue(hipStream_t s, hipEvent_t *ev = nullptr) {
     const int64_t n = m->n;
-    double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1;
+    double *part1 = red + kRedPart1, *part2 = red + kRedPart2;
     const int ub = upd_blocks(n);
+    last = BoxRef{box, last.seq + 2};
     if (launched > 0)
       hipLaunchKernelGGL((vec_ok ? k_mcg_update_dots<true> : k_mcg_update_dots<false>), dim3(ub),
                          dim3(256), 0, s, xs, r, p, w, dm, bm, n, ms, part1, part2,
-                         counters(red), hist);
+                         counters(red), hist, exit_test());
     else  // (the first iteration's sums come from k_mcg_init)
       hipLaunchKernelGGL(k_mcg_scalars1, dim3(1), dim3(kScalThreads), 0, s, ms, part1, part2, ub,
-                         hist);
-    // the refresh (its kernels return at once while the gate is closed)
-    const CgState *gate = &ms->gate;
-    const int rb = refresh_blocks(n);
-    hipLaunchKernelGGL(k_mcg_fold, dim3(rb), dim3(256), 0, s, x, xs, n, gate);
-    NK_TRY(launch_axhelm_gated(*m, ax, x, h1, h2, gate, s));
-    NK_TRY(gs_assemble(m->gs, ax, gate, s, flag, rb));
+                         hist, exit_test());
+    NK_TRY(enqueue_operator(s, ev));
+    ++launched;
+    return NKH_OK;
+  }
+
+  // The refresh that the last report asked for, and that iteration's operator.
+  // (With the refresh in every iteration, its kernels returning at once on
+  // small grids where none was due, a solve of 12 iterations with 2 refreshes
+  // on 9e6 nodes, lx1 8, took 3340 us, now 2830.)
+  int refresh(hipStream_t s, hipEvent_t *ev = nullptr) {
+    const int64_t n = m->n;
     last = BoxRef{box, last.seq + 2};
-    hipLaunchKernelGGL(k_mcg_resid, dim3(rb), dim3(256), 0, s, r, f, ax, dm, bm, n, ms, part1,
-                       part2, counters(red), hist, exit_test());
+    hipLaunchKernelGGL(k_mcg_fold, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, n);
+    NK_TRY(launch_axhelm(*m, ax, x, h1, h2, s));
+    NK_TRY(gs_assemble(m->gs, ax, nullptr, s, flag));
+    hipLaunchKernelGGL(k_mcg_resid, dim3(upd_blocks(n)), dim3(256), 0, s, r, f, ax, dm, bm, n, ms,
+                       red + kRedPart1, red + kRedPart2, counters(red), hist, exit_test());
+    return enqueue_operator(s, ev);
+  }
+
+  int enqueue_operator(hipStream_t s, hipEvent_t *ev) {
+    double *rho1 = red + kRedRho1;
     if (ev) NK_HIP(hipEventRecord(ev[0], s));
-    NK_TRY(launch_axhelm32_jac(*m, w, p, r, d, (float)h1.s, (float)h2.s, st, rho1, s));
+    NK_TRY(launch_axhelm32_jac(*m, w, p, r, d, (float)h1.s, (float)h2.s, &ms->gate, rho1, s));
     if (ev) NK_HIP(hipEventRecord(ev[1], s));
-    NK_TRY(gs_assemble_step(m->gs, w, st, s, flag, step_of(st, rho1, ax_grid_parts, hist),
+    NK_TRY(gs_assemble_step(m->gs, w, &ms->gate, s, flag, step_of(st, rho1, ax_grid_parts, hist),
                             last));
     if (ev) NK_HIP(hipEventRecord(ev[2], s));
     NK_HIP(hipGetLastError());
-    ++launched;
     return NKH_OK;
   }
 
@@ -1162,7 +1190,7 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
   // allocation-free solve) the state is copied back, later on every fourth
   // iteration.
   while (true) {
-    NK_TRY(run.enqueue(s, timed ? &ev[4 * run.launched] : nullptr));
+    NK_TRY(run.go_on(s, [&](int k) { return timed ? &ev[4 * k] : nullptr; }));
     if (run.box) {
       m.box_seq = run.last.seq;
       NK_TRY(run.wait(&hs, s));
@@ -1450,12 +1478,13 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
     NK_HIP(hipEventRecord(B.ev[0], s));
     int rc = NKH_OK;
     std::vector<int> open;
+    auto no_events = [](int) -> hipEvent_t * { return nullptr; };
     for (int k : active) {
       Run &run = runs[(size_t)k];
       run.box = B.box[(size_t)k];
       run.last.seq = B.seq[(size_t)k];
       NK_HIP(hipStreamWaitEvent(B.streams[(size_t)k], B.ev[0], 0));
-      if (rc == NKH_OK) rc = run.enqueue(B.streams[(size_t)k]);
+      if (rc == NKH_OK) rc = run.go_on(B.streams[(size_t)k], no_events);
       B.seq[(size_t)k] = run.last.seq;
       open.push_back(k);
     }
@@ -1477,7 +1506,7 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
           rc = NKH_ERR_STATE;
           break;
         }
-        if ((rc = run.enqueue(q)) != NKH_OK) break;
+        if ((rc = run.go_on(q, no_events)) != NKH_OK) break;
         B.seq[(size_t)k] = run.last.seq;
         next.push_back(k);
       }

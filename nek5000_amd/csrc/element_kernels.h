@@ -100,12 +100,11 @@ __device__ __forceinline__ void stnt(double v, double *p) { __builtin_nontempora
 // from *betap; with xacc, also the previous iteration's solution update
 // res += alpha p (hmholtz.f:2250-2251) on the p it reads, alpha from
 // *alphap -- the same arithmetic one iteration later, so that the update
-// kernel need not read p and x again.  MODE 3: MODE 0 gated by a state (returns while st->done),
-// for applies that a captured iteration runs only on some passes.
+// kernel need not read p and x again.
 // ---------------------------------------------------------------------------
 
 // One thread's t-column of the operand (node base + k NP^2, k = 0..NP-1):
-// u itself (MODE 0, 3), p = beta p + d r (MODE 1; without p in iteration 1) or
+// u itself (MODE 0), p = beta p + d r (MODE 1; without p in iteration 1) or
 // p = beta p + z with x += alpha p (MODE 2), stored where `store`.  Every load
 // is issued, unconditionally, before the first value is used: with each
 // load in a branch of its own the compiler waited for it there (NP = 8, MODE
@@ -214,9 +213,6 @@ __global__ void __launch_bounds__(NP * NP * EPB_,
   if constexpr (MODE == 2) {
     beta = *betap;
     if (xacc) alpha = *alphap;
-  }
-  if constexpr (MODE == 3) {
-    if (st->done) return;
   }
   const int tid = threadIdx.x;
   const int le = tid / NP2;
@@ -327,9 +323,6 @@ __global__ void __launch_bounds__(NP * NP * EPB_)
   if constexpr (MODE == 2) {
     beta = *betap;
     if (xacc) alpha = *alphap;
-  }
-  if constexpr (MODE == 3) {
-    if (st->done) return;
   }
   const int tid = threadIdx.x;
   const int le = tid / NP2;
@@ -471,9 +464,6 @@ __global__ void __launch_bounds__(mx_threads<NP>(),
   if constexpr (MODE == 2) {
     beta = *betap;
     if (xacc) alpha = *alphap;
-  }
-  if constexpr (MODE == 3) {
-    if (st->done) return;
   }
   const int tid = threadIdx.x;
   const bool own = tid < NP2;
@@ -647,9 +637,6 @@ __global__ void __launch_bounds__(mx_threads<NP>(), 2)
     beta = *betap;
     if (xacc) alpha = *alphap;
   }
-  if constexpr (MODE == 3) {
-    if (st->done) return;
-  }
   const int tid = threadIdx.x;
   const bool own = tid < NP2;
   const int i = own ? tid % NP : 0, j = own ? tid / NP : 0;
@@ -795,11 +782,11 @@ __global__ void __launch_bounds__(mx_threads<NP>(), 2)
 }
 
 // Per polynomial order: which of the two kernels (0: element staged in LDS,
-// 1: t-planes) for the plain apply (and its gated form), the CG-fused and
+// 1: t-planes) for the plain apply, the CG-fused and
 // the flexible-CG-fused apply, and how many blocks for the plain apply;
 // chosen by the autotuner on the first large apply of that order.
 struct AxhelmChoice {
-  int variant = 0;       // plain apply (MODE 0, MODE 3)
+  int variant = 0;       // plain apply (MODE 0)
   int grid = 0;          // plain apply: blocks (0 -> one per element group, up to 2^20)
   int variant_cg = 0;    // MODE 1
   int variant_flex = 0;  // MODE 2
@@ -837,13 +824,7 @@ static int axhelm_go(const Mesh &m, const DMat<NP> &Dm, double *au, const double
                      const double *alphap = nullptr) {
   const int64_t ngroups = (m.nel + EPB - 1) / EPB;
   int grid;
-  if (MODE == 3) {
-    // gated: most launches find the gate closed, and an empty launch costs
-    // in proportion to its blocks: 16 element groups per block, 64 to 4096
-    int64_t g = ngroups / 16;
-    g = g < 64 ? 64 : (g > 4096 ? 4096 : g);
-    grid = (int)(ngroups < g ? ngroups : g);
-  } else if (MODE >= 1) {
+  if (MODE >= 1) {
     // one partial sum per block: the fixed count the CG's scalar kernels read
     grid = axhelm_cg_grid(m);
   } else {
@@ -872,11 +853,7 @@ static int axhelm_go(const Mesh &m, const DMat<NP> &Dm, double *au, const double
     hipLaunchKernelGGL((k_axhelm<NP, MODE, H1F_, H2M_, EPB>), dim3(grid), block, 0, s, Dm,    \
                        m.Dd, au, u, m.g, m.n, h1.f, h1.s, h2.f, h2.s, m.bm1, m.nel, pout, r,   \
                        dinv, mult, st, rho_part, betap, xacc, alphap)
-  if constexpr (MODE == 3) {  // the mixed solver's: constant coefficients
-    NK_CHECK(!h1f && h2m != 2, NKH_ERR_ARG, "gated axhelm: constant h1 and h2 only");
-    if (h2m == 0) NK_LAUNCH(false, 0);
-    else NK_LAUNCH(false, 1);
-  } else if (h1f) {
+  if (h1f) {
     if (h2m == 0) NK_LAUNCH(true, 0);
     else if (h2m == 1) NK_LAUNCH(true, 1);
     else NK_LAUNCH(true, 2);

@@ -477,10 +477,9 @@ static int gs_blocks(int64_t ngroups) {
   return (int)(b < 64 ? 64 : (b > kGsBlocks ? kGsBlocks : b));
 }
 
-// nblocks (> 0): grid of the per-group kernel of the large groups
 template <typename T>
 static int gs_assemble_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s,
-                         const uint8_t *flag, int nblocks = 0) {
+                         const uint8_t *flag) {
   if (gs.ngroups == 0) return NKH_OK;
   const uint8_t *fl = flag ? flag : gs.flag;
   if (gs.npk > 0)
@@ -489,7 +488,7 @@ static int gs_assemble_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s
                        BoxRef{});
   const int64_t nbig = gs.ngroups - gs.gpk;
   if (nbig > 0) {
-    const int nb = nblocks > 0 ? nblocks : gs_blocks(nbig);
+    const int nb = gs_blocks(nbig);
     const int64_t chunk = (nbig + nb - 1) / nb;
     hipLaunchKernelGGL(k_gs_assemble<T>, dim3(nb), dim3(256), 0, s, w, gs.off, gs.idx, fl,
                        gs.gpk, gs.ngroups, chunk, st);
@@ -536,8 +535,8 @@ int gs_assemble_step(const GsMap &gs, float *w, const CgState *st, hipStream_t s
 }
 
 int gs_assemble(const GsMap &gs, double *w, const CgState *st, hipStream_t s,
-                const uint8_t *flag, int nblocks) {
-  return gs_assemble_t(gs, w, st, s, flag, nblocks);
+                const uint8_t *flag) {
+  return gs_assemble_t(gs, w, st, s, flag);
 }
 
 int gs_assemble(const GsMap &gs, float *w, const CgState *st, hipStream_t s,

@@ -289,9 +289,6 @@ int axhelm_autotune(const Mesh &m, double *au, const double *u, Coef h1, Coef h2
                     hipStream_t s);
 int axhelm_set_tuning(int np, int variant, int grid);  // all three applies
 int axhelm_tuning_fused(int np, int *variant_cg, int *variant_flex);
-// MODE 0 apply that returns while gate->done (replayed in captured loops).
-int launch_axhelm_gated(const Mesh &m, double *au, const double *u, Coef h1, Coef h2,
-                        const CgState *gate, hipStream_t s);
 // FP32 operator (mixed.hip): g32/bm1_32 current for the mesh's geometry.
 int ensure_geom32(Mesh &m, hipStream_t s);
 // FP32 Jacobi-CG apply: p = d*r + beta*p (beta = st->beta), w = A_L p with
@@ -329,9 +326,8 @@ int gs_op(const GsMap &gs, double *u, int op, hipStream_t s);
 // CG assembly: w <- mask * dssum(w) using the flags of gs_prepare; skipped
 // when st is given and st->done.
 // flag: group flags to use instead of gs.flag (a solve with its own mask)
-// nblocks: grid (a multiple of 8; 0 -> kGsBlocks)
 int gs_assemble(const GsMap &gs, double *w, const CgState *st, hipStream_t s,
-                const uint8_t *flag = nullptr, int nblocks = 0);
+                const uint8_t *flag = nullptr);
 int gs_assemble(const GsMap &gs, float *w, const CgState *st, hipStream_t s,
                 const uint8_t *flag = nullptr);
 // Per id group (single members included): S = sum of e; z_i <- mean over

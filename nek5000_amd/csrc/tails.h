@@ -1,8 +1,8 @@
 // Scalar work of the Krylov loops done by the kernels around it instead of by
 // one-block kernels of their own, each of which cost 3 to 5 us and a gap of 4
 // to 9 us between launches (MI355X).  Without them: Jacobi PCG on 336
-// elements, lx1 8, 420 -> 347 us a solve, on 9e6 nodes 7250 -> 7180; batch of
-// five 1810 -> 1660; GMRES lx1 6 2440 -> 2300; flexible CG in FP32 3640 -> 3490.
+// elements, lx1 8, 420 -> 347 us a solve, on 1.68e7 nodes 7250 -> 7180; batch
+// of five 1810 -> 1660; GMRES lx1 6 2440 -> 2300; flexible CG in FP32 3640 -> 3490.
 #pragma once
 #include "nekamd_internal.h"
 
@@ -18,7 +18,7 @@ inline int dot_blocks(int64_t n) {
 // Results that a block leaves for the last block of its grid, wherever that
 // runs: agent-scope stores and loads, which do not stay in an XCD's own L2.
 // (A fence per block in their place writes that L2 back each time: the
-// update-and-dots kernel on 9e6 nodes took 180 us without, 650 us with it.)
+// update-and-dots kernel on 1.68e7 nodes took 180 us without, 600 with it.)
 __device__ __forceinline__ void leave(double *p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
