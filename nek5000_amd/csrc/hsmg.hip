@@ -593,6 +593,8 @@ int launch_sch_out(EO *e, const R *wint, const R *wgh, int nh, int64_t nel, hipS
 //   MODE 4: MODE 3 with eb formed from the local solutions (eb = wint, eg =
 //           wgh, of type EB) by the overlap sum, rounded to EO as a stored
 //           overlap sum would be.
+//   MODE 5: MODE 2 from the coarse unknowns: node q of u is u[eb[q]], 0 where
+//           eb[q] < 0.
 template <int NV, int NU, int MODE, typename EB, typename UT, typename VT, typename WT,
           typename EO = EB>
 __global__ void k_tnsr(VT *__restrict__ v, const UT *__restrict__ u,
@@ -608,7 +610,13 @@ __global__ void k_tnsr(VT *__restrict__ v, const UT *__restrict__ u,
   for (int64_t e = blockIdx.x; e < nel; e += gridDim.x) {
     __syncthreads();
     for (int t = threadIdx.x; t < NU3; t += blockDim.x) {
-      double x = double(u[(int64_t)e * NU3 + t]);
+      double x;
+      if constexpr (MODE == 5) {
+        const int q = eb[(int64_t)e * NU3 + t];
+        x = q >= 0 ? double(u[q]) : 0.0;
+      } else {
+        x = double(u[(int64_t)e * NU3 + t]);
+      }
       if constexpr (MODE == 1) x = x * wdec(w, (int64_t)e * NU3 + t, nullptr);
       su[t] = x;
     }
@@ -632,7 +640,7 @@ __global__ void k_tnsr(VT *__restrict__ v, const UT *__restrict__ u,
       double s = 0.0;
       for (int m = 0; m < NU; ++m) s += s2[ij + NV * NV * m] * sA[k + NV * m];
       const int64_t o = (int64_t)e * NV3 + t;
-      if constexpr (MODE == 2) {
+      if constexpr (MODE == 2 || MODE == 5) {
         v[o] = VT(double(v[o]) * wdec(w, o, nullptr) + s);
       } else if constexpr (MODE == 3) {
         const int i = t % NV, j = (t / NV) % NV, k = t / (NV * NV);
@@ -1107,12 +1115,40 @@ static int coarse_solve(Mg &mg, double *e1, const double *r1, int crs_mode, hipS
     if (mg.null_space)
       hipLaunchKernelGGL(k_sub_mean_1b, dim3(1), dim3(1024), 0, s, mg.cx, n);
   }
-  hipLaunchKernelGGL(k_crs_scatter, dim3(mg_grid(8 * mg.nel)), dim3(256), 0, s, e1, mg.cx,
-                     mg.slot, 8 * mg.nel);
+  if (e1)
+    hipLaunchKernelGGL(k_crs_scatter, dim3(mg_grid(8 * mg.nel)), dim3(256), 0, s, e1, mg.cx,
+                       mg.slot, 8 * mg.nel);
   NK_HIP(hipGetLastError());
   return NKH_OK;
 }
 
+// e_2 = e_2 * (mask*wt) + J e_1 straight from the coarse solution (without
+// the scatter's launch and its pass over level 1)
+static int prolong_coarse(Mg &mg, hipStream_t s) {
+  MgLevel &C = mg.lev[1], &F = mg.lev[2];
+  const dim3 g((int)std::min<int64_t>(mg.nel, 1 << 20)), b(64);
+  const double *none = nullptr;
+  const int32_t *no_eg = nullptr;
+  NK_CHECK(C.nh == 2 && (F.nh == 3 || F.nh == 4), NKH_ERR_UNSUPPORTED,
+           "level transfer %d <-> %d not instantiated", F.nh, C.nh);
+  if (F.nh == 4)
+    hipLaunchKernelGGL((k_tnsr<4, 2, 5, int32_t, double, double, double>), g, b, 0, s, F.e, mg.cx,
+                       F.mswt, C.J, mg.nel, mg.slot, none, no_eg);
+  else
+    hipLaunchKernelGGL((k_tnsr<3, 2, 5, int32_t, double, double, double>), g, b, 0, s, F.e, mg.cx,
+                       F.mswt, C.J, mg.nel, mg.slot, none, no_eg);
+  NK_HIP(hipGetLastError());
+  return NKH_OK;
+}
+
+// Local nodes up to which the whole V-cycle runs on the caller's stream.  On
+// three streams the levels overlap, but a wait for another stream costs 10 to
+// 20 us, and there are four on the longest path.  One stream / three, us a
+// solve: GMRES on 3.7e5 nodes 1805 / 2318, flexible CG in FP32 on 2.5e6 nodes
+// 3428 / 3430 (the fine level's local solves take 30 us there, the coarse
+// chain 100); beyond, the overlap saves the coarse chain (1.4e7 nodes: 330 us
+// of it beside 320 of the fine level).
+constexpr int64_t kOneStream = 2000000;
 // hsmg.f:1855-1949 H1MG_SOLVE (additive V-cycle, sigma = 1): z = M r, r
 // already masked with the fine-level mask.
 // The V-cycle with the fine-level input r and output z stored as FT: double
@@ -1128,7 +1164,16 @@ static int mg_solve_t(Mesh &mesh, FT *z, const FT *r, hipStream_t s, int crs_mod
   Mg &mg = *mesh.mg;
   const int Lm = mg.lmax;
   const int64_t nel = mg.nel;
-  hipStream_t b = mg.sb;
+  const bool one = mesh.n <= kOneStream;
+  hipStream_t b = one ? s : mg.sb;
+  auto record = [&](hipEvent_t ev, hipStream_t q) -> int {
+    if (!one) NK_HIP(hipEventRecord(ev, q));
+    return NKH_OK;
+  };
+  auto wait = [&](hipStream_t q, hipEvent_t ev) -> int {
+    if (!one) NK_HIP(hipStreamWaitEvent(q, ev, 0));
+    return NKH_OK;
+  };
   // fine level on s: local solves and overlap sum.  With ids zero exactly
   // at element interiors, the dssum of the Schwarz sum, the weights, the
   // coarse correction and dsavg are done together after the join (gs_fin);
@@ -1168,15 +1213,15 @@ static int mg_solve_t(Mesh &mesh, FT *z, const FT *r, hipStream_t s, int crs_mod
       NK_TRY((run_tnsr<1, double, FT, double>(C.r, C.nh, r, T.nh, T.rwt, C.Jt, nel, s,
                                               (const double *)nullptr, C.mask)));
     NK_TRY(gs_op(C.gs, C.r, 0, s));
-    NK_HIP(hipEventRecord(mg.ev_lr[Lm - 1], s));
+    NK_TRY(record(mg.ev_lr[Lm - 1], s));
     rsrc = C.r;
     if (Lm - 1 == 2) {
       NK_TRY(run_tnsr<1>(L1.r, L1.nh, C.r, L2.nh, L2.rwt, L1.Jt, nel, s));
       l1_restricted = true;
     }
   }
-  NK_HIP(hipEventRecord(mg.ev_fork, s));
-  NK_HIP(hipStreamWaitEvent(b, mg.ev_fork, 0));
+  NK_TRY(record(mg.ev_fork, s));
+  NK_TRY(wait(b, mg.ev_fork));
   // the local solves and their overlap sum (into T.e / T.e32; with
   // fuse_ov the sum is formed after the join from the local solutions)
   // (the timer events bracket the local solves alone)
@@ -1198,46 +1243,57 @@ static int mg_solve_t(Mesh &mesh, FT *z, const FT *r, hipStream_t s, int crs_mod
   };
   // the Schwarz solve of intermediate level l on c (it only reads the
   // masked residual of its level)
-  hipStream_t c = mg.sc;
+  hipStream_t c = one ? s : mg.sc;
   auto level = [&](int l, hipEvent_t after) -> int {
     MgLevel &C = mg.lev[l];
-    NK_HIP(hipStreamWaitEvent(c, after, 0));
+    NK_TRY(wait(c, after));
     if constexpr (f32io)  // inner solve of the mixed solver: FP32 local solves
       NK_TRY((schwarz_local<float, double, double>(mg, l, C.r, C.e, c)));
     else
       NK_TRY(mg_schwarz_local(mg, l, C.r, C.e, c));
     NK_TRY(gs_op(C.gs, C.e, 0, c));
-    NK_HIP(hipEventRecord(mg.ev_le[l], c));
+    NK_TRY(record(mg.ev_le[l], c));
     return NKH_OK;
   };
-  NK_TRY(fine());
   // coarser levels on b: restrict, dssum, mask; then the coarse solve
-  for (int l = Lm - 1; l >= 2; --l) {
-    MgLevel &C = mg.lev[l], &F = mg.lev[l + 1];
-    if (l < Lm - 1) {  // (the level below the fine one was done on s above)
+  auto restricted = [&]() -> int {
+    for (int l = Lm - 2; l >= 2; --l) {  // (the level below the fine one: on s above)
+      MgLevel &C = mg.lev[l], &F = mg.lev[l + 1];
       NK_TRY(run_tnsr<1>(C.r, C.nh, rsrc, F.nh, F.rwt, C.Jt, nel, b, (const double *)nullptr,
                          C.mask));
       NK_TRY(gs_op(C.gs, C.r, 0, b));
-      NK_HIP(hipEventRecord(mg.ev_lr[l], b));
+      NK_TRY(record(mg.ev_lr[l], b));
+      rsrc = C.r;
     }
-    NK_TRY(level(l, mg.ev_lr[l]));
-    rsrc = C.r;
-  }
+    return NKH_OK;
+  };
   // the level-1 mask needs no pass of its own: the coarse gather reads only
   // unmasked vertices and the scatter writes 0 at masked ones (their slot is
   // -1), which is what masking r1 before and e1 after the solve would give
-  if (Lm == 2)
-    NK_TRY((run_tnsr<1, double, FT, double>(L1.r, L1.nh, r, L2.nh, L2.rwt, L1.Jt, nel, b)));
-  else if (!l1_restricted)
-    NK_TRY(run_tnsr<1>(L1.r, L1.nh, rsrc, L2.nh, L2.rwt, L1.Jt, nel, b));
-  NK_TRY(coarse_solve(mg, L1.e, L1.r, crs_mode, b));
+  auto coarse = [&]() -> int {
+    if (Lm == 2)
+      NK_TRY((run_tnsr<1, double, FT, double>(L1.r, L1.nh, r, L2.nh, L2.rwt, L1.Jt, nel, b)));
+    else if (!l1_restricted)
+      NK_TRY(run_tnsr<1>(L1.r, L1.nh, rsrc, L2.nh, L2.rwt, L1.Jt, nel, b));
+    return coarse_solve(mg, Lm > 2 ? nullptr : L1.e, L1.r, crs_mode, b);
+  };
+  auto levels = [&]() -> int {
+    for (int l = Lm - 1; l >= 2; --l) NK_TRY(level(l, mg.ev_lr[l]));
+    return NKH_OK;
+  };
+  // the fine level first: the host may wait in the coarse solve (AMG-PCG)
+  NK_TRY(fine());
+  NK_TRY(restricted());
+  NK_TRY(levels());
+  NK_TRY(coarse());
   for (int l = 2; l < Lm; ++l) {  // e_l = e_l * (mask*wt) + J e_{l-1}
     MgLevel &C = mg.lev[l - 1], &F = mg.lev[l];
-    NK_HIP(hipStreamWaitEvent(b, mg.ev_le[l], 0));
-    NK_TRY(run_tnsr<2>(F.e, F.nh, C.e, C.nh, F.mswt, C.J, nel, b));
+    NK_TRY(wait(b, mg.ev_le[l]));
+    if (l == 2) NK_TRY(prolong_coarse(mg, b));
+    else NK_TRY(run_tnsr<2>(F.e, F.nh, C.e, C.nh, F.mswt, C.J, nel, b));
   }
-  NK_HIP(hipEventRecord(mg.ev_join, b));
-  NK_HIP(hipStreamWaitEvent(s, mg.ev_join, 0));
+  NK_TRY(record(mg.ev_join, b));
+  NK_TRY(wait(s, mg.ev_join));
   // z = dssum(e)*(mask*wt) + J e_{lmax-1}, then dsavg (ic.f:1871-1897)
   MgLevel &C = mg.lev[Lm - 1];
   if (fp32 && fuse_ov) {
