@@ -50,7 +50,7 @@ typedef struct {
                       on the FP64 residual); both need uniform h1/h2, same tolerance */
   int param42;     /* param(42): PRES solver, 2 -> hmh_flex_cg with h1mg (hmholtz.f:646-653) */
   double param21;  /* param(21): PRES tolerance cap (>0) or relative tolerance (<0) (hmholtz.f:2206-2220) */
-  int param40;     /* param(40): coarse solver of h1mg, 0 (XXT) -> solved to 1e-13, 1 (AMG) -> one
+  int param40;     /* param(40): coarse solver of h1mg, 0 (XXT) -> solved directly or to 1e-13, 1 (AMG) -> one
                       AMG V-cycle (navier8.f:209-217, crs_amg.c:129-) */
   /* residual projection switches read by hsolve (navier4.f:589-606) */
   int param93;     /* param(93): number of projection vectors; 0 turns projection off */
