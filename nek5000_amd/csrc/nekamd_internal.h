@@ -350,7 +350,7 @@ int gs_prepare(const GsMap &gs, const double *mask, const double *mult, uint8_t 
 int run_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts, const double *mask,
              const double *mult, double tin, int maxit, const nkh_params &prm,
              nkh_result *res, double *history_host);
-// batched Jacobi-PCG solves (graph-captured iteration), see nkd_hmholtz_batch
+// batched Jacobi-PCG solves (each on its own stream), see nkd_hmholtz_batch
 int batch_create(int nb, const int *meshes, int *id);
 int batch_destroy(int id);
 int batch_meshes(int id, std::vector<int> *meshes);
