@@ -672,7 +672,7 @@ int ensure_small(Mesh &m) {
   // room for the mixed-precision solve's state (a CgState first)
   if (!m.st) NK_HIP(hipMalloc(&m.st, sizeof(McgState)));
   if (!m.red) NK_HIP(hipMalloc(&m.red, sizeof(double) * kRedSize));
-  if (!m.box) NK_TRY(box_alloc(&m.box));
+  if (m.reports && !m.box) NK_TRY(box_alloc(&m.box));
   return NKH_OK;
 }
 
@@ -1292,8 +1292,10 @@ int run_cggo_noalloc(Mesh &m, double *x, const double *f, const double *h1, cons
   double *sp = nullptr;
   NK_TRY(noalloc_scratch(&sp));
   // a view of the mesh whose solve buffers are the scratch: the geometry
-  // and gather-scatter map are the mesh's own, nothing of it is changed
+  // and gather-scatter map are the mesh's own, nothing of it is changed.
+  // Without a box: the state is copied back.
   Mesh v = m;
+  v.reports = false;
   v.box = nullptr;
   v.ws = sp;
   v.ws_doubles = kNoAllocWs;

@@ -148,7 +148,9 @@ struct Mesh {
   size_t ws_doubles = 0;
   CgState *st = nullptr;       // device
   double *red = nullptr;       // device, partial sums
-  HostBox *box = nullptr;      // the solves' reports to the host, and their count
+  // the solves' reports to the host, and their count
+  bool reports = true;         // false: no box (nkd_cggo_noalloc's view of the mesh)
+  HostBox *box = nullptr;
   unsigned long long box_seq = 0;
   BoxRef next_report() { return BoxRef{box, box ? ++box_seq : 0}; }
   Mg *mg = nullptr;            // H1 multigrid hierarchy (nkh_mg_setup)
