@@ -372,9 +372,8 @@ __global__ void __launch_bounds__(kScalThreads)
 
 // rho and alpha (the general path; the fused one has them in the assembly)
 __global__ void __launch_bounds__(kScalThreads)
-    k_cg_scalars2(CgState *__restrict__ st, StepLength step, BoxRef last) {
+    k_cg_scalars2(CgState *__restrict__ st, StepLength step) {
   if (!st->done) step_length(step);
-  else if (threadIdx.x == 0) box_report(last);  // the solve's last kernel
 }
 // rho = the count partials of the operator, alpha = rtz1 / rho
 inline StepLength step_of(CgState *st, const double *part, int count, double *hist) {
@@ -847,16 +846,19 @@ struct CgRun {
   bool fused = false, vec_ok = false, trivial = false;
   int niter = 0, launched = 0, ax_grid_parts = 0;
   double *hist = nullptr;
-  // An iteration makes two reports: the state after its exit test, and the
-  // end of its last kernel if the solve is done (a solve returns only when
-  // nothing of it is left to run).
+  // An iteration reports its state after the exit test.  The test that ends
+  // the solve is not its end: of the kernels behind it, which return at once,
+  // any block that starts late still reads the state (and the next solve in
+  // this work space, on another stream perhaps, sets it anew).  So the host
+  // then waits for everything enqueued.
   HostBox *box = nullptr;  // null: no reports
-  BoxRef last;             // the second report of the iteration enqueued last
-  BoxRef exit_test() const { return BoxRef{box, last.seq - 1}; }
+  BoxRef rep;              // the last one asked for
   int wait(CgState *hs, hipStream_t s) {
-    NK_TRY(box_wait(exit_test(), s));
+    NK_TRY(box_wait(rep, s));
     std::memcpy(hs, box->v, sizeof(CgState));
-    return hs->done ? box_wait(last, s) : NKH_OK;
+    if (!hs->done) return NKH_OK;
+    rep.seq += 1;
+    return box_join(rep, s);
   }
 
   // hmholtz.f:611-720 up to the loop: preconditioner, r = f, null-space check,
@@ -937,20 +939,19 @@ struct CgRun {
     const int64_t n = m->n;
     double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1;
     const int ub = upd_blocks(n);
-    last = BoxRef{box, last.seq + 2};
+    rep = BoxRef{box, rep.seq + 1};
     if (launched > 0)
       hipLaunchKernelGGL((vec_ok ? k_cg_update_dots<true> : k_cg_update_dots<false>), dim3(ub),
                          dim3(256), 0, s, x, r, p, w, dm, bm, n, st, part1, part2,
-                         counters(red), hist, exit_test());
+                         counters(red), hist, rep);
     else  // (the first iteration's sums come from k_cg_init)
       hipLaunchKernelGGL(k_cg_scalars1, dim3(1), dim3(kScalThreads), 0, s, st, part1, part2, ub,
-                         hist, exit_test());
+                         hist, rep);
     if (fused) {
       if (ev) NK_HIP(hipEventRecord(ev[0], s));
       NK_TRY(launch_axhelm_cg(*m, w, p, r, d, h1, h2, mult, st, rho1, s));
       if (ev) NK_HIP(hipEventRecord(ev[1], s));
-      NK_TRY(gs_assemble_step(m->gs, w, st, s, flag, step_of(st, rho1, ax_grid_parts, hist),
-                              last));
+      NK_TRY(gs_assemble_step(m->gs, w, st, s, flag, step_of(st, rho1, ax_grid_parts, hist)));
       if (ev) NK_HIP(hipEventRecord(ev[2], s));
     } else {
       NK_TRY(launch_axhelm_cg(*m, w, p, r, d, h1, h2, mult, st, nullptr, s));
@@ -959,7 +960,7 @@ struct CgRun {
       hipLaunchKernelGGL(k_dot3_guarded, dim3(kRedBlocks), dim3(256), 0, s, w, p, mult, n, st,
                          rho1);
       hipLaunchKernelGGL(k_cg_scalars2, dim3(1), dim3(kScalThreads), 0, s, st,
-                         step_of(st, rho1, kRedBlocks, hist), last);
+                         step_of(st, rho1, kRedBlocks, hist));
     }
     NK_HIP(hipGetLastError());
     ++launched;
@@ -997,18 +998,17 @@ struct McgRun {
   bool trivial = false, vec_ok = false, fused = true;
   int niter = 0, launched = 0, ax_grid_parts = 0;
   double *hist = nullptr;
-  // An iteration makes two reports: the state after its exit test, and the
-  // end of its last kernel if the solve is done (a solve returns only when
-  // nothing of it is left to run).
+  // the reports and the end of a solve as in CgRun
   HostBox *box = nullptr;
+  BoxRef rep;
   bool due = false;  // the last report asked for a refresh
-  BoxRef last;             // the second report of the iteration enqueued last
-  BoxRef exit_test() const { return BoxRef{box, last.seq - 1}; }
   int wait(CgState *hs, hipStream_t s) {
-    NK_TRY(box_wait(exit_test(), s));
+    NK_TRY(box_wait(rep, s));
     std::memcpy(hs, box->v, sizeof(CgState));
     due = box->v[kBoxDue] != 0.0;
-    return hs->done ? box_wait(last, s) : NKH_OK;
+    if (!hs->done) return NKH_OK;
+    rep.seq += 1;
+    return box_join(rep, s);
   }
 
   int begin(Mesh &mesh, double *ws, double *red_, void *st_, double *x_, const double *f_,
@@ -1094,14 +1094,14 @@ struct McgRun {
     const int64_t n = m->n;
     double *part1 = red + kRedPart1, *part2 = red + kRedPart2;
     const int ub = upd_blocks(n);
-    last = BoxRef{box, last.seq + 2};
+    rep = BoxRef{box, rep.seq + 1};
     if (launched > 0)
       hipLaunchKernelGGL((vec_ok ? k_mcg_update_dots<true> : k_mcg_update_dots<false>), dim3(ub),
                          dim3(256), 0, s, xs, r, p, w, dm, bm, n, ms, part1, part2,
-                         counters(red), hist, exit_test());
+                         counters(red), hist, rep);
     else  // (the first iteration's sums come from k_mcg_init)
       hipLaunchKernelGGL(k_mcg_scalars1, dim3(1), dim3(kScalThreads), 0, s, ms, part1, part2, ub,
-                         hist, exit_test());
+                         hist, rep);
     NK_TRY(enqueue_operator(s, ev));
     ++launched;
     return NKH_OK;
@@ -1113,12 +1113,12 @@ struct McgRun {
   // on 9e6 nodes, lx1 8, took 3340 us, now 2830.)
   int refresh(hipStream_t s, hipEvent_t *ev = nullptr) {
     const int64_t n = m->n;
-    last = BoxRef{box, last.seq + 2};
+    rep = BoxRef{box, rep.seq + 1};
     hipLaunchKernelGGL(k_mcg_fold, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, n);
     NK_TRY(launch_axhelm(*m, ax, x, h1, h2, s));
     NK_TRY(gs_assemble(m->gs, ax, nullptr, s, flag));
     hipLaunchKernelGGL(k_mcg_resid, dim3(upd_blocks(n)), dim3(256), 0, s, r, f, ax, dm, bm, n, ms,
-                       red + kRedPart1, red + kRedPart2, counters(red), hist, exit_test());
+                       red + kRedPart1, red + kRedPart2, counters(red), hist, rep);
     return enqueue_operator(s, ev);
   }
 
@@ -1127,8 +1127,7 @@ struct McgRun {
     if (ev) NK_HIP(hipEventRecord(ev[0], s));
     NK_TRY(launch_axhelm32_jac(*m, w, p, r, d, (float)h1.s, (float)h2.s, &ms->gate, rho1, s));
     if (ev) NK_HIP(hipEventRecord(ev[1], s));
-    NK_TRY(gs_assemble_step(m->gs, w, &ms->gate, s, flag, step_of(st, rho1, ax_grid_parts, hist),
-                            last));
+    NK_TRY(gs_assemble_step(m->gs, w, &ms->gate, s, flag, step_of(st, rho1, ax_grid_parts, hist)));
     if (ev) NK_HIP(hipEventRecord(ev[2], s));
     NK_HIP(hipGetLastError());
     return NKH_OK;
@@ -1170,7 +1169,7 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
   }
   CgState hs{};
   run.box = m.box;
-  run.last.seq = m.box_seq;
+  run.rep.seq = m.box_seq;
   // CTIMER mirror: event pairs around axhelm and gs of every launched iteration
   const bool timed = allow_timers && timers().on;
   const int niter = run.niter;
@@ -1192,8 +1191,9 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
   while (true) {
     NK_TRY(run.go_on(s, [&](int k) { return timed ? &ev[4 * k] : nullptr; }));
     if (run.box) {
-      m.box_seq = run.last.seq;
-      NK_TRY(run.wait(&hs, s));
+      const int rc = run.wait(&hs, s);
+      m.box_seq = run.rep.seq;
+      NK_TRY(rc);
     } else if (run.launched < 8 || run.launched % 4 == 0 || run.launched > niter) {
       NK_HIP(hipMemcpyAsync(&hs, run.st, sizeof(CgState), hipMemcpyDeviceToHost, s));
       NK_HIP(hipStreamSynchronize(s));
@@ -1484,10 +1484,10 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
     for (int k : active) {
       Run &run = runs[(size_t)k];
       run.box = B.box[(size_t)k];
-      run.last.seq = B.seq[(size_t)k];
+      run.rep.seq = B.seq[(size_t)k];
       NK_HIP(hipStreamWaitEvent(B.streams[(size_t)k], B.ev[0], 0));
       if (rc == NKH_OK) rc = run.go_on(B.streams[(size_t)k], no_events);
-      B.seq[(size_t)k] = run.last.seq;
+      B.seq[(size_t)k] = run.rep.seq;
       open.push_back(k);
     }
     // round robin over the solves that have not ended: their report is read,
@@ -1498,7 +1498,9 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
         Run &run = runs[(size_t)k];
         hipStream_t q = B.streams[(size_t)k];
         CgState hs;
-        if ((rc = run.wait(&hs, q)) != NKH_OK) break;
+        rc = run.wait(&hs, q);
+        B.seq[(size_t)k] = run.rep.seq;
+        if (rc != NKH_OK) break;
         if (hs.done) {
           run.result(hs, &res[k]);
           continue;
@@ -1509,7 +1511,7 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
           break;
         }
         if ((rc = run.go_on(q, no_events)) != NKH_OK) break;
-        B.seq[(size_t)k] = run.last.seq;
+        B.seq[(size_t)k] = run.rep.seq;
         next.push_back(k);
       }
       open.swap(next);

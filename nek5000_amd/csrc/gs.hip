@@ -318,16 +318,12 @@ __global__ void __launch_bounds__(256)
     k_gs_assemble_pk(T *__restrict__ w, const int32_t *__restrict__ pk_m,
                      const int32_t *__restrict__ pk_g, const uint64_t *__restrict__ pk_head,
                      const int32_t *__restrict__ idx, const uint8_t *__restrict__ flag,
-                     int64_t npk, const CgState *__restrict__ st, int first, StepLength step,
-                     BoxRef last) {
-  const bool done = st && st->done;
-  if ((int)blockIdx.x < first) {  // block 0: the step length, or the end of the solve
-    if (blockIdx.x != 0) return;
-    if (!done) step_length(step);
-    else if (threadIdx.x == 0) box_report(last);
+                     int64_t npk, const CgState *__restrict__ st, int first, StepLength step) {
+  if (st && st->done) return;
+  if ((int)blockIdx.x < first) {  // block 0: the step length
+    if (blockIdx.x == 0) step_length(step);
     return;
   }
-  if (done) return;
   const int p = pk_index(first);
   if (p >= npk) return;
   const PkLane L = pk_lane(pk_m, pk_head, idx, p);
@@ -484,8 +480,7 @@ static int gs_assemble_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s
   const uint8_t *fl = flag ? flag : gs.flag;
   if (gs.npk > 0)
     hipLaunchKernelGGL(k_gs_assemble_pk<T>, dim3(pk_blocks(gs.npk)), dim3(256), 0, s, w,
-                       gs.pk_m, gs.pk_g, gs.pk_head, gs.idx, fl, gs.npk, st, 0, StepLength{},
-                       BoxRef{});
+                       gs.pk_m, gs.pk_g, gs.pk_head, gs.idx, fl, gs.npk, st, 0, StepLength{});
   const int64_t nbig = gs.ngroups - gs.gpk;
   if (nbig > 0) {
     const int nb = gs_blocks(nbig);
@@ -498,9 +493,8 @@ static int gs_assemble_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s
 }
 
 __global__ void __launch_bounds__(1024)
-    k_gs_step(const CgState *__restrict__ st, StepLength step, BoxRef last) {
+    k_gs_step(const CgState *__restrict__ st, StepLength step) {
   if (!(st && st->done)) step_length(step);
-  else if (threadIdx.x == 0) box_report(last);
 }
 
 // The step length rides in the packet kernel as 8 blocks ahead of the
@@ -511,27 +505,27 @@ __global__ void __launch_bounds__(1024)
 // and the step length its own after that.
 template <typename T>
 static int gs_assemble_step_t(const GsMap &gs, T *w, const CgState *st, hipStream_t s,
-                              const uint8_t *flag, const StepLength &a, const BoxRef &last) {
+                              const uint8_t *flag, const StepLength &a) {
   if (gs.npk > 0 && gs.ngroups == gs.gpk) {
     hipLaunchKernelGGL(k_gs_assemble_pk<T>, dim3(pk_blocks(gs.npk) + 8), dim3(256), 0, s, w,
                        gs.pk_m, gs.pk_g, gs.pk_head, gs.idx, flag ? flag : gs.flag, gs.npk, st,
-                       8, a, last);
+                       8, a);
   } else {
     NK_TRY(gs_assemble_t(gs, w, st, s, flag));
-    hipLaunchKernelGGL(k_gs_step, dim3(1), dim3(1024), 0, s, st, a, last);
+    hipLaunchKernelGGL(k_gs_step, dim3(1), dim3(1024), 0, s, st, a);
   }
   NK_HIP(hipGetLastError());
   return NKH_OK;
 }
 
 int gs_assemble_step(const GsMap &gs, double *w, const CgState *st, hipStream_t s,
-                     const uint8_t *flag, const StepLength &a, const BoxRef &last) {
-  return gs_assemble_step_t(gs, w, st, s, flag, a, last);
+                     const uint8_t *flag, const StepLength &a) {
+  return gs_assemble_step_t(gs, w, st, s, flag, a);
 }
 
 int gs_assemble_step(const GsMap &gs, float *w, const CgState *st, hipStream_t s,
-                     const uint8_t *flag, const StepLength &a, const BoxRef &last) {
-  return gs_assemble_step_t(gs, w, st, s, flag, a, last);
+                     const uint8_t *flag, const StepLength &a) {
+  return gs_assemble_step_t(gs, w, st, s, flag, a);
 }
 
 int gs_assemble(const GsMap &gs, double *w, const CgState *st, hipStream_t s,

@@ -1669,7 +1669,7 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
                                    &mg.fst->alpha)) != NKH_OK)
         break;
       if (tm.on) (void)hipEventRecord(ev[1], s);
-      if ((rc = gs_assemble_step(m.gs, w, nullptr, s, nullptr, step, BoxRef{})) != NKH_OK) break;
+      if ((rc = gs_assemble_step(m.gs, w, nullptr, s, nullptr, step)) != NKH_OK) break;
       if (tm.on) (void)hipEventRecord(ev[2], s);
     } else {
       hipLaunchKernelGGL(k_fcg_p, dim3(mg_grid(n)), b, 0, s, p, z, mg.fst, n);

@@ -706,7 +706,7 @@ int run_flex_cg_mixed(Mesh &m, double *res, const SolveFacts &facts, const doubl
         hipLaunchKernelGGL(k_mx_dots<float>, Gd, B, 0, s, mg.xz, mg.xr, mg.xw, mg.xwt, n, pa, pb,
                            cnt, st);
       NK_TRY(launch_axhelm32_flex(m, mg.xw, mg.xp, mg.xz, h1f, h2f, st, den_part, s));
-      NK_TRY(gs_assemble_step(m.gs, mg.xw, nullptr, s, nullptr, step, BoxRef{}));
+      NK_TRY(gs_assemble_step(m.gs, mg.xw, nullptr, s, nullptr, step));
       const BoxRef rep = m.next_report();
       if (wtc)
         hipLaunchKernelGGL(k_mx_update<uint8_t>, Gd, B, 0, s, mg.xx, mg.xr, mg.xp, mg.xw, wtc, st,

@@ -135,11 +135,10 @@ __device__ inline void step_length(const StepLength &a) {
   }
 }
 
-// gs_assemble, then a's step length; once st is done, neither, and the report
-// `last` instead (nothing enqueued here runs after it).
+// gs_assemble, then a's step length; once st is done, neither.
 int gs_assemble_step(const GsMap &gs, double *w, const CgState *st, hipStream_t s,
-                     const uint8_t *flag, const StepLength &a, const BoxRef &last);
+                     const uint8_t *flag, const StepLength &a);
 int gs_assemble_step(const GsMap &gs, float *w, const CgState *st, hipStream_t s,
-                     const uint8_t *flag, const StepLength &a, const BoxRef &last);
+                     const uint8_t *flag, const StepLength &a);
 
 }  // namespace nekamd

@@ -1,0 +1,58 @@
+"""A solve returns only when nothing of it is left to run: the next one, on
+another stream and without a synchronization by the caller, uses the same work
+space and state at once, and the solution can be read there.  Each result
+equals, bit for bit, that of the solve alone."""
+import numpy as np
+import pytest
+
+from problems import Problem, box
+
+pytestmark = pytest.mark.gpu
+
+REPEATS = 12
+
+
+def _alternate(jobs, solve):
+    """solve(job) -> (solution, iterations), alone and then on two streams in
+    turn, each solution copied on the other stream right after its solve."""
+    import torch
+
+    alone = []
+    for job in jobs:
+        u, its = solve(job)
+        torch.cuda.synchronize()
+        alone.append((u.cpu().numpy(), its))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = []
+    for k in range(REPEATS * len(jobs)):
+        with torch.cuda.stream(streams[k % 2]):
+            u, its = solve(jobs[k % len(jobs)])
+        with torch.cuda.stream(streams[(k + 1) % 2]):
+            got.append((u, u.clone(), its))
+    torch.cuda.synchronize()
+    for k, (u, copy, its) in enumerate(got):
+        ref, ref_its = alone[k % len(jobs)]
+        assert its == ref_its
+        assert np.array_equal(u.cpu().numpy(), ref), k
+        assert np.array_equal(copy.cpu().numpy(), ref), k
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_cggo(gpu, fused):
+    # weights that do not sum to 1 per node take the general path
+    P = Problem(box((4, 3, 3), 6, deform=0.1))
+    F = gpu.box_field(P.box)
+    h1, h2, mult = F.zeros() + 1.0, F.zeros() + 3.0, F.mult * (1.0 if fused else 0.5)
+    prm = gpu.default_params(istep=20, param22=0.0, restol=0.0)
+    jobs = []
+    for k, tol in enumerate((-1e-9, -1e-3, -1e-6)):
+        f = P.field.dssum(P.bm1 * P.uniform_field(70 + k)) * P.mask
+        jobs.append((F.to_dev(f), tol))
+
+    def solve(job):
+        u = F.zeros()
+        out = F.cggo(u, job[0], h1, h2, F.mask, mult, job[1], 200, params=prm)
+        return u, out["niter"]
+
+    _alternate(jobs, solve)
+    F.destroy()
