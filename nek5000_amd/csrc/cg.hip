@@ -851,14 +851,12 @@ struct CgRun {
   // any block that starts late still reads the state (and the next solve in
   // this work space, on another stream perhaps, sets it anew).  So the host
   // then waits for everything enqueued.
-  HostBox *box = nullptr;  // null: no reports
-  BoxRef rep;              // the last one asked for
+  Reports reports;
+  BoxRef rep;  // the last one asked for
   int wait(CgState *hs, hipStream_t s) {
     NK_TRY(box_wait(rep, s));
-    std::memcpy(hs, box->v, sizeof(CgState));
-    if (!hs->done) return NKH_OK;
-    rep.seq += 1;
-    return box_join(rep, s);
+    std::memcpy(hs, rep.b->v, sizeof(CgState));
+    return hs->done ? box_join(reports.next(), s) : NKH_OK;
   }
 
   // hmholtz.f:611-720 up to the loop: preconditioner, r = f, null-space check,
@@ -939,7 +937,7 @@ struct CgRun {
     const int64_t n = m->n;
     double *part1 = red + kRedPart1, *part2 = red + kRedPart2, *rho1 = red + kRedRho1;
     const int ub = upd_blocks(n);
-    rep = BoxRef{box, rep.seq + 1};
+    rep = reports.next();
     if (launched > 0)
       hipLaunchKernelGGL((vec_ok ? k_cg_update_dots<true> : k_cg_update_dots<false>), dim3(ub),
                          dim3(256), 0, s, x, r, p, w, dm, bm, n, st, part1, part2,
@@ -999,16 +997,14 @@ struct McgRun {
   int niter = 0, launched = 0, ax_grid_parts = 0;
   double *hist = nullptr;
   // the reports and the end of a solve as in CgRun
-  HostBox *box = nullptr;
+  Reports reports;
   BoxRef rep;
   bool due = false;  // the last report asked for a refresh
   int wait(CgState *hs, hipStream_t s) {
     NK_TRY(box_wait(rep, s));
-    std::memcpy(hs, box->v, sizeof(CgState));
-    due = box->v[kBoxDue] != 0.0;
-    if (!hs->done) return NKH_OK;
-    rep.seq += 1;
-    return box_join(rep, s);
+    std::memcpy(hs, rep.b->v, sizeof(CgState));
+    due = rep.b->v[kBoxDue] != 0.0;
+    return hs->done ? box_join(reports.next(), s) : NKH_OK;
   }
 
   int begin(Mesh &mesh, double *ws, double *red_, void *st_, double *x_, const double *f_,
@@ -1094,7 +1090,7 @@ struct McgRun {
     const int64_t n = m->n;
     double *part1 = red + kRedPart1, *part2 = red + kRedPart2;
     const int ub = upd_blocks(n);
-    rep = BoxRef{box, rep.seq + 1};
+    rep = reports.next();
     if (launched > 0)
       hipLaunchKernelGGL((vec_ok ? k_mcg_update_dots<true> : k_mcg_update_dots<false>), dim3(ub),
                          dim3(256), 0, s, xs, r, p, w, dm, bm, n, ms, part1, part2,
@@ -1113,7 +1109,7 @@ struct McgRun {
   // on 9e6 nodes, lx1 8, took 3340 us, now 2830.)
   int refresh(hipStream_t s, hipEvent_t *ev = nullptr) {
     const int64_t n = m->n;
-    rep = BoxRef{box, rep.seq + 1};
+    rep = reports.next();
     hipLaunchKernelGGL(k_mcg_fold, dim3(upd_blocks(n)), dim3(256), 0, s, x, xs, n);
     NK_TRY(launch_axhelm(*m, ax, x, h1, h2, s));
     NK_TRY(gs_assemble(m->gs, ax, nullptr, s, flag));
@@ -1168,8 +1164,7 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
     return NKH_OK;
   }
   CgState hs{};
-  run.box = m.box;
-  run.rep.seq = m.box_seq;
+  run.reports = Reports{m.box, &m.box_seq};
   // CTIMER mirror: event pairs around axhelm and gs of every launched iteration
   const bool timed = allow_timers && timers().on;
   const int niter = run.niter;
@@ -1188,19 +1183,22 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
   // iteration while the operator of this one runs.  Without a report (the
   // allocation-free solve) the state is copied back, later on every fourth
   // iteration.
-  while (true) {
-    NK_TRY(run.go_on(s, [&](int k) { return timed ? &ev[4 * k] : nullptr; }));
-    if (run.box) {
-      const int rc = run.wait(&hs, s);
-      m.box_seq = run.rep.seq;
-      NK_TRY(rc);
-    } else if (run.launched < 8 || run.launched % 4 == 0 || run.launched > niter) {
-      NK_HIP(hipMemcpyAsync(&hs, run.st, sizeof(CgState), hipMemcpyDeviceToHost, s));
-      NK_HIP(hipStreamSynchronize(s));
+  auto iterate = [&]() -> int {
+    while (true) {
+      NK_TRY(run.go_on(s, [&](int k) { return timed ? &ev[4 * k] : nullptr; }));
+      if (run.reports.box) {
+        NK_TRY(run.wait(&hs, s));
+      } else if (run.launched < 8 || run.launched % 4 == 0 || run.launched > niter) {
+        NK_HIP(hipMemcpyAsync(&hs, run.st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+        NK_HIP(hipStreamSynchronize(s));
+      }
+      if (hs.done) return NKH_OK;
+      NK_CHECK(run.launched <= niter + 1, NKH_ERR_STATE, "cggo: state machine did not terminate");
     }
-    if (hs.done) break;
-    NK_CHECK(run.launched <= niter + 1, NKH_ERR_STATE, "cggo: state machine did not terminate");
-  }
+  };
+  const int rc = iterate();
+  if (rc != NKH_OK) (void)hipStreamSynchronize(s);  // an error leaves work in flight
+  NK_TRY(rc);
   if (timed) {
     NK_HIP(hipEventRecord(t_solve1, s));
     NK_HIP(hipEventSynchronize(t_solve1));
@@ -1441,7 +1439,7 @@ int batch_facts(int id, const nkh_batch_solve *solves, bool chk, SolveFacts *out
     NK_CHECK(m->gs.ngroups == B.nflag[(size_t)k], NKH_ERR_STATE,
              "batch: the gather-scatter map of solve %d changed", k);
     const nkh_batch_solve &q = solves[k];
-    rep[(size_t)k] = BoxRef{B.box[(size_t)k], ++B.seq[(size_t)k]};
+    rep[(size_t)k] = Reports{B.box[(size_t)k], &B.seq[(size_t)k]}.next();
     NK_TRY(enqueue_facts(*m, q.h1, q.h2, q.mask, q.mult, q.rhs, ask, B.red[(size_t)k],
                          B.flag[(size_t)k], rep[(size_t)k], s));
   }
@@ -1483,11 +1481,12 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
     auto no_events = [](int) -> hipEvent_t * { return nullptr; };
     for (int k : active) {
       Run &run = runs[(size_t)k];
-      run.box = B.box[(size_t)k];
-      run.rep.seq = B.seq[(size_t)k];
-      NK_HIP(hipStreamWaitEvent(B.streams[(size_t)k], B.ev[0], 0));
+      run.reports = Reports{B.box[(size_t)k], &B.seq[(size_t)k]};
+      if (rc == NKH_OK && hipStreamWaitEvent(B.streams[(size_t)k], B.ev[0], 0) != hipSuccess) {
+        set_error("batch: a solve's stream cannot wait for its set-up");
+        rc = NKH_ERR_HIP;
+      }
       if (rc == NKH_OK) rc = run.go_on(B.streams[(size_t)k], no_events);
-      B.seq[(size_t)k] = run.rep.seq;
       open.push_back(k);
     }
     // round robin over the solves that have not ended: their report is read,
@@ -1498,9 +1497,7 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
         Run &run = runs[(size_t)k];
         hipStream_t q = B.streams[(size_t)k];
         CgState hs;
-        rc = run.wait(&hs, q);
-        B.seq[(size_t)k] = run.rep.seq;
-        if (rc != NKH_OK) break;
+        if ((rc = run.wait(&hs, q)) != NKH_OK) break;
         if (hs.done) {
           run.result(hs, &res[k]);
           continue;
@@ -1511,7 +1508,6 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
           break;
         }
         if ((rc = run.go_on(q, no_events)) != NKH_OK) break;
-        B.seq[(size_t)k] = run.rep.seq;
         next.push_back(k);
       }
       open.swap(next);

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/nekamd.h"
+#include "reports.h"
 
 namespace nekamd {
 
@@ -99,20 +100,6 @@ struct CgState {
   int param18;
 };
 
-// Host memory that kernels report to: the thread that holds a result writes
-// it to v and then the report's number to seq, where the host, waiting for
-// that number, finds it a few microseconds later (a copy and a stream
-// synchronization leave the GPU idle for about 40 us; MI355X).
-struct HostBox {
-  unsigned long long seq;
-  unsigned long long pad[7];
-  double v[56];
-};
-// one report: its place and number (b null: none is made)
-struct BoxRef {
-  HostBox *b = nullptr;
-  unsigned long long seq = 0;
-};
 __device__ __forceinline__ void box_report(const BoxRef &r) {
   if (!r.b) return;
   __threadfence_system();
@@ -152,7 +139,7 @@ struct Mesh {
   bool reports = true;         // false: no box (nkd_cggo_noalloc's view of the mesh)
   HostBox *box = nullptr;
   unsigned long long box_seq = 0;
-  BoxRef next_report() { return BoxRef{box, box ? ++box_seq : 0}; }
+  BoxRef next_report() { return Reports{box, &box_seq}.next(); }
   Mg *mg = nullptr;            // H1 multigrid hierarchy (nkh_mg_setup)
   // FP32 copies of g and bm1 for the single-precision operator (built on
   // first use, rebuilt when geom_version moves)
