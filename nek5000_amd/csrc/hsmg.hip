@@ -1738,6 +1738,10 @@ int run_flex_cg(Mesh &m, double *res, const SolveFacts &facts, const double *wt,
     NK_HIP(hipMemcpyAsync(&hs, mg.fst, sizeof(FcgState), hipMemcpyDeviceToHost, s));
     NK_HIP(hipStreamSynchronize(s));
   }
+  // The report that ended the loop came from the last block of a kernel whose
+  // other blocks may still be storing, and the solution was finished after it:
+  // the next solve, perhaps on another stream, uses p and the state at once.
+  NK_TRY(box_join(m.next_report(), s));
   if (out) {
     out->niter = iter;
     out->converged = hs.done;

@@ -56,3 +56,28 @@ def test_cggo(gpu, fused):
 
     _alternate(jobs, solve)
     F.destroy()
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_flexible_cg(gpu, fused):
+    # a pressure mask that is not the hierarchy's fine mask takes the general
+    # path: here the hierarchy has Neumann faces on top, the mask Dirichlet ones
+    b = box((4, 3, 3), 6, deform=0.1)
+    P = Problem(b)
+    F = gpu.box_field(b)
+    fbc = b.fast_bc()
+    top = (np.arange(b.nel) // (b.nelx * b.nely)) == b.nelz - 1
+    fbc[top, 5] = 2  # Neumann
+    F.h1mg_setup(b.fast_bc() if fused else fbc, b.vertex, *b.xyz())
+    h1, h2 = F.zeros() + 1.0, F.zeros()
+    jobs = [(F.to_dev(P.field.dssum(P.bm1 * P.uniform_field(80 + k)) * P.mask), tol)
+            for k, tol in enumerate((-1e-9, -1e-2, -1e-5))]
+
+    def solve(job):
+        u = job[0].clone()
+        out = F.hmh_flex_cg(u, h1, h2, F.mult, 60,
+                            params=gpu.default_params(istep=20, param21=job[1], param42=2))
+        return u, out["niter"]
+
+    _alternate(jobs, solve)
+    F.destroy()
