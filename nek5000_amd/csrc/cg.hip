@@ -1159,8 +1159,10 @@ int drive_cggo(Mesh &m, double *x, const double *f, const SolveFacts &facts,
   Run run;
   NK_TRY(run.begin(m, m.ws, m.red, m.st, x, f, facts, mask, mult, tin, maxit, prm,
                    history_host != nullptr, s));
-  if (run.trivial) {
+  if (run.trivial) {  // x = 0 is enqueued: returned when it is there, as any solution
     run.result(CgState{}, res);
+    if (m.box) return box_join(m.next_report(), s);
+    NK_HIP(hipStreamSynchronize(s));
     return NKH_OK;
   }
   CgState hs{};
@@ -1522,8 +1524,14 @@ int batch_drive(CgBatch &B, const double *const *x, const double *const *f,
     }
     NK_TRY(rc);
   }
+  int zero = -1;  // a solve whose x = 0 is enqueued on s
   for (int k = 0; k < B.nb; ++k)
-    if (runs[(size_t)k].trivial) runs[(size_t)k].result(CgState{}, &res[k]);
+    if (runs[(size_t)k].trivial) {
+      runs[(size_t)k].result(CgState{}, &res[k]);
+      zero = k;
+    }
+  if (zero >= 0)
+    NK_TRY(box_join(Reports{B.box[(size_t)zero], &B.seq[(size_t)zero]}.next(), s));
   if (launches_out) *launches_out = launches;
   return NKH_OK;
 }

@@ -81,3 +81,40 @@ def test_flexible_cg(gpu, fused):
 
     _alternate(jobs, solve)
     F.destroy()
+
+
+@pytest.mark.parametrize("kind", ["hmholtz", "mixed", "noalloc", "batch"])
+def test_zero_right_hand_side(gpu, kind):
+    # the solution 0 is there when the call returns, read on another stream
+    import torch
+
+    F = gpu.box_field(box((10, 10, 10), 8))
+    h1, h2, zero = F.zeros() + 1.0, F.zeros() + 3.0, F.zeros()
+    prm = gpu.default_params(istep=20, precision=2 if kind == "mixed" else 0)
+    us = [F.zeros() + 1.0 for _ in range(20)]
+    rhs = zero.clone()
+    B = gpu.Batch([F, F]) if kind == "batch" else None
+    q = [dict(u=None, rhs=rhs, h1=h1, h2=h2, mask=F.mask, mult=F.mult, tli=-1e-8),
+         dict(u=F.zeros(), rhs=F.mass()[0] * F.mask, h1=h1, h2=h2, mask=F.mask, mult=F.mult,
+              tli=-1e-8)]
+    streams, copies = [torch.cuda.Stream(), torch.cuda.Stream()], []
+    torch.cuda.synchronize()
+    for u in us:
+        with torch.cuda.stream(streams[0]):
+            if kind == "batch":
+                q[0]["u"] = u
+                niter = B.hmholtz(q, 900, params=prm)[0][0]["niter"]
+            elif kind == "noalloc":
+                niter = F.cggo(u, rhs, h1, h2, F.mask, F.mult, -1e-8, 900, params=prm,
+                               noalloc=True)["niter"]
+            else:
+                niter = F.hmholtz("VELX", u, rhs, h1, h2, F.mask, F.mult, -1e-8, 900,
+                                  params=prm)["niter"]
+        assert niter == 0
+        with torch.cuda.stream(streams[1]):
+            copies.append(u.clone())
+    torch.cuda.synchronize()
+    assert all(bool((c == 0.0).all()) for c in copies)
+    if B is not None:
+        B.destroy()
+    F.destroy()
