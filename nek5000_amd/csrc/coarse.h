@@ -84,6 +84,8 @@ struct CoarseSolver {
             const std::vector<double> &val, const std::vector<double> &xyz, hipStream_t s);
   int setup_amg(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
                 const std::vector<double> &val);
+  int build_amg(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
+                const std::vector<double> &val);
   // x = A^-1 b, directly, or to the relative residual rtol (or rtol_use when
   // > 0) by PCG, where the host waits on stream s.
   int solve(double *xout, const double *b, hipStream_t s, double rtol_use = 0.0);

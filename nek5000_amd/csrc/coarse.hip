@@ -613,7 +613,17 @@ int CoarseSolver::setup(const std::vector<int32_t> &rowptr, const std::vector<in
   return NKH_OK;
 }
 
+// The hierarchy is there whole or not at all: it may be asked for inside a
+// solve, and again by the next one after a failure.
 int CoarseSolver::setup_amg(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
+                            const std::vector<double> &val) {
+  const int rc = build_amg(rowptr, col, val);
+  if (rc != NKH_OK) release_amg();
+  has_amg = rc == NKH_OK;
+  return rc;
+}
+
+int CoarseSolver::build_amg(const std::vector<int32_t> &rowptr, const std::vector<int32_t> &col,
                             const std::vector<double> &val) {
   release_amg();
   Csr A;
@@ -678,7 +688,6 @@ int CoarseSolver::setup_amg(const std::vector<int32_t> &rowptr, const std::vecto
     NK_TRY(dalloc(&L.r, L.n));
     NK_TRY(dalloc(&L.b, L.n));
   }
-  has_amg = true;
   if (nlevels_amg == 0) return NKH_OK;  // dense solve of the whole problem
   for (double **q : {&x, &rb[0], &rb[1], &z, &w, &p[0], &p[1]}) NK_TRY(dalloc(q, n));
   NK_TRY(dalloc(&part, 4 * kCrsBlocks));
