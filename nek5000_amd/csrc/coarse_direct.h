@@ -22,18 +22,29 @@ struct DirectCoarse {
   int32_t *si_rp = nullptr, *si_ci = nullptr;
   double *si_v = nullptr;
   double *y = nullptr, *g = nullptr, *xs = nullptr;
+  // steps of refinement in a solve; where there are any, the problem's rows, a
+  // residual and a correction
+  int refine = 0;
+  int32_t *a_rp = nullptr, *a_ci = nullptr;
+  double *a_v = nullptr, *rr = nullptr, *dd = nullptr;
 
   bool ready() const { return n > 0; }
   // rows of the assembled SPD problem, and three coordinates per unknown (the
   // dissection splits along them).  *ok = false, nothing kept: the problem is
-  // too large for this solver or not positive definite to rounding, or memory
-  // is short.
+  // too large for this solver, a pivot is rounding or the residual of a solve
+  // is too large (kPivotMin, kMaxResidual), or memory is short.
   int setup(const std::vector<int32_t> &rp, const std::vector<int32_t> &ci,
             const std::vector<double> &v, const std::vector<double> &xyz, hipStream_t s,
             bool *ok);
   // x = A^-1 b, enqueued on s (x and b distinct)
   int solve(double *x, const double *b, hipStream_t s) const;
   void release();
+
+ private:
+  // one pass of the inverses, without refinement
+  int apply(double *x, const double *b, hipStream_t s) const;
+  bool refine_to(const std::vector<int32_t> &rp, const std::vector<int32_t> &ci,
+                 const std::vector<double> &v, const std::vector<double> &xyz, hipStream_t s);
 };
 
 }  // namespace nekamd
