@@ -3,7 +3,9 @@ kernels is not full (several elements share a block below lx1 8), at every kind
 of default kernel (element-staged, matrix cores by element and by planes) and
 for constant and varying h1 and h2, against the oracle.  Bounds: the operator
 sums 3 lx1 products per node twice, 1e-13 of the largest value; the solves stop
-at 1e-10."""
+at 1e-10, their iteration counts within 1 of the oracle's, give or take how far
+those move when the right-hand side moves by one rounding (0, but 283 to 286 of
+284 iterations at lx1 16 with varying h1 and h2)."""
 import numpy as np
 import pytest
 
@@ -41,6 +43,12 @@ def test_ragged(gpu, lx1, kinds):
     x = F.zeros()
     out = F.hmholtz("VELX", x, F.to_dev(rhs), *hd, F.mask, F.mult, -1e-10, 400,
                     params=gpu.default_params(istep=20, param22=0.0, restol=0.0))
-    assert abs(out["niter"] - ito) <= 1
+    rng, its = np.random.default_rng(lx1), [ito]
+    for _ in range(4):
+        r = rhs * (1.0 + np.finfo(float).eps * rng.choice([-1.0, 1.0], rhs.shape))
+        its.append(P.field.hmholtz(r, *h, -1e-10, 400, O.Params(20, 0.0, 0.0, 0.0))[2])
+    slack = 1 + max(its) - min(its)
+    print(out["niter"], its, flush=True)
+    assert min(its) - slack <= out["niter"] <= max(its) + slack
     assert np.linalg.norm(x.cpu().numpy() - uo) <= 1e-8 * np.linalg.norm(uo)
     F.destroy()
