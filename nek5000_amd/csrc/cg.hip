@@ -1312,12 +1312,13 @@ int run_cggo_noalloc(Mesh &m, double *x, const double *f, const double *h1, cons
 // ---------------------------------------------------------------------------
 // Batched Jacobi-PCG: several hmholtz solves (different meshes, h1/h2,
 // masks, sizes; the same lx1 or not) iterate together, each with its own work
-// space, state, gs group flags and stream.  The host enqueues the next
-// iteration of whichever solve has reported its exit test, so that the solves
-// run side by side and none waits for another.  (A captured graph of eight
-// iterations of all of them, built on every call, took longer to build than
-// small solves take to run: five solves of 560 to 1,320 elements 3.3 ms per
-// call with it.)
+// space, state, gs group flags and stream.  The host takes the open solves in
+// turn, waits for the report of one's exit test and enqueues its next
+// iteration: they run side by side, in step with the slowest of them.  (A
+// captured graph of eight iterations of all of them, built on every call, took
+// longer to build than small solves take to run: five solves of 560 to 1,320
+// elements 3.3 ms a call with it, 1.7 so; 64 of 336 elements 54 and 13 ms, one
+// solve after another 23.)
 // ---------------------------------------------------------------------------
 struct CgBatch {
   int nb = 0;

@@ -182,7 +182,8 @@ __device__ __forceinline__ void column_mass(double (&m)[NP], int64_t base,
 // at least: left alone, the compiler hoists every factor load and takes up
 // to 256 registers at NP >= 9 (NP = 12, 1.67e7 nodes, plain: 640 us against
 // 427).  MODE 1 at 1.67e7 nodes, us before -> now: NP = 6 412 -> 300, NP = 8
-// 326 -> 269 (6.0 TB/s).
+// 326 -> 269 (6.0 TB/s).  (NP = 14 with varying h1 spills 3 registers for it,
+// 30 with varying h2 as well; the matrix cores are faster there.)
 template <int NP, int MODE, bool H1F, int H2M, int EPB_ = epb<NP>()>
 __global__ void __launch_bounds__(NP * NP * EPB_,
                                   min_waves((24 * NP + 16) * (NP + 1) * NP * EPB_, NP * NP * EPB_))
@@ -795,8 +796,10 @@ struct AxhelmChoice {
 // Untuned (meshes of less than 2^20 nodes): per order the kernel that is the
 // fastest or near it at 6e4 to 9e5 nodes -- element-staged up to NP = 8, the
 // matrix cores beyond, staging the element (4) or groups of planes (5).  us
-// at 2.5e5 nodes, element-staged / matrix cores, CG-fused apply: NP = 8 13 /
-// 18 (4), 10 26 / 22 (5), 12 37 / 29 (5), 14 53 / 39 (4), 16 67 / 49 (5).
+// at 2.5e5 nodes, element-staged / 4 / 5, CG-fused apply: NP = 8 9.4 / 14.6 /
+// 17.8, 9 22.7 / 23.0 / 20.6, 10 22.4 / 18.6 / 17.8, 11 27.2 / 22.2 / 23.8, 12
+// 32.5 / 24.0 / 25.7, 13 40.9 / 30.2 / 30.7, 14 46.8 / 31.9 / 32.9, 15 60.2 /
+// 35.6 / 37.5, 16 58.0 / 41.1 / 37.2.
 constexpr AxhelmChoice axhelm_default(int np) {
   const int v = np < 9 ? 0 : (np == 11 || (np >= 13 && np <= 15) ? 4 : 5);
   return AxhelmChoice{v, 0, v, v, false};

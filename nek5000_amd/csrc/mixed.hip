@@ -261,6 +261,10 @@ __device__ __forceinline__ void column_in32(float (&v)[NP], int64_t base, bool s
   }
 }
 
+// Three wavefronts per SIMD at NP = 9 and 10, where the compiler otherwise takes
+// 172 to 256 registers for what 168 hold without scratch (9e6 nodes, us, JAC
+// and flexible CG with a mass term: NP = 9 121 -> 96 and 147 -> 84, NP = 10 168
+// -> 143 and 160 -> 124).
 template <int NP, bool H2, bool JAC>
 __global__ void __launch_bounds__(NP * NP * epb<NP>(), NP == 9 || NP == 10 ? 3 : 1)
     k_axhelm32(DMatF<NP> Dk, const double *__restrict__ Dg, float *__restrict__ w,
@@ -512,9 +516,10 @@ __global__ void __launch_bounds__(mx_threads<NP>(), 2)
 // Kernel of the FP32 operator per order: 0 vector FMA (k_axhelm32), 1 the
 // matrix cores (k_axhelm32_mxp, lx1 = 8..16); nkh_axhelm32_set_variant fixes
 // it.  Defaults: the faster one at 9e6 nodes, us vector / matrix cores, JAC
-// and flexible CG: lx1 = 8 76 / 79 and 64 / 70, 9 97 / 108 and 85 / 98, 10
-// 135 / 105 and 90 / 93, 12 185 / 123 and 109 / 115, 14 230 / 155 and 214 /
-// 146, 16 197 / 149 and 158 / 123.
+// (with a mass term) and flexible CG (without): lx1 = 8 74 / 77 and 58 / 65, 9
+// 96 / 104 and 81 / 92, 10 143 / 104 and 90 / 90, 11 131 / 106 and 143 / 95, 12
+// 220 / 114 and 204 / 106, 13 648 / 143 and 666 / 132, 14 528 / 158 and 359 /
+// 150, 15 655 / 162 and 627 / 150, 16 192 / 148 and 195 / 120.
 int g_ax32_variant[kMaxNP + 1] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 1};
 
 template <int NP, bool JAC>

@@ -84,10 +84,10 @@ struct GsMap {
   uint64_t *pk_head = nullptr;  // device, npk: bit l set where a group starts at lane l
 };
 
-// State of one PCG solve, resident on the device.  The scalar kernels update
-// it; the vector kernels read alpha/beta from it and return at once when
-// `done` is set, so the host can enqueue iterations ahead without reading
-// the residual back every iteration.
+// State of one PCG solve, resident on the device.  The last block of the dots
+// and a block of the assembly update it; the vector kernels read alpha/beta
+// from it and return at once when `done` is set: the operator and the assembly
+// behind an exit test are enqueued before the host has read its report.
 struct CgState {
   double rtz1, rtz2, rho, alpha, beta;
   double rbn0, rbn2, tol, tin, vol, param22;
