@@ -141,7 +141,8 @@ def cpu_baseline(nel1d, lx1, deform, target_seconds, solver="hsmg"):
 def order_sweep(orders=range(3, 16)):
     """Polynomial-order sweep (jittered boxes, E^(1/3) ~ 368/N so every order
     carries about 5e7 unique DOF; h1 = h2 = 1; f ~ U(-1,1)): per order the
-    autotuner's choice (made on the first apply), the CG-fused axhelm
+    autotuner's choice for constant coefficients (made by the first solve),
+    the CG-fused axhelm
     kernel's time per kernel variant (0/1 element/plane staged, 2/3 the
     same with the wide slab packing, 4/5 the r/s contractions on the FP64
     matrix cores with the element / groups of t-planes staged, at N = 7..15;
@@ -188,13 +189,11 @@ def order_sweep(orders=range(3, 16)):
         one = torch.ones_like(rhs)
         free = float(torch.sum(F.mask * F.mult))
         setup = time.time() - t0
-        au = torch.zeros_like(rhs)
-        F.axhelm(au, rhs, one, one)  # the first apply of the order tunes it
-        torch.cuda.synchronize()
+        u = torch.zeros_like(rhs)
+        timed_pcg(F, u, rhs, one, 1)  # the first solve of the order tunes it
         chosen = solver.axhelm_tuning(N + 1)
         chosen_fused = solver.axhelm_tuning_fused(N + 1)
 
-        u = torch.zeros_like(rhs)
         per_variant = {}
         for v in (0, 1, 2, 3, 4, 5):
             solver.set_axhelm_tuning(N + 1, v, 0)
@@ -232,7 +231,7 @@ def order_sweep(orders=range(3, 16)):
         log(f"[sweep] {row}")
         rows.append(row)
         F.destroy()
-        del F, rhs, one, au, u, bm1
+        del F, rhs, one, u, bm1
         torch.cuda.empty_cache()
     print(json.dumps({"sweep": "order", "precision": "fp64", "rows": rows}), flush=True)
 
@@ -334,7 +333,7 @@ def batch_run(steps=2):
     it for any field of a transient run; N = 7, f ~ U(-1,1) per unique node,
     Jacobi PCG to 1e-8 relative, at most 900 iterations as cggo's maxcg):
     one after another through hmholtz in FP64 (the baseline), and batched
-    (nkd_hmholtz_batch: the iteration of all five in one hipGraph) in FP64
+    (nkd_hmholtz_batch: side by side, each on its own stream) in FP64
     and in mixed precision (FP32 iteration, FP64 refreshes).  Prints one
     JSON line."""
     import torch
@@ -385,7 +384,7 @@ def batch_run(steps=2):
     for tag, fn, precision in (("sequential_fp64", run_seq, 0), ("batched_fp64", run_batch, 0),
                                ("batched_mixed", run_batch, 2),
                                ("sequential_mixed", run_seq, 2)):
-        fn(precision)  # warm-up (graph capture, autotuning, FP32 factors)
+        fn(precision)  # warm-up (autotuning, FP32 factors)
         best = None
         for _ in range(steps):
             r = fn(precision)
@@ -430,8 +429,8 @@ def main():
     ap.add_argument("--maxit", type=int, default=900,
                     help="iteration cap per solve (900 = the reference's maxcg)")
     ap.add_argument("--crs", type=int, default=0,
-                    help="coarse solver of the V-cycle: 0 solved to 1e-13 (the reference's "
-                         "exact XXT), 1 one AMG V-cycle (its param(40)=1)")
+                    help="coarse solver of the V-cycle: 0 solved, directly or to 1e-13 (the "
+                         "reference's exact XXT), 1 one AMG V-cycle (its param(40)=1)")
     ap.add_argument("--precision", type=int, default=0, choices=(0, 1, 2),
                     help="main line's nkh_params.precision (profiling the mixed solvers)")
     ap.add_argument("--fdm-variant", type=int, default=0, choices=(0, 1, 2, 3),
@@ -441,8 +440,8 @@ def main():
     ap.add_argument("--no-variants", action="store_true",
                     help="skip the extra short run of the other coarse solver")
     ap.add_argument("--batch", action="store_true",
-                    help="instead of the bench line: five solves of a time step batched in one "
-                         "graph vs one after another")
+                    help="instead of the bench line: five solves of a time step batched "
+                         "vs one after another")
     ap.add_argument("--adjoint", action="store_true",
                     help="instead of the bench line: adjoint gradient timing and finite-"
                          "difference check at E=32^3, N=7")
@@ -620,7 +619,7 @@ def main():
         if hsmg:
             other = 1 - args.crs
             measure("coarse: " + ("one AMG V-cycle (param40=1)" if other == 1 else
-                                  "AMG-PCG to 1e-13"), params_for(other))
+                                  "solved"), params_for(other))
             measure("mixed: FP32 fine-level smoother, FP64 Krylov and coarse",
                     params_for(args.crs, 1))
             measure("mixed + one-V-cycle coarse", params_for(1, 1))
@@ -745,7 +744,9 @@ def main():
             "multigrid": mg_info,
             "coarse_solver": (None if not hsmg else
                               ("one AMG V-cycle (param40=1)" if args.crs == 1 else
-                               "AMG-preconditioned CG to 1e-13 (exact, as XXT)")),
+                               "AMG-preconditioned CG to 1e-13 (exact, as XXT)"
+                               if mg_info["crs_avg_iters"] > 0 else
+                               "explicit inverses (exact, as XXT)")),
             "variants": variants,
             "seconds_per_solve": elapsed / args.steps,
             "free_dof": free_dof, "iterations_per_solve": iters,
