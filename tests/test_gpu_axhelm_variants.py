@@ -215,7 +215,7 @@ def test_tuning_arguments_checked(gpu):
 
 @pytest.mark.parametrize("variant", [4, 5])
 def test_gated_apply_matrix_core_variants(gpu, variant):
-    """The gated apply (the mixed Jacobi PCG's FP64 residual refreshes) on the
+    """The FP64 operator of the mixed Jacobi PCG's residual refreshes on the
     matrix cores: the mixed solve's true FP64 residual, recomputed with the
     oracle's operator, meets the tolerance, in about the FP64 solve's
     iteration count."""
@@ -231,7 +231,7 @@ def test_gated_apply_matrix_core_variants(gpu, variant):
     try:
         for tag, v, prec in (("fp64", 0, 0), ("mixed", variant, 2)):
             gpu.set_axhelm_tuning(lx1, v, 0)
-            say(f"[gated variants] lx1={lx1} {tag} variant={v}")
+            say(f"[refresh variants] lx1={lx1} {tag} variant={v}")
             u = F.zeros()
             r = F.to_dev(rhs)
             prm = gpu.default_params(istep=20, param22=0.0, restol=0.0, precision=prec)

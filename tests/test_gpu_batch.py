@@ -1,7 +1,6 @@
 """Batched hmholtz solves (nkh_batch_create / nkd_hmholtz_batch): solves on
 different meshes, orders, coefficients and masks -- one mesh used twice with
-two masks -- iterate together with the steady-state iteration of the whole
-batch captured in one hipGraph and replayed.  Every solve's iteration count
+two masks -- iterate together, each on its own stream.  Every solve's iteration count
 and solution equal, bit for bit, those of nkd_hmholtz on the same solve
 (the same kernels in the same order), and agree with the oracle."""
 import sys
@@ -55,12 +54,12 @@ def test_batch_equals_single_solves(gpu):
         solves.append(dict(u=F.zeros(), rhs=b.clone(), h1=h1, h2=h2, mask=mask, mult=F.mult,
                            tli=tli))
     B = gpu.Batch([c[0] for c in cases])
-    for rep in range(2):  # the batch again (a new graph) gives the same
+    for rep in range(2):  # the batch again gives the same
         for q in solves:
             q["u"].zero_()
         outs, launches = B.hmholtz(
             [dict(q, rhs=q["rhs"].clone()) for q in solves], 900, params=prm)
-        say(f"[batch] rep {rep}: graph launches {launches}, iterations "
+        say(f"[batch] rep {rep}: iterations enqueued {launches}, iterations "
             f"{[o['niter'] for o in outs]} vs single {[r[1]['niter'] for r in ref]}")
         for k, (q, o) in enumerate(zip(solves, outs)):
             assert o["niter"] == ref[k][1]["niter"], k

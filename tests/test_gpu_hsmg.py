@@ -5,9 +5,9 @@ against the oracle on the same seeded inputs.
 Tolerances (FP64): the hierarchy's integer facts (levels, points per level,
 coarse unknowns) exactly; one V-cycle z = M r within 1e-10 relative L2 (the
 FDM eigenvectors come from the same Cholesky + Jacobi algorithm compiled by
-a different compiler, and above 600 unknowns the coarse problem is solved by
-AMG-preconditioned CG to a 1e-13 relative residual instead of a direct
-factor); flexible-CG iteration counts
+a different compiler, and the coarse problem is solved by explicit inverses,
+beyond about 60,000 unknowns by AMG-preconditioned CG to a 1e-13 relative
+residual, instead of a factor); flexible-CG iteration counts
 within +-1, residual-norm histories within 1e-6 relative over the common
 iterations (plus 1e-15 of the initial residual: below that the last digits
 are round-off), solutions within 1e-9 relative L2.
@@ -43,8 +43,8 @@ MG_CASES = [
     dict(nel=(4, 3, 3), lx1=7, periodic_x=True, jitter=0.04, seed=7),
     dict(nel=(2, 3, 3), lx1=10, deform=0.1),
     dict(nel=(3, 3, 2), lx1=6, neumann_top=True),
-    # more than 600 coarse unknowns: the coarse problem goes through the
-    # AMG-preconditioned CG instead of the dense inverse
+    # 990 coarse unknowns (beyond the AMG's dense last level, which param40 = 1
+    # applies)
     dict(nel=(12, 11, 10), lx1=4, deform=0.05),
 ]
 
@@ -478,8 +478,8 @@ def test_pressure_null_space(gpu, case):
     (crs_xxt.c:883-955), flexible CG and GMRES end with ortho
     (hmholtz.f:2272, gmres.f:427,534).  A consistent right-hand side; the
     GPU against the oracle (iterations +-1, histories 1e-6, solutions 1e-9),
-    the solution's local-node mean zero.  The second mesh has more than 600
-    coarse unknowns: AMG-preconditioned CG on the coarse problem."""
+    the solution's local-node mean zero.  The second mesh has more coarse
+    unknowns than the AMG's dense last level."""
     P, mg, F = build(gpu, case)
     assert O.lib().nko_mg_null_space(mg.h) == 1
     h1 = np.ones(P.shape)
